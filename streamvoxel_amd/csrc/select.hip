@@ -342,17 +342,13 @@ __global__ __launch_bounds__(kWG) void apportion_kernel(const int64_t* __restric
   });
 }
 
-// The same for one window of at most kWaveBlocks blocks, run by one wave without workgroup barriers: the keys in
-// LDS (`skey`, kWaveBlocks entries), an MSB-first 8-bit radix select over the 64-bit keys with the histogram
-// (`hist`, 256 entries) in LDS, then the `extra` smallest (key, block index) get one more voxel. Called by lanes
-// 0..63 of one wave; block j is handled by lane j % 64 throughout, so its global reads and writes need no fence.
-constexpr int kWaveBlocks = 1024;
-
-__device__ __forceinline__ void wave_sync_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
+// The same for one window of at most kGroupBlocks blocks, by a workgroup of 256 threads: every thread holds the keys of
+// blocks t, t + 256, ... in registers; an MSB-first 8-bit radix select finds the threshold, one LDS histogram a digit,
+// and ends as soon as the threshold's bin is taken whole (mostly after three or four of the eight digits). A serial
+// chain of loads, digits and barriers that runs beside the entropy pass; by one wave with the keys in LDS it took longer
+// than the entropy pass beside it (one window of 256 fp32 classes as planes: 28.8 us for the launch, 23.4 us now).
+constexpr int kGroupBlocks = 1024;
+constexpr int kGroupThreads = 256;
 
 struct ApportionArgs {
   const int64_t* n_total;
@@ -364,112 +360,123 @@ struct ApportionArgs {
   int64_t* target;
 };
 
-__device__ void apportion_window(const ApportionArgs& a, int64_t b, int lane, uint64_t* skey, uint32_t* hist) {
+struct ApportionShared {
+  uint32_t hist[256];
+  int64_t red[kGroupThreads / 64];
+  uint32_t ties[kGroupBlocks / 64];  // of the blocks [64 i, 64 i + 64)
+};
+
+__device__ void apportion_group(const ApportionArgs& a, int64_t b, ApportionShared& sh) {
 #pragma clang fp contract(off)
-  const int64_t nb = a.nb;
+  constexpr int kPer = kGroupBlocks / kGroupThreads;
+  const int nb = static_cast<int>(a.nb);
+  const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, w = tid >> 6;
   const double f = a.frac[b];
-  const int64_t* nt = a.n_total + b * nb;
-  const int64_t* ps = a.pos + b * nb;
-  int64_t* tg = a.target + b * nb;
-  constexpr int kUnrollBlocks = 4;
-  int64_t local = 0;
-  for (int64_t j0 = lane; j0 < nb; j0 += 64 * kUnrollBlocks) {
-    // Loads are unconditional (clamped index) so that all of them are in flight at once.
-    int64_t ntv[kUnrollBlocks], psv[kUnrollBlocks];
+  const int64_t* nt = a.n_total + b * a.nb;
+  const int64_t* ps = a.pos + b * a.nb;
+  int64_t* tg = a.target + b * a.nb;
+  // Loads are unconditional (clamped index) so that all of them are in flight at once.
+  int64_t ntv[kPer], psv[kPer];
 #pragma unroll
-    for (int u = 0; u < kUnrollBlocks; ++u) {
-      const int64_t j = j0 + 64 * u < nb ? j0 + 64 * u : nb - 1;
-      ntv[u] = nt[j];
-      psv[u] = ps[j];
-    }
+  for (int u = 0; u < kPer; ++u) {
+    const int j = min(tid + kGroupThreads * u, nb - 1);
+    ntv[u] = nt[j];
+    psv[u] = ps[j];
+  }
+  const int64_t want = a.committed[b] + a.k[b];
+  uint64_t key[kPer];
+  int64_t quota[kPer], local = 0;
 #pragma unroll
-    for (int u = 0; u < kUnrollBlocks; ++u) {
-      const int64_t j = j0 + 64 * u;
-      if (j < nb) {
-        const double ideal = f * static_cast<double>(ntv[u]);
-        const double shifted = ideal + 1e-9;
-        const double base = floor(shifted);
-        const double neg_frac = -(ideal - base);
-        const double scaled = neg_frac * 1e6;
-        const double key = scaled + static_cast<double>(psv[u]);
-        skey[j] = ordered_u64(key);
-        tg[j] = static_cast<int64_t>(base);
-        local += static_cast<int64_t>(base);
-      }
-    }
+  for (int u = 0; u < kPer; ++u) {
+    const double ideal = f * static_cast<double>(ntv[u]);
+    const double shifted = ideal + 1e-9;
+    const double base = floor(shifted);
+    const double neg_frac = -(ideal - base);
+    const double scaled = neg_frac * 1e6;
+    key[u] = ordered_u64(scaled + static_cast<double>(psv[u]));
+    quota[u] = static_cast<int64_t>(base);
+    local += tid + kGroupThreads * u < nb ? quota[u] : 0;
   }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) local += __shfl_xor(local, off, 64);
-  const int64_t extra = a.committed[b] + a.k[b] - local;
-  if (extra <= 0) return;
+  if (lane == 0) sh.red[w] = local;
+  __syncthreads();
+  int64_t extra = want;
+#pragma unroll
+  for (int i = 0; i < kGroupThreads / 64; ++i) extra -= sh.red[i];
+  // key & mask < prefix: one more; key & mask == prefix: the first `take` of them in block order.
+  uint64_t prefix = 0, mask = 0;
+  int take = 0;
+  bool all_ties = true;
   if (extra >= nb) {
-    for (int64_t j = lane; j < nb; j += 64) tg[j] += 1;
-    return;
-  }
-  wave_sync_lds();
-  // Threshold key T and how many T-ties to take (remaining) after the last digit.
-  uint64_t prefix = 0, hi_mask = 0;
-  int64_t remaining = extra;
-  for (int shift = 56; shift >= 0; shift -= 8) {
+    take = nb;  // every block (mask 0: all keys tie)
+  } else if (extra > 0) {
+    take = static_cast<int>(extra);
+    all_ties = false;
+    for (int shift = 56; shift >= 0 && !all_ties; shift -= 8) {
+      sh.hist[tid] = 0u;
+      __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 4; ++q) hist[4 * lane + q] = 0u;
-    wave_sync_lds();
-    for (int64_t j = lane; j < nb; j += 64) {
-      const uint64_t key = skey[j];
-      if ((key & hi_mask) == prefix) atomicAdd(&hist[(key >> shift) & 0xff], 1u);
-    }
-    wave_sync_lds();
-    const uint32_t hs[4] = {hist[4 * lane], hist[4 * lane + 1], hist[4 * lane + 2], hist[4 * lane + 3]};
-    const int64_t mine = static_cast<int64_t>(hs[0]) + hs[1] + hs[2] + hs[3];
-    int64_t incl = mine;
+      for (int u = 0; u < kPer; ++u) {
+        if (tid + kGroupThreads * u < nb && (key[u] & mask) == prefix) atomicAdd(&sh.hist[(key[u] >> shift) & 0xff], 1u);
+      }
+      __syncthreads();
+      // Every wave scans the bins for itself (four a lane): the bin that holds the take-th key.
+      const uint4 h4 = *reinterpret_cast<const uint4*>(&sh.hist[4 * lane]);
+      const int hs[4] = {static_cast<int>(h4.x), static_cast<int>(h4.y), static_cast<int>(h4.z), static_cast<int>(h4.w)};
+      const int mine = hs[0] + hs[1] + hs[2] + hs[3];
+      int incl = mine;
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int64_t up = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += up;
-    }
-    // The lane whose four bins hold the remaining-th key finds the bin; everyone reads it from that lane.
-    const uint64_t who = __ballot(incl - mine < remaining && remaining <= incl);
-    const int src = __builtin_ctzll(who);
-    int64_t before = incl - mine;
-    int bin = 4 * lane + 3;
-    bool found = false;
+      for (int off = 1; off < 64; off <<= 1) {
+        const int up = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += up;
+      }
+      const uint64_t who = __ballot(incl - mine < take && take <= incl);
+      const int src = __builtin_ctzll(who);
+      int before = incl - mine, bin = 4 * lane, held = hs[0];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (!found) {
-        if (before + hs[q] < remaining) {
+      for (int q = 0; q < 3; ++q) {
+        if (bin == 4 * lane + q && before + hs[q] < take) {
           before += hs[q];
-        } else {
-          bin = 4 * lane + q;
-          found = true;
+          bin = 4 * lane + q + 1;
+          held = hs[q + 1];
         }
       }
+      prefix |= static_cast<uint64_t>(__builtin_amdgcn_readlane(bin, src)) << shift;
+      take -= __builtin_amdgcn_readlane(before, src);
+      mask |= 0xffull << shift;
+      all_ties = take == __builtin_amdgcn_readlane(held, src);
+      __syncthreads();  // the bins have been read
     }
-    prefix |= static_cast<uint64_t>(__shfl(bin, src, 64)) << shift;
-    remaining -= __shfl(before, src, 64);
-    hi_mask |= static_cast<uint64_t>(0xff) << shift;
-    wave_sync_lds();
   }
-  // key < T: one more; key == T: the first `remaining` in block order.
-  int64_t ties_before = 0;
-  for (int64_t j0 = 0; j0 < nb; j0 += 64) {
-    const int64_t j = j0 + lane;
-    const uint64_t key = j < nb ? skey[j] : ~0ull;
-    const bool tie = j < nb && key == prefix;
-    const uint64_t tb = __ballot(tie);
-    const int64_t rank = ties_before + __popcll(tb & ((1ull << lane) - 1ull));
-    if (j < nb && (key < prefix || (tie && rank < remaining))) tg[j] += 1;
-    ties_before += __popcll(tb);
+  if (take > 0 && !all_ties) {
+    // More keys equal the threshold than are taken: their ranks in block order.
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const uint64_t tb = __ballot(tid + kGroupThreads * u < nb && key[u] == prefix);
+      if (lane == 0) sh.ties[(kGroupThreads * u + tid) >> 6] = static_cast<uint32_t>(__popcll(tb));
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int j = tid + kGroupThreads * u;
+    const uint64_t high = key[u] & mask;
+    bool more = take > 0 && (high < prefix || (high == prefix && all_ties));
+    if (take > 0 && !all_ties) {
+      const uint64_t tb = __ballot(j < nb && key[u] == prefix);
+      int rank = __popcll(tb & ((1ull << lane) - 1ull));
+      for (int i = 0; i < (j >> 6); ++i) rank += static_cast<int>(sh.ties[i]);
+      more = more || (key[u] == prefix && rank < take);
+    }
+    if (j < nb) tg[j] = quota[u] + (more ? 1 : 0);
   }
 }
 
-// Standalone: one wave per window, 4 windows per workgroup.
-__global__ __launch_bounds__(256) void apportion_wave_kernel(ApportionArgs a, int64_t batch) {
-  __shared__ uint64_t skey[4][kWaveBlocks];
-  __shared__ uint32_t hist[4][256];
-  const int w = threadIdx.x >> 6;
-  const int64_t b = static_cast<int64_t>(blockIdx.x) * 4 + w;
-  if (b >= batch) return;
-  apportion_window(a, b, threadIdx.x & 63, skey[w], hist[w]);
+// Standalone: one workgroup per window.
+__global__ __launch_bounds__(kGroupThreads) void apportion_group_kernel(ApportionArgs a) {
+  __shared__ __attribute__((aligned(16))) ApportionShared sh;
+  apportion_group(a, blockIdx.x, sh);
 }
 
 // ------------------------------------------------------------------------------------------ in-block selection
@@ -903,14 +910,14 @@ __global__ __launch_bounds__(256) void committed_kernel(const uint8_t* __restric
   if (threadIdx.x == 0) committed[b] = red[0] + red[1] + red[2] + red[3];
 }
 
-// Apportionment alone (the fused entropy pass runs it on the side when the window has at most kWaveBlocks
+// Apportionment alone (the fused entropy pass runs it on the side when the window has at most kGroupBlocks
 // blocks).
 static int launch_apportion(int64_t batch, const Geometry& g, const int64_t* k, const int64_t* pos,
                             const double* frac, const int64_t* n_total, const int64_t* committed, const QuotaWs& w,
                             hipStream_t s, const char* name) {
-  if (g.nb <= kWaveBlocks) {
+  if (g.nb <= kGroupBlocks) {
     const ApportionArgs a{n_total, pos, frac, k, committed, g.nb, w.target};
-    apportion_wave_kernel<<<static_cast<unsigned>(cdiv(batch, 4)), 256, 0, s>>>(a, batch);
+    apportion_group_kernel<<<static_cast<unsigned>(batch), kGroupThreads, 0, s>>>(a);
   } else {
     apportion_kernel<<<static_cast<unsigned>(batch), kWG, 0, s>>>(n_total, pos, frac, k, committed, g.nb, w.keys,
                                                                    w.target);
@@ -971,16 +978,15 @@ struct KeyStore {
   }
 };
 
-// Workgroups [0, side) apportion window blockIdx.x (one wave); the rest run the entropy pass over the logits and
+// Workgroups [0, side) apportion window blockIdx.x; the rest run the entropy pass over the logits and
 // write the keys. The apportionment depends only on the selection state, so it runs alongside the HBM-bound pass.
 template <typename T, int LAYOUT, int NV, int LPV = 16, int CMAX = 256>
 __global__ __launch_bounds__(256) void ease_stats_kernel(const T* __restrict__ x, int64_t batch, int64_t n, int64_t C,
                                                          int64_t sb, int64_t sc, int64_t sn, KeyStore ks,
                                                          ApportionArgs ap, int side, VoxelRows rows, int nv = 0) {
-  __shared__ uint64_t skey[kWaveBlocks];
-  __shared__ uint32_t hist[256];
+  __shared__ __attribute__((aligned(16))) ApportionShared sh;
   if (static_cast<int>(blockIdx.x) < side) {
-    if (threadIdx.x < 64) apportion_window(ap, blockIdx.x, threadIdx.x, skey, hist);
+    apportion_group(ap, blockIdx.x, sh);
     return;
   }
   const int64_t blk = blockIdx.x - side, nblk = gridDim.x - side;
@@ -1093,8 +1099,8 @@ static int ease_select_impl(const void* logits, int dtype, int64_t classes, int6
   }
   const QuotaWs w = carve(workspace, batch, g);
   hipStream_t s = as_stream(stream);
-  // Windows of at most kWaveBlocks blocks are apportioned by side workgroups of the entropy pass.
-  const int side = g.nb <= kWaveBlocks ? static_cast<int>(batch) : 0;
+  // Windows of at most kGroupBlocks blocks are apportioned by side workgroups of the entropy pass.
+  const int side = g.nb <= kGroupBlocks ? static_cast<int>(batch) : 0;
   if (side == 0) {
     rc = launch_apportion(batch, g, k, pos, frac, n_total, committed, w, s, name);
     if (rc != SVHIP_OK) return rc;

@@ -388,3 +388,28 @@ def test_ease_select_bit_identical_from_class_planes_and_voxel_rows(dev):
     assert torch.equal(sels[0].scores.view(torch.int32), sels[1].scores.view(torch.int32))
     assert torch.equal(sels[0].chosen, sels[1].chosen)
     assert not bool(sels[0].bad.any())
+
+
+@pytest.mark.parametrize('Y,Z,X', [(4, 4, 4), (4, 16, 16), (100, 16, 16), (256, 16, 16)])
+@pytest.mark.parametrize('repeat', [1, 7, 4096])
+def test_apportionment_with_colliding_keys(dev, Y, Z, X, repeat):
+    """Blocks of equal fraction and equal position collide and share the extra voxels in block order: 1, 16, 400 and
+    1024 blocks, positions repeated `repeat` times (all equal at the largest), extra counts from none to every block
+    and past it. Bit-exact against the oracle."""
+    from streamvoxel_amd.sampling.block_quota import quota_select
+    b, shape = 4, (Y, Z, X)
+    nb = Y * Z * X // 64
+    g = np.random.default_rng(nb + repeat)
+    pos = (np.arange(nb, dtype=np.int64) // repeat)[g.permutation(nb)]
+    n_total = np.full(nb, 64, np.int64)
+    score = -g.random(shape).astype(np.float32)
+    selectable = np.ones(shape, bool)
+    frac = 0.1
+    base = int(np.floor(frac * 64 + 1e-9)) * nb
+    for extra in sorted({0, 1, nb // 3, nb - 1, nb, nb + 5}):
+        k = base + extra
+        _case(f'apportion nb={nb} repeat={repeat} extra={extra}')
+        expect = S.quota_select_nosync(score, selectable, k, b, pos, frac, n_total, 0)
+        res = quota_select(torch.from_numpy(score).to(dev), torch.from_numpy(selectable).to(dev), k, b,
+                           torch.from_numpy(pos).to(dev), frac, torch.from_numpy(n_total).to(dev), 0)
+        assert np.array_equal(res.cpu().numpy(), expect), extra
