@@ -108,7 +108,7 @@ class CachedContext:
 
     def set_length(self, index, length):
         self.host_lengths[index] = int(length)
-        self.lengths[index] = int(length)
+        self.lengths[index].fill_(int(length))   # a fill on the stream; an item assignment copies from the host
 
     def attend(self, layer, query, out=None, n=None):
         """Attention of `query` [n,H,Q,D] (bf16) over the cached keys of the first n windows."""

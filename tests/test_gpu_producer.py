@@ -193,3 +193,48 @@ def test_kv_write_row_major_v_and_e4m3_codes(dev):
     assert torch.equal(outs[False], outs[True])
     # Every e4m3 magnitude code 0..0x7e appears among the K codes.
     assert set(range(0x7f)) <= set(np.unique(ck_want.numpy() & 0x7f).tolist())
+
+
+@pytest.mark.parametrize('H,D,Pn,L,kcap', [(1, 48, 0, 1, 1), (5, 48, 63, 66, 131), (4, 96, 64, 64, 192),
+                                           (3, 120, 1, 200, 257), (6, 128, 130, 0, 130), (2, 8, 5, 70, 77)])
+@pytest.mark.parametrize('fp8', [False, True])
+@pytest.mark.parametrize('vt', [False, True])
+def test_kv_write_16_byte_runs_against_pairs(dev, H, D, Pn, L, kcap, fp8, vt):
+    """Rows of 16-byte runs take the vector kernels, local keys moved by two elements the pair kernels: the same
+    codes, scales and zero tail from both (head counts that leave a group part full, the widths where a group holds
+    fewer heads, tiles that mix prefix, local and empty keys, capacities that end inside a run)."""
+    from streamvoxel_amd import _lib
+    _case(f'kv_write runs H={H} D={D} P={Pn} L={L} kcap={kcap} fp8={fp8} vt={vt}')
+    g = torch.Generator().manual_seed(H * D + L)
+    normal = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(dev)
+    pk, pv, lk, lv = normal(H, Pn, D), normal(H, Pn, D), normal(H, L, D), normal(H, L, D)
+    rotate = D % 6 == 0 and L > 0
+    pos = (torch.randint(0, 4096, (L, 3), generator=g).float() / 8).to(dev) if rotate else None
+    freq = P.rope_frequencies(D).to(dev) if rotate else None
+    lib = _lib.load()
+    nbytes = int(lib.svhip_kv_write_workspace_bytes(H, kcap))
+    code, dtype = (_lib.SVHIP_FP8_E4M3, torch.uint8) if fp8 else (_lib.SVHIP_BF16, torch.int16)
+    row = kcap + (-kcap) % 16                     # V^T rows on 16-byte boundaries
+    outs = []
+    for shift in (0, 2):
+        def moved(t):
+            buf = torch.zeros(t.numel() + 8, dtype=t.dtype, device=dev)
+            view = buf[shift:shift + t.numel()].view(t.shape)
+            view.copy_(t)
+            return view
+        k, v = moved(lk), moved(lv)
+        ck = torch.full((H, kcap, D), 0x55, dtype=dtype, device=dev)
+        cv = torch.full((H, D, row) if vt else (H, kcap, D), 0x55, dtype=dtype, device=dev)
+        scv = (cv.stride(0), 1, cv.stride(1)) if vt else (cv.stride(0), cv.stride(1), 1)
+        ks, vs = torch.zeros(H, device=dev), torch.zeros(H, device=dev)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        _lib.check(lib.svhip_kv_write(
+            _lib.ptr(pk) if Pn else None, _lib.ptr(pv) if Pn else None, Pn, pk.stride(0), pk.stride(1), pv.stride(0),
+            pv.stride(1), _lib.ptr(k) if L else None, _lib.ptr(v) if L else None, L, k.stride(0), k.stride(1),
+            v.stride(0), v.stride(1), _lib.ptr(pos), 3, _lib.ptr(freq), H, D, _lib.ptr(ck), ck.stride(0),
+            ck.stride(1), _lib.ptr(cv), *scv, kcap, code, _lib.ptr(ks), _lib.ptr(vs), _lib.ptr(ws), nbytes,
+            _lib.stream_of(ck)), 'svhip_kv_write')
+        torch.cuda.synchronize()
+        outs.append((ck, cv, ks, vs))
+    # V^T's padding past the capacity is left as it was by both.
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
