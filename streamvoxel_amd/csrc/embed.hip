@@ -9,17 +9,21 @@
 // offset order, rounded to bf16, then the bias is added in bf16 (one more rounding), as embedding_bag(mode='sum')
 // followed by `out + bias` compute it in bf16.
 //
-// Workgroup = 8 patch tokens of one window, 32 lanes per token, each lane 16-byte column chunks lane + 32 c; the
-// table rows (reused across the batch) are gathered OB offsets at a time (8, or 4 for rows wider than 768) so that
-// OB loads per chunk are in flight.
+// Bound: 64 gathered rows a token (805 MB of 16-byte gathers for 8 windows at width 768), from the L2s; the table
+// (30 MB) does not fit an XCD's 4 MB. So the columns are cut into 8 slices, one per XCD (consecutive workgroups go
+// round robin to the XCDs): an XCD gathers from its slice of the table only (3.75 MB at width 768), and the rows of the
+// few cells that fill a window (the mask token, air) stay in the CUs' L1. A lane holds one 16-byte column chunk of one
+// token and takes the offsets in order, kEmbedBatch loads in flight. 8 windows, width 768, half of the voxels masked:
+// 44.3 us with whole rows per workgroup (18 TB/s of gathers), 34.8 us here (23 TB/s); 16 loads in flight 35.4 us.
 #include "common.hpp"
 
 namespace svhip {
 
 constexpr int kEmbedThreads = 256;
-constexpr int kEmbedLanes = 32;                              // lanes per patch token
-constexpr int kEmbedTokens = kEmbedThreads / kEmbedLanes;  // patch tokens per workgroup
-constexpr int kEmbedMaxOffsets = 64;                        // p^3 up to 4^3
+constexpr int kEmbedSlices = 8;         // column slices, one per XCD
+constexpr int kEmbedBatch = 8;          // table loads a lane has in flight
+constexpr int kEmbedMaxTokens = 64;     // patch tokens per workgroup
+constexpr int kEmbedMaxOffsets = 64;    // p^3 up to 4^3
 constexpr int kEmbedMaxWidth = 2048;
 
 struct EmbedArgs {
@@ -30,91 +34,88 @@ struct EmbedArgs {
   int64_t B, Y, Z, X, p, cells, W;
   int64_t stb, sob, son;
   int* bad;               // set when a token lies outside [0, cells)
+  int slice_chunks;       // 16-byte chunks of a column slice
+  int wg_tokens;          // patch tokens of a workgroup: kEmbedThreads / slice_chunks, at most kEmbedMaxTokens
 };
 
-template <int CPL>
+// P: the patch edge 4 at compile time (the index arithmetic of the table rows is a third of the work otherwise), or 0.
+template <int P>
 __global__ __launch_bounds__(kEmbedThreads) void patch_embed_kernel(EmbedArgs a) {
-  constexpr int OB = CPL <= 3 ? 8 : 4;
-  __shared__ int s_row[kEmbedTokens][kEmbedMaxOffsets];  // table row of every (token, offset)
-  const int64_t gy = a.Y / a.p, gz = a.Z / a.p, gx = a.X / a.p;
-  const int64_t per_window = gy * gz * gx;
-  const int64_t first = static_cast<int64_t>(blockIdx.x) * kEmbedTokens;  // flat (b, n) of slot 0
-  const int p3 = static_cast<int>(a.p * a.p * a.p);
-  for (int i = threadIdx.x; i < kEmbedTokens * p3; i += kEmbedThreads) {
-    const int t = i / p3, o = i - t * p3;
-    const int64_t flat = first + t;
-    int row = 0;
-    if (flat < a.B * per_window) {
-      const int64_t b = flat / per_window, n = flat - b * per_window;
-      const int64_t py = n / (gz * gx), pz = (n / gx) % gz, px = n % gx;
-      const int dy = o / static_cast<int>(a.p * a.p), dz = (o / static_cast<int>(a.p)) % static_cast<int>(a.p);
-      const int dx = o % static_cast<int>(a.p);
-      const int64_t y = py * a.p + dy, z = pz * a.p + dz, x = px * a.p + dx;
-      int64_t cell = a.tokens[b * a.stb + (y * a.Z + z) * a.X + x];
-      if (cell < 0 || cell >= a.cells) {
-        atomicOr(a.bad, 1);
-        cell = 0;
-      }
-      row = static_cast<int>(cell) * p3 + o;
-    }
-    s_row[t][o] = row;
+  // Table row of every (token, offset); offsets past p^3 are never read.
+  // (in 16-byte units).
+  __shared__ __attribute__((aligned(16))) uint32_t s_row[kEmbedMaxTokens][kEmbedMaxOffsets + 4];
+  __shared__ int64_t s_base[kEmbedMaxTokens];  // element of every token's first voxel
+  const int p = P ? P : static_cast<int>(a.p), p3 = p * p * p;
+  const uint32_t gx = static_cast<uint32_t>(a.X / p), gzx = static_cast<uint32_t>(a.Z / p) * gx;
+  const uint32_t per_window = static_cast<uint32_t>(a.Y / p) * gzx;  // B per_window < 2^31 (checked by the host)
+  const int slice = static_cast<int>(blockIdx.x % kEmbedSlices);
+  const uint32_t first = blockIdx.x / kEmbedSlices * a.wg_tokens;  // flat (b, n) of token 0
+  const int chunks = static_cast<int>(a.W / 8);
+  const int chunk0 = slice * a.slice_chunks;
+  if (chunk0 >= chunks) return;
+  const int count = min(static_cast<int>(static_cast<uint32_t>(a.B) * per_window - first), a.wg_tokens);
+  if (static_cast<int>(threadIdx.x) < count) {
+    const uint32_t flat = first + threadIdx.x;
+    const uint32_t b = flat / per_window, n = flat - b * per_window;
+    const uint32_t py = n / gzx, zx = n - py * gzx, pz = zx / gx, px = zx - pz * gx;
+    s_base[threadIdx.x] = b * a.stb + (static_cast<int64_t>(py) * a.Z + pz) * p * a.X + static_cast<int64_t>(px) * p;
   }
   __syncthreads();
-  const int t = threadIdx.x / kEmbedLanes, lane = threadIdx.x % kEmbedLanes;
-  const int64_t flat = first + t;
-  if (flat >= a.B * per_window) return;
-  const int chunks = static_cast<int>(a.W / 8);
-  float acc[CPL][8];
-#pragma unroll
-  for (int c = 0; c < CPL; ++c) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[c][j] = 0.f;
-  }
-  for (int o0 = 0; o0 < p3; o0 += OB) {
-    uint4 w[OB][CPL];
-#pragma unroll
-    for (int u = 0; u < OB; ++u) {
-      const int o = o0 + u;
-      const uint16_t* src = a.table + static_cast<int64_t>(s_row[t][o < p3 ? o : 0]) * a.W;
-#pragma unroll
-      for (int c = 0; c < CPL; ++c) {
-        const int ch = lane + kEmbedLanes * c;
-        w[u][c] = (o < p3 && ch < chunks) ? *reinterpret_cast<const uint4*>(src + 8 * ch)
-                                          : make_uint4(0u, 0u, 0u, 0u);
-      }
+  const uint32_t row_units = static_cast<uint32_t>(chunks);
+  for (int i = threadIdx.x; i < count * p3; i += kEmbedThreads) {
+    const int t = i / p3, o = i - t * p3;  // with P = 4 a thread keeps its offset o
+    const int dy = o / (p * p), dz = (o / p) % p, dx = o % p;
+    int64_t cell = a.tokens[s_base[t] + (dy * a.Z + dz) * a.X + dx];
+    if (cell < 0 || cell >= a.cells) {
+      atomicOr(a.bad, 1);
+      cell = 0;
     }
-    // Offsets in order: the sum of each column is taken o = 0, 1, 2, ... (zeros past p^3 leave it unchanged).
-#pragma unroll
-    for (int u = 0; u < OB; ++u) {
-#pragma unroll
-      for (int c = 0; c < CPL; ++c) {
-        const uint32_t e[4] = {w[u][c].x, w[u][c].y, w[u][c].z, w[u][c].w};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          acc[c][j] += bf16_bits_to_float(static_cast<uint16_t>(e[j >> 1] >> (16 * (j & 1))));
-        }
-      }
-    }
+    s_row[t][o] = (static_cast<uint32_t>(cell) * p3 + o) * row_units;
   }
-  const int64_t b = flat / per_window, n = flat - b * per_window;
-  uint16_t* dst = a.out + b * a.sob + n * a.son;
+  __syncthreads();
+  const int t = static_cast<int>(threadIdx.x) / a.slice_chunks;
+  const int ch = chunk0 + static_cast<int>(threadIdx.x) % a.slice_chunks;
+  if (t >= count || ch >= chunks) return;
+  const uint4* base = reinterpret_cast<const uint4*>(a.table) + ch;
+  float acc[8];
 #pragma unroll
-  for (int c = 0; c < CPL; ++c) {
-    const int ch = lane + kEmbedLanes * c;
-    if (ch >= chunks) continue;
-    uint32_t out[4];
+  for (int j = 0; j < 8; ++j) acc[j] = 0.f;
+  auto add = [&](const uint4& w) __attribute__((always_inline)) {
+    const uint32_t e[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-    for (int j = 0; j < 8; j += 2) {
-      float v0 = acc[c][j], v1 = acc[c][j + 1];
-      bf16_round2(v0, v1);
-      if (a.bias) {
-        v0 += bf16_bits_to_float(a.bias[8 * ch + j]);
-        v1 += bf16_bits_to_float(a.bias[8 * ch + j + 1]);
-      }
-      out[j / 2] = bf16_pack2(v0, v1);
+    for (int j = 0; j < 4; ++j) {
+      acc[2 * j] += __uint_as_float(e[j] << 16);
+      acc[2 * j + 1] += __uint_as_float(e[j] & 0xffff0000u);
     }
-    *reinterpret_cast<uint4*>(dst + 8 * ch) = make_uint4(out[0], out[1], out[2], out[3]);
+  };
+  // Offsets in order: the sum of each column is taken o = 0, 1, 2, ...
+  int o0 = 0;
+  for (; o0 + kEmbedBatch <= p3; o0 += kEmbedBatch) {
+    uint4 w[kEmbedBatch];
+#pragma unroll
+    for (int u = 0; u < kEmbedBatch; ++u) {
+      w[u] = base[s_row[t][o0 + u]];
+    }
+#pragma unroll
+    for (int u = 0; u < kEmbedBatch; ++u) add(w[u]);
   }
+  for (; o0 < p3; ++o0) {
+    add(base[s_row[t][o0]]);
+  }
+  const uint32_t flat = first + t;
+  const uint32_t b = flat / per_window, n = flat - b * per_window;
+  uint32_t out[4];
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    float v0 = acc[j], v1 = acc[j + 1];
+    bf16_round2(v0, v1);
+    if (a.bias) {
+      v0 += bf16_bits_to_float(a.bias[8 * ch + j]);
+      v1 += bf16_bits_to_float(a.bias[8 * ch + j + 1]);
+    }
+    out[j / 2] = bf16_pack2(v0, v1);
+  }
+  *reinterpret_cast<uint4*>(a.out + b * a.sob + n * a.son + 8 * ch) = make_uint4(out[0], out[1], out[2], out[3]);
 }
 
 }  // namespace svhip
@@ -134,25 +135,25 @@ extern "C" int svhip_patch_embed(const int64_t* tokens, const void* table, const
                 kEmbedMaxOffsets);
   SVHIP_REQUIRE(W >= 8 && W % 8 == 0 && W <= kEmbedMaxWidth, "%s: width %lld unsupported (a multiple of 8 up to %d)",
                 name, (long long)W, kEmbedMaxWidth);
-  SVHIP_REQUIRE(cells * patch * patch * patch < (1ll << 31), "%s: table too large", name);
+  SVHIP_REQUIRE(cells * patch * patch * patch < (1ll << 31) && cells * patch * patch * patch * (W / 8) < (1ll << 32),
+                "%s: table too large", name);
   SVHIP_REQUIRE(reinterpret_cast<uintptr_t>(table) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
                     so_b % 8 == 0 && so_n % 8 == 0,
                 "%s: table and output rows must start on 16-byte boundaries", name);
   const int64_t tokens_total = B * (Y / patch) * (Z / patch) * (X / patch);
   if (tokens_total == 0) return SVHIP_OK;
+  const int64_t slice_chunks = cdiv(W / 8, kEmbedSlices);
+  const int64_t wg_tokens = kEmbedThreads / slice_chunks < kEmbedMaxTokens ? kEmbedThreads / slice_chunks
+                                                                          : kEmbedMaxTokens;
   EmbedArgs a{tokens, static_cast<const uint16_t*>(table), static_cast<const uint16_t*>(bias),
-              static_cast<uint16_t*>(out), B, Y, Z, X, patch, cells, W, st_b, so_b, so_n, bad};
-  const int64_t grid = cdiv(tokens_total, kEmbedTokens);
-  SVHIP_REQUIRE(grid < (1ll << 31), "%s: grid too large", name);
-  const int cpl = static_cast<int>(cdiv(W / 8, kEmbedLanes));
-  hipStream_t s = as_stream(stream);
-  const unsigned g = static_cast<unsigned>(grid);
-  switch (cpl) {
-    case 1: patch_embed_kernel<1><<<g, kEmbedThreads, 0, s>>>(a); break;
-    case 2: patch_embed_kernel<2><<<g, kEmbedThreads, 0, s>>>(a); break;
-    case 3: patch_embed_kernel<3><<<g, kEmbedThreads, 0, s>>>(a); break;
-    case 4: patch_embed_kernel<4><<<g, kEmbedThreads, 0, s>>>(a); break;
-    default: patch_embed_kernel<8><<<g, kEmbedThreads, 0, s>>>(a); break;
+              static_cast<uint16_t*>(out), B, Y, Z, X, patch, cells, W, st_b, so_b, so_n, bad,
+              static_cast<int>(slice_chunks), static_cast<int>(wg_tokens)};
+  const int64_t grid = cdiv(tokens_total, wg_tokens) * kEmbedSlices;
+  SVHIP_REQUIRE(grid < (1ll << 31) && tokens_total < (1ll << 31), "%s: grid too large", name);
+  if (patch == 4) {
+    patch_embed_kernel<4><<<static_cast<unsigned>(grid), kEmbedThreads, 0, as_stream(stream)>>>(a);
+  } else {
+    patch_embed_kernel<0><<<static_cast<unsigned>(grid), kEmbedThreads, 0, as_stream(stream)>>>(a);
   }
   SVHIP_LAUNCHED(name);
   return SVHIP_OK;

@@ -58,6 +58,28 @@ def test_gather_patch(dev, W, shape, C, p):
     assert bool(((out.cpu().double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize('W,shape,p', [(8, (12, 8, 4), 4), (72, (8, 8, 8), 4), (64, (6, 3, 9), 3), (2048, (4, 4, 8), 4),
+                                       (520, (5, 3, 2), 1)])
+def test_gather_patch_column_slices(dev, W, shape, p):
+    """Widths that leave column slices empty or part full, patch counts that leave a workgroup part full, patch edges
+    with offsets past a whole batch of loads: bit for bit torch's embedding bag plus the bias."""
+    from streamvoxel_amd.stream.forward import GatherPatch
+    _case(f'gather patch slices W={W} shape={shape} p={p}')
+    B, C = 3, 11
+    g = torch.Generator().manual_seed(W + p)
+    conv = torch.nn.Conv3d(C + 1, W, p, stride=p).to(torch.bfloat16).to(dev)
+    tokens = torch.randint(0, C + 1, (B, *shape), generator=g)
+    gp = GatherPatch(conv)
+    out = gp(tokens.to(dev))
+    Y, Z, X = shape
+    cells = tokens.reshape(B, Y // p, p, Z // p, p, X // p, p).permute(0, 1, 3, 5, 2, 4, 6).reshape(-1, p ** 3)
+    index = (cells * p ** 3 + torch.arange(p ** 3)).to(dev)
+    ref = (torch.nn.functional.embedding_bag(index, gp.table, mode='sum') + gp.bias).reshape(B, -1, W)
+    torch.cuda.synchronize()
+    assert int(gp.bad.item()) == 0
+    assert torch.equal(out, ref)
+
+
 def test_gather_patch_flags_tokens_out_of_range(dev):
     from streamvoxel_amd.stream.forward import GatherPatch
     _case('gather patch out-of-range token')
