@@ -185,6 +185,20 @@ int svhip_xattn_fwd(const void* q, const void* k, const void* v, void* o, int kv
                     int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* stream);
 
 /*
+ * svhip_xattn_fwd with scratch memory, with which the keys of a (window, head) may be split over several workgroups
+ * (few windows, or windows of different lengths, otherwise leave part of the chip idle): 16-byte aligned, at least
+ * svhip_xattn_workspace_bytes(B, H, Q, D, kv_cap) bytes, its content of no meaning before or after the call. The
+ * query returns 0 where these sizes are never split; a NULL workspace never splits. The parts are joined in fp32.
+ */
+size_t svhip_xattn_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap);
+int svhip_xattn_fwd_ws(const void* q, const void* k, const void* v, void* o, int kv_dtype, const int32_t* kv_len,
+                       const int32_t* cu_seqlens, const float* k_scale, const float* v_scale, int64_t B, int64_t H,
+                       int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q, int64_t sk_b,
+                       int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k, int64_t sv_d,
+                       int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* workspace,
+                       size_t workspace_bytes, void* stream);
+
+/*
  * svhip_xattn_fwd with a boolean key mask: key j of window b is attended iff kv_mask[b * sm_b + j] != 0 (bytes,
  * at least kv_cap per window; with cu_seqlens, j counts from the window's first row), within the window length
  * (kv_len[b], or the cu_seqlens length, or kv_cap when both are NULL; clamped to kv_cap, the width of the mask
@@ -198,6 +212,17 @@ int svhip_xattn_fwd_masked(const void* q, const void* k, const void* v, void* o,
                            int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q, int64_t sk_b,
                            int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k, int64_t sv_d,
                            int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* stream);
+
+/*
+ * svhip_xattn_fwd_masked with the scratch memory of svhip_xattn_fwd_ws (used where kv_len is given). kv_len may come
+ * with cu_seqlens here: a window then ends at the smaller of the two lengths.
+ */
+int svhip_xattn_fwd_masked_ws(const void* q, const void* k, const void* v, void* o, const uint8_t* kv_mask,
+                              int64_t sm_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B, int64_t H,
+                              int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q,
+                              int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k,
+                              int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* workspace,
+                              size_t workspace_bytes, void* stream);
 
 /*
  * The effective window lengths of a key mask: out[b] (int32, device) = 1 + the last key j < n_b with

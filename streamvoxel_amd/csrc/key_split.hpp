@@ -1,0 +1,224 @@
+// What the cross-attention kernels share: the tile of a workgroup, the window lengths and the key split.
+//
+// A kernel's parameters P carry B, H, Q, D, q_tiles, the window lengths (kv_len / cu_seqlens / kv_cap, kv_mask), the
+// output (o, so_*), v_scale, and for the split form `part` (the slots of the parts, [team][2][query tile] of
+// split_slot_floats(D) floats) and `teams` (teams of q_tiles workgroups in the grid, a multiple of kXcds).
+#pragma once
+
+#include "common.hpp"
+
+namespace svhip {
+
+constexpr int kQTile = 128;   // queries per workgroup
+constexpr int kKB = 64;       // keys per block
+constexpr int kThreads = 256;
+constexpr int kCusPerXcd = 32;  // MI355X: 8 XCDs x 32 CUs
+constexpr int kXcds = 8;
+// Key split: windows a plan covers (one lane each), the key blocks below which no window's keys are split, the
+// smallest range worth a team, and the rounds of resident workgroups above which, and the share of them filled from
+// which, the unsplit launch is kept.
+constexpr int kSplitMaxWindows = 64;
+constexpr int kSplitMinBlocks = 24;
+constexpr int kSplitMinRange = 6;
+constexpr int kSplitMaxRounds = 4;
+constexpr int kSplitFullPercent = 85;
+
+// Keys of window b.
+template <typename P>
+__device__ __forceinline__ int window_length(const P& p, int64_t b) {
+  int64_t L;
+  if (p.cu_seqlens) {
+    L = static_cast<int64_t>(p.cu_seqlens[b + 1]) - p.cu_seqlens[b];
+    if (p.kv_len && L > p.kv_len[b]) L = p.kv_len[b];  // cut at the last attended key
+  } else if (p.kv_len) {
+    L = p.kv_len[b];
+    if (L > p.kv_cap) L = p.kv_cap;
+  } else {
+    L = p.kv_cap;  // key-mask form without lengths: every key up to the capacity, the mask decides
+  }
+  if (p.kv_mask && L > p.kv_cap) L = p.kv_cap;  // the mask rows hold kv_cap keys
+  return L < 0 ? 0 : static_cast<int>(L);
+}
+
+// Key split. One workgroup per (window, head, query tile) leaves CUs idle when there are few of them (one window: 96
+// of 256 CUs, each a serial chain of 153 key blocks) or when the windows' lengths differ (the longest one's chain
+// runs on alone). The split form lays the key blocks of all (window, head) units end to end and cuts that line into
+// equal ranges, one per team; a team is q_tiles workgroups that walk the same keys for their own query tiles, on one
+// XCD, so its L2 still serves a block to all of them. The grid is what the chip holds at once, so every CU has the
+// same count of key blocks to do. A range that holds a unit whole writes its output; a part of a unit leaves O, its
+// running max and its row sum in fp32, in the team's slot 0 (the range starts inside the unit) or 1 (it only ends
+// inside it), and split_join_kernel joins the parts.
+// The lengths are on the device, so every workgroup forms the plan for itself: lane b holds window b's block count.
+struct SplitPlan {
+  int before, blocks;  // of lane b: blocks of one head in the windows before b, and in b
+  int total;           // blocks of the line
+  int teams;           // ranges the line is cut into
+  bool whole;          // every window is short: ranges are cut at unit boundaries
+};
+
+template <typename P>
+__device__ __forceinline__ SplitPlan split_plan(const P& p) {
+  SplitPlan s;
+  const int lane = threadIdx.x & 63;
+  s.blocks = lane < p.B ? (window_length(p, lane) + kKB - 1) / kKB : 0;
+  int incl = s.blocks, longest = s.blocks;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int up = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += up;
+    longest = max(longest, __shfl_xor(longest, off, 64));
+  }
+  s.before = incl - s.blocks;
+  s.total = __builtin_amdgcn_readlane(incl, 63) * static_cast<int>(p.H);
+  s.whole = __builtin_amdgcn_readfirstlane(longest) < kSplitMinBlocks;
+  s.teams = s.whole ? p.teams : min(p.teams, (s.total + kSplitMinRange - 1) / kSplitMinRange);
+  return s;
+}
+
+// First block (on the line) of team t's range (t <= teams).
+template <typename P>
+__device__ __forceinline__ int split_cut(const P& p, const SplitPlan& s, int t) {
+  if (!s.whole) return static_cast<int>(static_cast<int64_t>(s.total) * t / s.teams);
+  const int H = static_cast<int>(p.H), units = H * static_cast<int>(p.B);
+  const int u = static_cast<int>(static_cast<int64_t>(units) * t / s.teams);  // the range starts with unit u = b H + h
+  if (u >= units) return s.total;
+  const int b = u / H, h = u - b * H;
+  return H * __builtin_amdgcn_readlane(s.before, b) + h * __builtin_amdgcn_readlane(s.blocks, b);
+}
+
+// The window whose blocks hold position pos < total of the line.
+template <typename P>
+__device__ __forceinline__ int split_window(const P& p, const SplitPlan& s, int pos) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t at = __builtin_amdgcn_ballot_w64(lane < p.B && static_cast<int>(p.H) * s.before <= pos);
+  return __popcll(at) - 1;
+}
+
+// The workspace: the slots of the parts, then for every unit the first and last team that hold a part of it (last <
+// first where one range holds it whole), written by the workgroups that start the units.
+__device__ __forceinline__ void split_store(float* slot, int d0, int ql, float a, float b, float c, float d) {
+  *reinterpret_cast<float4*>(slot + (static_cast<int64_t>(d0 >> 2) * kQTile + ql) * 4) = make_float4(a, b, c, d);
+}
+
+__host__ __device__ __forceinline__ int64_t split_slot_floats(int64_t D) { return kQTile * (D + 2); }
+
+template <typename P>
+__device__ __forceinline__ int2* split_units(const P& p) {
+  return reinterpret_cast<int2*>(p.part + 2ll * p.teams * p.q_tiles * split_slot_floats(p.D));
+}
+
+// `first`: the unit's first block on the line. No range of a line that is cut inside units is empty (teams is at most
+// total / kSplitMinRange, rounded up), so the last team is the last t with floor(total t / teams) <= the last block.
+__device__ __forceinline__ int2 split_unit_teams(int team, int first, int unit_blocks, bool whole, int total, int teams) {
+  if (whole) return make_int2(0, -1);
+  return make_int2(team, static_cast<int>((static_cast<int64_t>(first + unit_blocks) * teams - 1) / total));
+}
+
+// Joins the parts of the units that the split kernel cut: O = sum_i w_i O_i, l = sum_i w_i l_i with w_i =
+// exp2(m_i - max m) over the parts in key order, then v_scale O / l in the output's type. Workgroup = (unit, query
+// tile, kJoinDims head_dim elements); a thread holds 4 of them of kJoinItems queries. The parts are read once, from the
+// last-level cache where they were just written, the loads of kJoinAhead parts in flight (one part at a time, with the
+// plan formed here again, the join took 18-23 us of a layer; now 11-14). Windows without keys get their zeros here.
+constexpr int kJoinDims = 32;
+constexpr int kJoinItems = kQTile * (kJoinDims / 4) / kThreads;
+constexpr int kJoinAhead = 3;
+template <typename T, typename P>
+__global__ __launch_bounds__(kThreads) void split_join_kernel(P p) {
+  const int u = static_cast<int>(blockIdx.x / p.q_tiles), qt = static_cast<int>(blockIdx.x % p.q_tiles);
+  const int H = static_cast<int>(p.H);
+  const int64_t b = u / H, h = u % H;
+  const bool empty = window_length(p, b) == 0;
+  const int2 teams = split_units(p)[u];  // (left as it was for an empty window)
+  const int t0 = empty ? 0 : teams.x, t1 = empty ? -1 : teams.y;
+  if (!empty && t1 < t0) return;  // one range holds the unit: its output is written
+  const int64_t slot_floats = split_slot_floats(p.D);
+  const int d0 = static_cast<int>(blockIdx.y) * kJoinDims + 4 * (threadIdx.x % (kJoinDims / 4));
+  if (d0 >= p.D) return;
+  const int ql0 = threadIdx.x / (kJoinDims / 4);
+  constexpr int kStep = kQTile / kJoinItems;  // queries between a thread's items
+  float m[kJoinItems], l[kJoinItems];
+  float4 o[kJoinItems];
+#pragma unroll
+  for (int i = 0; i < kJoinItems; ++i) {
+    m[i] = -INFINITY;
+    l[i] = 0.f;
+    o[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  for (int t = t0; t <= t1; t += kJoinAhead) {
+    float mi[kJoinAhead][kJoinItems], li[kJoinAhead][kJoinItems];
+    float4 oi[kJoinAhead][kJoinItems];
+#pragma unroll
+    for (int a = 0; a < kJoinAhead; ++a) {
+      // The first part is the one its team's range ends in (slot 1), the others begin their teams' ranges (slot 0).
+      const int ta = min(t + a, t1);
+      const float* slot = p.part + (static_cast<int64_t>(2 * ta + (ta == t0 ? 1 : 0)) * p.q_tiles + qt) * slot_floats;
+#pragma unroll
+      for (int i = 0; i < kJoinItems; ++i) {
+        const int ql = ql0 + i * kStep;
+        mi[a][i] = slot[kQTile * p.D + ql];
+        li[a][i] = slot[kQTile * (p.D + 1) + ql];
+        oi[a][i] = *reinterpret_cast<const float4*>(slot + (static_cast<int64_t>(d0 >> 2) * kQTile + ql) * 4);
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < kJoinAhead; ++a) {
+#pragma unroll
+      for (int i = 0; i < kJoinItems; ++i) {
+        if (t + a > t1 || li[a][i] == 0.f) continue;
+        const float mn = fmaxf(m[i], mi[a][i]);
+        const float x = __builtin_amdgcn_exp2f(m[i] - mn), y = __builtin_amdgcn_exp2f(mi[a][i] - mn);
+        m[i] = mn;
+        l[i] = l[i] * x + li[a][i] * y;
+        o[i].x = o[i].x * x + oi[a][i].x * y;
+        o[i].y = o[i].y * x + oi[a][i].y * y;
+        o[i].z = o[i].z * x + oi[a][i].z * y;
+        o[i].w = o[i].w * x + oi[a][i].w * y;
+      }
+    }
+  }
+  T* Op = static_cast<T*>(p.o) + b * p.so_b + h * p.so_h;
+  const float vs = p.v_scale ? p.v_scale[b * p.H + h] : 1.f;
+#pragma unroll
+  for (int i = 0; i < kJoinItems; ++i) {
+    const int64_t q = static_cast<int64_t>(qt) * kQTile + ql0 + i * kStep;
+    if (q >= p.Q) continue;
+    const float inv = l[i] == 0.f ? 0.f : vs / l[i];
+    if constexpr (sizeof(T) == 4) {
+      float* out = Op + q * p.so_q + d0;  // rows of any alignment
+      out[0] = o[i].x * inv;
+      out[1] = o[i].y * inv;
+      out[2] = o[i].z * inv;
+      out[3] = o[i].w * inv;
+    } else {
+      *reinterpret_cast<uint2*>(Op + q * p.so_q + d0) = make_uint2(bf16_pack2(o[i].x * inv, o[i].y * inv),
+                                                                   bf16_pack2(o[i].z * inv, o[i].w * inv));
+    }
+  }
+}
+
+// Teams of the split form for these sizes, or 0 where the launch keeps one workgroup per (window, head, query tile):
+// windows beyond one wave's lanes, no window long enough to be split, or query tiles that fill the rounds of resident
+// workgroups by themselves. There the longest-first order balances uneven windows as well, without the parts' 50 MB
+// (8 windows x 12 heads x 1024 queries, 768 tiles = one full round of 3 per CU: 223-230 us unsplit, 232-240 split; of
+// it the kernel 224-230 against 241 and the join 17). One window of 12 heads (96 tiles) goes from 105 to 53 us, the 512
+// tiles of 8 windows x 8 heads x 48 from 180 to 158.
+// resident: workgroups of the split kernel that a CU holds.
+inline int split_teams(int64_t B, int64_t H, int64_t Q, int64_t kv_cap, int resident) {
+  const int64_t q_tiles = cdiv(Q, kQTile);
+  const int64_t per_xcd = kCusPerXcd * resident, slots = kXcds * per_xcd;
+  if (B < 1 || B > kSplitMaxWindows || q_tiles < 1 || q_tiles > per_xcd / 4) return 0;
+  if (cdiv(kv_cap, kKB) < kSplitMinBlocks) return 0;
+  const int64_t tiles = B * H * q_tiles, rounds = cdiv(tiles, slots);
+  if (rounds > kSplitMaxRounds || tiles * 100 >= rounds * slots * kSplitFullPercent) return 0;
+  if (B * H * cdiv(kv_cap, kKB) >= (1ll << 31)) return 0;
+  return static_cast<int>(kXcds * (per_xcd / q_tiles));
+}
+
+inline size_t split_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap, int resident) {
+  const int64_t teams = split_teams(B, H, Q, kv_cap, resident);
+  return teams ? static_cast<size_t>(2 * teams * cdiv(Q, kQTile) * split_slot_floats(D)) * sizeof(float) +
+                     static_cast<size_t>(B * H) * sizeof(int2)
+               : 0;
+}
+
+}  // namespace svhip

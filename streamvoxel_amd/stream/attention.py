@@ -94,33 +94,40 @@ def attention(query, key, val, lengths=None, cu_seqlens=None, scale=None, k_scal
         raise ValueError('head_dim mismatch')
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     lib = _lib.load()
+    # Scratch for the parts of a window whose keys several workgroups share (none where these sizes never split).
+    width = kcap if key_mask is None or cu_seqlens is None else key_mask.shape[1]
+    nbytes = int(lib.svhip_xattn_workspace_bytes(B, H, Q, D, width))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device) if nbytes else None
     if key_mask is not None:
         if fp8:
             raise TypeError('the key mask takes bf16 K/V')
         if cu_seqlens is None and key_mask.shape[1] < kcap:
             raise ValueError(f'key_mask holds {key_mask.shape[1]} keys per window, the cache {kcap}')
         mask_cap = kcap if cu_seqlens is None else key_mask.shape[1]
-        if cu_seqlens is None:
-            # The windows' lengths cut at their last attended keys (the same output): the kernel ranks the
-            # windows by them, which balances the CUs when the mask, not `lengths`, holds the window lengths.
+        if cu_seqlens is None or nbytes:
+            # The windows' lengths cut at their last attended keys (the same output): the kernel shares the key
+            # blocks out by them, which balances the CUs when the mask, not `lengths`, holds the window lengths.
+            if cu_seqlens is not None:
+                lengths = cu_seqlens[1:] - cu_seqlens[:-1]
             cut = torch.empty(B, dtype=torch.int32, device=query.device)
             _lib.check(lib.svhip_mask_lengths(_lib.ptr(key_mask.view(torch.uint8)), key_mask.stride(0),
                                               _lib.ptr(lengths), B, mask_cap, _lib.ptr(cut), _lib.stream_of(query)),
                        'svhip_mask_lengths')
             lengths = cut
-        _lib.check(lib.svhip_xattn_fwd_masked(
+        _lib.check(lib.svhip_xattn_fwd_masked_ws(
             _lib.ptr(query), _lib.ptr(key), _lib.ptr(val), _lib.ptr(out), _lib.ptr(key_mask.view(torch.uint8)),
             key_mask.stride(0), _lib.ptr(lengths), _lib.ptr(cu_seqlens), B, H, Q, D, mask_cap,
             query.stride(0), query.stride(1), query.stride(2),
-            *sk, *sv, out.stride(0), out.stride(1), out.stride(2), scale, _lib.stream_of(query)),
-            'svhip_xattn_fwd_masked')
+            *sk, *sv, out.stride(0), out.stride(1), out.stride(2), scale, _lib.ptr(ws), nbytes,
+            _lib.stream_of(query)), 'svhip_xattn_fwd_masked')
         return out
     kp = key.view(torch.uint8) if fp8 else key
     vp = val.view(torch.uint8) if fp8 else val
-    _lib.check(lib.svhip_xattn_fwd(
+    _lib.check(lib.svhip_xattn_fwd_ws(
         _lib.ptr(query), _lib.ptr(kp), _lib.ptr(vp), _lib.ptr(out), code, _lib.ptr(lengths), _lib.ptr(cu_seqlens),
         _lib.ptr(k_scale), _lib.ptr(v_scale), B, H, Q, D, kcap, query.stride(0), query.stride(1), query.stride(2),
-        *sk, *sv, out.stride(0), out.stride(1), out.stride(2), scale, _lib.stream_of(query)), 'svhip_xattn_fwd')
+        *sk, *sv, out.stride(0), out.stride(1), out.stride(2), scale, _lib.ptr(ws), nbytes, _lib.stream_of(query)),
+        'svhip_xattn_fwd')
     return out
 
 

@@ -1,0 +1,142 @@
+"""The key split of the cross attention against the float64 oracle and against the unsplit launch of the same call.
+
+Window lengths where the split can go wrong: ranges that end on a unit's first and last block, one block past the
+length from which windows are split, empty windows between long ones, a single window cut into many parts, parts that
+a key mask empties. The bars are the unsplit kernels' (bf16 2e-2 and 1e-2 of the largest value: the
+parts are kept and joined in fp32, so the split adds no rounding of its own to them)."""
+import math
+
+import pytest
+import torch
+
+from oracle import attention as A
+
+pytestmark = pytest.mark.gpu
+
+EDGE = 24 * 64                      # the keys from which a window is split
+
+
+def _case(msg):
+    print(f'[gpu-case] {msg}', flush=True)
+
+
+@pytest.fixture(scope='module')
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip('no GPU')
+    import streamvoxel_amd
+    streamvoxel_amd.load()
+    return torch.device('cuda:0')
+
+
+def qkv(B, H, Q, kcap, D, seed, dtype, spread=1.0):
+    g = torch.Generator().manual_seed(seed)
+    s = spread / math.sqrt(D)
+    return [(torch.randn(B, H, n, D, generator=g) * s).to(dtype) for n in (Q, kcap, kcap)]
+
+
+def check(got, ref, atol, rtol):
+    err = (got.double().cpu() - ref).abs().max().item()
+    assert err <= atol and err <= rtol * ref.abs().max().item(), (err, ref.abs().max().item())
+
+
+LENGTHS = [[EDGE - 64, 1, 0, 700],                       # no window is split
+           [EDGE - 63], [EDGE], [EDGE + 1],              # the edge itself
+           [6000],                                       # one window, many parts
+           [0, 5000, 0, 0, 1, 4097, 64, 0],              # empty and short windows between long ones
+           [2048, 2048, 2048, 2048]]                     # equal ranges
+
+
+@pytest.mark.parametrize('lengths', LENGTHS, ids=lambda x: '-'.join(map(str, x)))
+@pytest.mark.parametrize('D,H,Q', [(48, 3, 130), (64, 4, 128), (96, 2, 257), (128, 1, 33)])
+def test_split_windows_match_the_oracle(dev, lengths, D, H, Q):
+    from streamvoxel_amd import _lib
+    from streamvoxel_amd.stream.attention import attention
+    _case(f'split bf16 D={D} H={H} Q={Q} lengths={lengths}')
+    B, kcap = len(lengths), max(lengths) + 5
+    kcap += -kcap % 8
+    q, k, v = qkv(B, H, Q, kcap, D, sum(lengths) + D, torch.bfloat16, 2.0)
+    assert int(_lib.load().svhip_xattn_workspace_bytes(B, H, Q, D, kcap)) > 0
+    ref = A.cross_attention(q, k, v, lengths)
+    lt = torch.tensor(lengths, dtype=torch.int32, device=dev)
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    out = attention(qd, kd, vd, lengths=lt)
+    out_t = attention(qd, kd, vd.transpose(2, 3).contiguous().transpose(2, 3), lengths=lt)
+    mask = torch.arange(kcap, device=dev)[None] < lt[:, None]
+    out_m = attention(qd, kd, vd, key_mask=mask)
+    cu = torch.tensor([0] + torch.tensor(lengths).cumsum(0).tolist(), dtype=torch.int32, device=dev)
+    kp, vp = (torch.cat([x[b, :, :n] for b, n in enumerate(lengths)], 1).contiguous() for x in (kd, vd))
+    out_p = attention(qd, kp, vp, cu_seqlens=cu)
+    torch.cuda.synchronize()
+    check(out, ref, 2e-2, 1e-2)
+    for b, n in enumerate(lengths):
+        if n == 0:
+            assert not out[b].any()
+    # Every layout of the same keys is cut alike and gives the same bits.
+    assert torch.equal(out, out_t) and torch.equal(out, out_m) and torch.equal(out, out_p)
+
+
+@pytest.mark.parametrize('D', [48, 64])
+def test_split_under_masks_with_holes(dev, D):
+    from streamvoxel_amd.stream.attention import attention
+    B, H, Q, kcap = 4, 3, 140, 4000
+    _case(f'split bf16 key mask D={D}')
+    q, k, v = qkv(B, H, Q, kcap, D, D, torch.bfloat16, 2.0)
+    g = torch.Generator().manual_seed(D)
+    mask = torch.rand(B, kcap, generator=g) < 0.5
+    mask[0, 200:3000] = False                     # whole parts of the window masked
+    mask[1] = False                               # no attended key at all
+    mask[2, :3900] = False                        # only the last part holds attended keys
+    scores = (q.double() @ k.double().transpose(2, 3)) / math.sqrt(D)
+    w = scores.masked_fill(~mask[:, None, None], -math.inf).softmax(-1).nan_to_num(0.0)
+    ref = w @ v.double()
+    out = attention(q.to(dev), k.to(dev), v.to(dev), key_mask=mask.to(dev))
+    torch.cuda.synchronize()
+    assert not out[1].any()
+    check(out, ref, 2e-2, 1e-2)
+
+
+def test_split_e4m3_against_unsplit(dev):
+    """The same e4m3 cache through the split call and through the C entry without a workspace."""
+    from streamvoxel_amd import _lib
+    from streamvoxel_amd.stream.attention import attention, quantize_e4m3
+    lengths = [4000, 0, 2500, 63]
+    B, H, Q, D, kcap = 4, 4, 200, 64, 4032
+    _case('split e4m3')
+    q, k, v = qkv(B, H, Q, kcap, D, 3, torch.bfloat16, 2.0)
+    (kc, ks), (vc, vs) = quantize_e4m3(k.to(dev)), quantize_e4m3(v.to(dev))
+    lt = torch.tensor(lengths, dtype=torch.int32, device=dev)
+    qd = q.to(dev)
+    for vt in (False, True):
+        val = vc.transpose(2, 3).contiguous().transpose(2, 3) if vt else vc
+        out = attention(qd, kc, val, lengths=lt, k_scale=ks, v_scale=vs)
+        one = torch.empty_like(out)
+        _lib.check(_lib.load().svhip_xattn_fwd(
+            _lib.ptr(qd), _lib.ptr(kc.view(torch.uint8)), _lib.ptr(val.view(torch.uint8)), _lib.ptr(one),
+            _lib.SVHIP_FP8_E4M3, _lib.ptr(lt), None, _lib.ptr(ks), _lib.ptr(vs), B, H, Q, D, kcap, *qd.stride()[:3],
+            *kc.stride()[:3], *val.stride(), *one.stride()[:3], 1 / math.sqrt(D), _lib.stream_of(qd)),
+            'svhip_xattn_fwd')
+        torch.cuda.synchronize()
+        check(out, one.double().cpu(), 2e-2, 1e-2)
+        assert not out[1].any()
+
+
+def test_split_replays_in_a_graph(dev):
+    """Captured: the scratch comes from the graph's pool, and lengths changed between replays are planned anew."""
+    from streamvoxel_amd.stream.attention import attention
+    B, H, Q, D, kcap = 2, 4, 128, 64, 6016
+    _case('split in a graph')
+    q, k, v = (x.to(dev) for x in qkv(B, H, Q, kcap, D, 9, torch.bfloat16, 2.0))
+    lt = torch.tensor([6000, 100], dtype=torch.int32, device=dev)
+    out = torch.empty_like(q)
+    attention(q, k, v, lengths=lt, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        attention(q, k, v, lengths=lt, out=out)
+    for lengths in ([6000, 100], [0, 6016], [64, 1500], [3000, 3001]):
+        lt.copy_(torch.tensor(lengths, dtype=torch.int32))
+        graph.replay()
+        want = attention(q, k, v, lengths=lt)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), lengths
