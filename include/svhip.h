@@ -238,8 +238,8 @@ int svhip_mask_lengths(const uint8_t* kv_mask, int64_t sm_b, const int32_t* kv_l
 /*
  * Cross attention in fp32 arithmetic: fp32 q/k/v/o with the layouts and strides of svhip_xattn_fwd (elements, not
  * bytes; rows 16-byte aligned; V as rows or as V^T), padded with kv_len or packed with cu_seqlens; head_dim 16, 32,
- * 48 or 64. Every product, sum and exponential is fp32 (the VALU; no rounding of the operands), at the fp32 FMA
- * rate. A window with no key gives zeros.
+ * 48 or 64. Every product, sum and exponential is fp32 (the products on the fp32 matrix cores; no rounding of the
+ * operands). A window with no key gives zeros.
  * Replaces: the SDPA of SlotCrossAttention.forward (streamvoxel/stream/engine.py:28-47) as the reference runs it on
  * fp32 tensors (its CPU path, the single-column configuration) where the window lengths hold its mask; any other
  * mask takes svhip_xattn_fwd_f32_masked.
@@ -264,6 +264,18 @@ int svhip_xattn_fwd_f32_masked(const float* q, const float* k, const float* v, f
                                int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q,
                                int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k,
                                int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* stream);
+
+/*
+ * The two fp32 forms (kv_mask may be NULL) with scratch memory for the key split, as svhip_xattn_fwd_ws has it: at
+ * least svhip_xattn_f32_workspace_bytes bytes, 16-byte aligned. The parts are kept and joined in fp32.
+ */
+size_t svhip_xattn_f32_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap);
+int svhip_xattn_fwd_f32_ws(const float* q, const float* k, const float* v, float* o, const uint8_t* kv_mask,
+                           int64_t sm_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B, int64_t H,
+                           int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q,
+                           int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k,
+                           int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* workspace,
+                           size_t workspace_bytes, void* stream);
 
 /*
  * AxialRoPE of bf16 activations: x [B,H,N,D] (element (b,h,n,d) at b*sx_b + h*sx_h + n*sx_n + d) -> out (same

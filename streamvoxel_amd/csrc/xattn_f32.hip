@@ -1,30 +1,41 @@
-// Cross attention in fp32 arithmetic: fp32 Q/K/V/O, every product, sum and exponential in fp32 on the VALU.
+// Cross attention in fp32 arithmetic: fp32 Q/K/V/O, every product, sum and exponential in fp32.
 //
 // The single-column configuration runs the reference's cross attention in fp32 (the masked SDPA of
 // SlotCrossAttention.forward, streamvoxel/stream/engine.py:28-47, on fp32 tensors). The bf16 kernel rounds its
-// operands to bf16 for the matrix cores; this one keeps the reference's arithmetic width, for callers that hand
-// over fp32 tensors and want fp32 results (it runs on the VALU at the fp32 FMA rate, well below the bf16 kernel's
-// throughput).
+// operands to bf16 for the matrix cores; this one keeps the reference's arithmetic width: both products are
+// v_mfma_f32_32x32x2_f32 (fp32 operands and accumulation, no rounding of either operand).
 //
-// Work item: one workgroup = (window b, head h, 64-query tile), 8 waves; lane l of every wave holds query l of the
-// tile (q and the running O in registers). Wave w takes the window's 16-key blocks w, w + 8, w + 16, ...: it
-// stages a block's K and V rows in its own LDS area (16-byte loads, the next block's loads in flight while the
-// current one is computed, keys >= L as zeros), reads each row back with one address for all lanes (an LDS
-// broadcast), forms the 16 scores, raises its running max m (log2 units) to the block's, rescales O and l once and
-// adds the 16 weighted V rows. The eight partial (m, l, O) are merged pairwise through LDS in three rounds.
+// Bound: the fp32 matrix cores (64 FLOP a cycle and SIMD, a sixteenth of bf16; a large fp32 matrix product reaches
+// 154 TFLOP/s on the card). A 32-key x 32-query half costs 64 of these products at head_dim 64 (4096 cycles) against
+// 16 exponentials, so the softmax and the LDS reads hide behind them; K and V are staged once for the workgroup's
+// 128 queries.
+//
+// Work item: one workgroup = (window b, head h, 128-query tile), 4 waves x 32 queries, 64-key blocks in LDS (the next
+// block's loads in flight in registers while the current one is computed). Per wave and 32-key half:
+//   S^T[key, q] = K . Q^T     A = K rows from LDS, B = the wave's Q (registers). The k order is free as long as both
+//                             operands share it: lane half hh takes head_dim 8 s + 4 hh + j at step 4 s + j, so a
+//                             lane reads K in 16-byte chunks.
+//   P^T = exp2(S^T - m)       online softmax, lane (col, hh) owns query col and the keys 8 (i / 4) + 4 hh + i % 4
+//   O^T[d, q] += V^T . P^T    step i pairs the keys of accumulator entry i of both lane halves, so P^T is the B
+//                             operand as it stands; A = V[that key][32 j + col] from LDS.
+// The split form (SPLIT) is the bf16 kernel's: see key_split.hpp.
+//
+// One window of 12 x 64 heads, 1024 queries, 9744 keys: 816 us on the VALU (one query a lane, K and V rows broadcast from
+// LDS: 37 TFLOP/s), 283 us here (108 TFLOP/s), 12 us of it the join. The matrix cores are busy 0.70 of the kernel: the
+// three waves of a SIMD do not finish together, and the last one alone does not fill them.
 //
 // KMASK: a key mask on top of the window length (the reference's `prefix_valid ++ local_valid`): key j of window b
-// is attended only where kv_mask[b * sm_b + j] != 0. A block's 16 mask bytes are read one per lane and gathered
-// by a ballot; a block (and every block before it) may then hold no attended key, so the running max may stay
-// -inf, against which nothing is added.
-#include "common.hpp"
+// is attended only where kv_mask[b * sm_b + j] != 0. A block that the mask wholly masks is skipped; a query may have
+// seen no attended key yet, its running max then stays -inf and the exponentials are taken against 0.
+#include "key_split.hpp"
 
 namespace svhip {
 
-constexpr int kF32Waves = 8;
-constexpr int kF32Threads = 64 * kF32Waves;
-constexpr int kF32Keys = 16;  // keys per block
-constexpr int kF32MaxD = 64;
+constexpr int kF32Row = 64;      // floats of an LDS row (one key)
+constexpr int kF32Resident = 3;  // workgroups per CU (three waves per SIMD)
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 struct XattnF32Params {
   const float* q;
@@ -34,230 +45,296 @@ struct XattnF32Params {
   const int32_t* kv_len;
   const int32_t* cu_seqlens;
   const uint8_t* kv_mask;  // KMASK: [B, kv_cap] bytes, rows sm_b apart
+  const float* v_scale;    // none (the join's output scale)
   int64_t sm_b;
-  int64_t B, H, Q, kv_cap;
+  int64_t B, H, Q, D, kv_cap;
   int64_t sq_b, sq_h, sq_q;
   int64_t sk_b, sk_h, sk_k;
   int64_t sv_b, sv_h, sv_k, sv_d;
   int64_t so_b, so_h, so_q;
   float scale_log2;  // softmax scale * log2(e)
   int q_tiles;
+  float* part;
+  int teams;
 };
+
+// LDS rows are 256 bytes, every bank once. K: 16 rows are read at one 16-byte chunk, so chunk c of row r lies at
+// c ^ (r % 16). V: a read takes 32 consecutive floats of row r in lane half 0 and of row r + 4 in half 1, so the
+// halves of the rows with bit 2 set are swapped.
+__device__ __forceinline__ int f32_swz_k(int r, int c) { return c ^ (r & 15); }
+__device__ __forceinline__ int f32_swz_v(int r, int c) { return c ^ (((r >> 2) & 1) << 3); }
 
 // VT: V given as V^T rows (keys contiguous, element (key, d) at d * sv_d + key), else V rows (head_dim
 // contiguous). Rows start 16-byte aligned (checked by the entry point).
-template <int D, bool VT, bool KMASK>
-__global__ __launch_bounds__(kF32Threads) void xattn_f32_kernel(XattnF32Params p) {
-  constexpr int kBlock = kF32Keys * D;   // floats of one staged K (or V) block
-  constexpr int kPer = kBlock / 256;     // float4 per lane and block
-  static_assert(kBlock % 256 == 0, "head_dim a multiple of 16");
-  // Staging (8 waves x K, V blocks, [key][d]) during the loop; the merge area ([wave][D + 2][lane] for four
-  // waves) afterwards.
-  constexpr int kStage = kF32Waves * 2 * kF32Keys * kF32MaxD;
-  constexpr int kMerge = 4 * (kF32MaxD + 2) * 64;
-  __shared__ __attribute__((aligned(16))) float s_buf[kStage > kMerge ? kStage : kMerge];
-  const int lane = threadIdx.x & 63;
+template <int D, bool VT, bool KMASK, bool SPLIT>
+__global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(XattnF32Params p) {
+  constexpr int kChunks = D / 4;                      // 16-byte chunks of a key's row
+  constexpr int kPer = kKB * kChunks / kThreads;      // chunks per thread and block
+  constexpr int kTiles = (D + 31) / 32;               // output tiles of 32 head_dim elements
+  static_assert(kKB * kChunks % kThreads == 0, "head_dim a multiple of 16");
+  __shared__ __attribute__((aligned(16))) float sK[kKB * kF32Row], sV[kKB * kF32Row];
+  [[maybe_unused]] __shared__ int s_before[SPLIT ? kSplitMaxWindows : 1], s_blocks[SPLIT ? kSplitMaxWindows : 1];
+  [[maybe_unused]] __shared__ int s_total, s_teams;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t unit = blockIdx.x / p.q_tiles;
-  const int qt = static_cast<int>(blockIdx.x % p.q_tiles);
-  const int64_t b = unit / p.H, h = unit % p.H;
-  int64_t L, off = 0;
-  if (p.cu_seqlens) {
-    off = p.cu_seqlens[b];
-    L = static_cast<int64_t>(p.cu_seqlens[b + 1]) - off;
-    if (KMASK && L > p.kv_cap) L = p.kv_cap;  // the mask rows hold kv_cap keys
+  const int wg = static_cast<int>(blockIdx.x);
+  int qt, team = 0, pos = 0, range_end = 0;
+  int64_t b = 0, h = 0;
+  if constexpr (SPLIT) {
+    const int seq = wg >> 3;
+    qt = seq % p.q_tiles;
+    team = (seq / p.q_tiles) * kXcds + (wg & 7);
+    const SplitPlan plan = split_plan(p);
+    if (team >= plan.teams) return;
+    pos = split_cut(p, plan, team);
+    range_end = split_cut(p, plan, team + 1);
+    if (pos >= range_end) return;
+    if (threadIdx.x < kSplitMaxWindows) {
+      s_before[threadIdx.x] = plan.before;
+      s_blocks[threadIdx.x] = plan.blocks;
+    }
+    if (threadIdx.x == 0) {
+      s_total = plan.total;
+      s_teams = plan.teams;
+    }
+    __syncthreads();
   } else {
-    L = p.kv_len ? p.kv_len[b] : p.kv_cap;    // no kv_len (key mask only): every key of the row
-    if (L > p.kv_cap) L = p.kv_cap;
+    qt = wg % p.q_tiles;
+    const int64_t unit = wg / p.q_tiles;
+    b = unit / p.H;
+    h = unit % p.H;
   }
-  if (L < 0) L = 0;
-  const uint8_t* mrow = KMASK ? p.kv_mask + b * p.sm_b : nullptr;
-  const int64_t q = static_cast<int64_t>(qt) * 64 + lane;
-  const bool q_ok = q < p.Q;
-  const float* K = p.k + (p.cu_seqlens ? 0 : b * p.sk_b) + h * p.sk_h + off * p.sk_k;
-  const float* V = p.v + (p.cu_seqlens ? 0 : b * p.sv_b) + h * p.sv_h + off * p.sv_k;
-  float* sK = s_buf + w * 2 * kBlock;
-  float* sV = sK + kBlock;
-
-  float qv[D], o[D];
-#pragma unroll
-  for (int d = 0; d < D; d += 4) {
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (q_ok) x = *reinterpret_cast<const float4*>(p.q + b * p.sq_b + h * p.sq_h + q * p.sq_q + d);
-    qv[d] = x.x;
-    qv[d + 1] = x.y;
-    qv[d + 2] = x.z;
-    qv[d + 3] = x.w;
-  }
-#pragma unroll
-  for (int d = 0; d < D; ++d) o[d] = 0.f;
   const float sl2 = p.scale_log2;
-  float m = -INFINITY, l = 0.f;
 
-  // Block loads: float4 r of this lane is element 4 (lane + 64 r) of the block: K row / V row (key, d) with
-  // d = e % D, or V^T row d = e / 16 at keys 4 ((e % 16) / 4) .. + 3 (4 consecutive keys of one head_dim element).
-  // Every load is issued (keys >= L read row L - 1, in bounds) and a select puts zeros there: no branch in the loop,
-  // so the compiler keeps each row's reads next to its products.
-  float4 nk[kPer], nv[kPer];
-  const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  auto load_block = [&](int64_t kv0) __attribute__((always_inline)) {
+  do {
+    // SPLIT: the thread index is opaque in every part, so that no part's addresses are kept through the key blocks.
+    int tid = threadIdx.x;
+    if constexpr (SPLIT) asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, col = lane & 31, hh = lane >> 5;
+    const int64_t q = static_cast<int64_t>(qt) * kQTile + w * 32 + col;
+    const bool q_ok = q < p.Q;
+    int blk0 = 0, blk1 = 0, unit_blocks = 0;
+    if constexpr (SPLIT) {
+      SplitPlan plan;
+      plan.before = s_before[lane];
+      plan.blocks = s_blocks[lane];
+      const int bw = split_window(p, plan, pos);
+      unit_blocks = __builtin_amdgcn_readlane(plan.blocks, bw);
+      const int rel = pos - static_cast<int>(p.H) * __builtin_amdgcn_readlane(plan.before, bw);
+      const int hw = rel / unit_blocks;
+      b = bw;
+      h = hw;
+      blk0 = rel - hw * unit_blocks;
+      blk1 = min(unit_blocks, blk0 + (range_end - pos));
+      pos += blk1 - blk0;
+      if (blk0 == 0 && qt == 0 && tid == 0) {
+        split_units(p)[b * p.H + h] =
+            split_unit_teams(team, pos - blk1, unit_blocks, blk1 == unit_blocks, s_total, s_teams);
+      }
+    }
+    const int L = window_length(p, b);
+    if constexpr (!SPLIT) blk1 = unit_blocks = (L + kKB - 1) / kKB;
+    const int64_t off = p.cu_seqlens ? p.cu_seqlens[b] : 0;
+    const uint8_t* mrow = KMASK ? p.kv_mask + b * p.sm_b : nullptr;
+    const float* K = p.k + (p.cu_seqlens ? 0 : b * p.sk_b) + h * p.sk_h + off * p.sk_k;
+    const float* V = p.v + (p.cu_seqlens ? 0 : b * p.sv_b) + h * p.sv_h + off * p.sv_k;
+
+    // Q as B operands: entry 4 s + j is head_dim 8 s + 4 hh + j.
+    float qf[D / 2];
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const int e = 4 * (lane + 64 * r);
-      const int64_t key = kv0 + e / D;
-      const int64_t kc = key < L ? key : L - 1;
-      const int d = e % D;
-      const float4 xk = *reinterpret_cast<const float4*>(K + kc * p.sk_k + d);
-      nk[r] = key < L ? xk : zero4;
-      if constexpr (VT) {
-        const int dv = e / kF32Keys;
-        const int64_t k4 = kv0 + (e % kF32Keys);
-        const float* row = V + dv * p.sv_d;
-        float xv[4];
+    for (int s = 0; s < D / 8; ++s) {
+      float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (q_ok) x = *reinterpret_cast<const float4*>(p.q + b * p.sq_b + h * p.sq_h + q * p.sq_q + 8 * s + 4 * hh);
+      qf[4 * s] = x.x;
+      qf[4 * s + 1] = x.y;
+      qf[4 * s + 2] = x.z;
+      qf[4 * s + 3] = x.w;
+    }
+    f32x16_t o[kTiles];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int64_t kj = k4 + j < L ? k4 + j : L - 1;
-          const float x = row[kj];
-          xv[j] = k4 + j < L ? x : 0.f;
+    for (int j = 0; j < kTiles; ++j) o[j] = f32x16_t{0};
+    float m = -INFINITY, l = 0.f;  // l: the lane's own keys
+
+    // Block loads: chunk c = thread + 256 r is key c / kChunks, head_dim 4 (c % kChunks) .. + 3 (of V^T key c % 64,
+    // head_dim 4 (c / 64) .. + 3: consecutive lanes read consecutive keys of a row). Every load is issued
+    // (keys >= L read row L - 1, in bounds); their scores are masked, and V rows past L are zeros so that 0 . V
+    // stays 0.
+    f32x4_t nk[kPer], nv[kPer];
+    auto load_block = [&](int kv0) __attribute__((always_inline)) {
+      // Opaque again: the chunks' addresses are formed per block (hidden behind the products); hoisted, they took 16
+      // registers and were spilled.
+      int tb = tid;
+      asm volatile("" : "+v"(tb));
+#pragma unroll
+      for (int r = 0; r < kPer; ++r) {
+        const int c = tb + kThreads * r;
+        const int key = kv0 + c / kChunks, d = 4 * (c % kChunks);
+        const int64_t kc = key < L ? key : L - 1;
+        nk[r] = *reinterpret_cast<const f32x4_t*>(K + kc * p.sk_k + d);
+        if constexpr (VT) {
+          const int kt = kv0 + c % kKB;
+          const float* src = V + 4 * (c / kKB) * p.sv_d + (kt < L ? kt : L - 1);
+          nv[r] = f32x4_t{src[0], src[p.sv_d], src[2 * p.sv_d], src[3 * p.sv_d]};
+          if (kt >= L) nv[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        } else {
+          nv[r] = *reinterpret_cast<const f32x4_t*>(V + kc * p.sv_k + d);
+          if (key >= L) nv[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
-        nv[r] = make_float4(xv[0], xv[1], xv[2], xv[3]);
+      }
+    };
+    auto store_block = [&]() __attribute__((always_inline)) {
+      int tb = tid;
+      asm volatile("" : "+v"(tb));
+#pragma unroll
+      for (int r = 0; r < kPer; ++r) {
+        const int c = tb + kThreads * r;
+        const int key = c / kChunks, dc = c % kChunks;
+        *reinterpret_cast<f32x4_t*>(sK + key * kF32Row + 4 * f32_swz_k(key, dc)) = nk[r];
+        const int vkey = VT ? c % kKB : key, vc = VT ? c / kKB : dc;
+        *reinterpret_cast<f32x4_t*>(sV + vkey * kF32Row + 4 * f32_swz_v(vkey, vc)) = nv[r];
+      }
+    };
+    // Bit i: key kv0 + i is below L and attended (wave-uniform; lane i's byte).
+    auto load_mask = [&](int kv0) __attribute__((always_inline)) -> int {
+      const int j = kv0 + lane;
+      if constexpr (KMASK) {
+        const int jc = j < L ? j : L - 1;
+        return (mrow[jc] != 0 && j < L) ? 1 : 0;
       } else {
-        const float4 xv = *reinterpret_cast<const float4*>(V + kc * p.sv_k + d);
-        nv[r] = key < L ? xv : zero4;
+        return j < L ? 1 : 0;
       }
-    }
-  };
-  auto store_block = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      const int e = 4 * (lane + 64 * r);
-      *reinterpret_cast<float4*>(sK + e) = nk[r];
-      if constexpr (VT) {
-        const int dv = e / kF32Keys, kk = e % kF32Keys;
-        sV[kk * D + dv] = nv[r].x;
-        sV[(kk + 1) * D + dv] = nv[r].y;
-        sV[(kk + 2) * D + dv] = nv[r].z;
-        sV[(kk + 3) * D + dv] = nv[r].w;
-      } else {
-        *reinterpret_cast<float4*>(sV + e) = nv[r];
-      }
-    }
-  };
-
-  int64_t kv0 = static_cast<int64_t>(w) * kF32Keys;
-  if (kv0 < L) {
-    load_block(kv0);
-    store_block();
-  }
-  for (; kv0 < L; kv0 += kF32Waves * kF32Keys) {
-    // KMASK: bit i of `attended` = key kv0 + i below L and attended (lane i reads its byte; lanes 16-63 repeat
-    // lanes 0-15); wave-uniform.
-    uint32_t attended = 0xffffu;
-    if constexpr (KMASK) {
-      const int left = static_cast<int>(L - kv0);  // keys of the window from kv0 on (>= 1; L < 2^31)
-      const int kk = min(lane & (kF32Keys - 1), left - 1);
-      attended = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(mrow[kv0 + kk] != 0)) & 0xffffu;
-      if (left < kF32Keys) attended &= (1u << left) - 1u;
-    }
-    const int64_t next = kv0 + kF32Waves * kF32Keys;
-    load_block(next);  // in flight while this block is computed (zeros past the window)
-    float t[kF32Keys];
-    float mb = -INFINITY;
-#pragma unroll
-    for (int i = 0; i < kF32Keys; ++i) {
-      const float* kr = sK + i * D;
-      float acc = 0.f;
-#pragma unroll
-      for (int d = 0; d < D; d += 4) {
-        const float4 x = *reinterpret_cast<const float4*>(kr + d);
-        acc = __builtin_fmaf(qv[d], x.x, acc);
-        acc = __builtin_fmaf(qv[d + 1], x.y, acc);
-        acc = __builtin_fmaf(qv[d + 2], x.z, acc);
-        acc = __builtin_fmaf(qv[d + 3], x.w, acc);
-      }
-      // Branch-free: keys >= L (zero rows, acc = 0) take the bias -inf. A select on acc would let the compiler put
-      // each row's products under a branch and hoist every row's LDS reads above all of them.
-      const float bias = (KMASK ? ((attended >> i) & 1u) != 0u : kv0 + i < L) ? 0.f : -INFINITY;
-      t[i] = __builtin_fmaf(acc, sl2, bias);
-      mb = fmaxf(mb, t[i]);
-    }
-    const float mn = fmaxf(m, mb);  // finite without a key mask: the block holds at least one key
-    // With a key mask mn is -inf while no attended key has come: the exponentials are then taken against 0, which
-    // gives 0 for every weight and for alpha (O and l hold nothing yet).
-    const float mref = (KMASK && mn == -INFINITY) ? 0.f : mn;
-    const float alpha = __builtin_amdgcn_exp2f(m - mref);  // 0 on the wave's first block
-    m = mn;
-    l *= alpha;
-#pragma unroll
-    for (int d = 0; d < D; ++d) o[d] *= alpha;
-#pragma unroll
-    for (int i = 0; i < kF32Keys; ++i) {
-      const float pw = __builtin_amdgcn_exp2f(t[i] - mref);  // 0 for keys >= L and keys not attended
-      l += pw;
-      const float* vr = sV + i * D;
-#pragma unroll
-      for (int d = 0; d < D; d += 4) {
-        const float4 x = *reinterpret_cast<const float4*>(vr + d);
-        o[d] = __builtin_fmaf(pw, x.x, o[d]);
-        o[d + 1] = __builtin_fmaf(pw, x.y, o[d + 1]);
-        o[d + 2] = __builtin_fmaf(pw, x.z, o[d + 2]);
-        o[d + 3] = __builtin_fmaf(pw, x.w, o[d + 3]);
-      }
-    }
-    store_block();
-  }
-
-  // Merge: round r, waves [n/2, n) hand their (O, m, l) to waves [0, n/2) (n = 8, 4, 2).
-  float* part = s_buf;
-  for (int n = kF32Waves; n > 1; n >>= 1) {
-    const int half = n >> 1;
-    __syncthreads();
-    if (w >= half && w < n) {
-      float* dst = part + (w - half) * (kF32MaxD + 2) * 64 + lane;
-#pragma unroll
-      for (int d = 0; d < D; ++d) dst[d * 64] = o[d];
-      dst[D * 64] = m;
-      dst[(D + 1) * 64] = l;
+    };
+    int on = 0;
+    if (blk0 < blk1) {
+      load_block(blk0 * kKB);
+      on = load_mask(blk0 * kKB);
+      store_block();
     }
     __syncthreads();
-    if (w < half) {
-      const float* src = part + w * (kF32MaxD + 2) * 64 + lane;
-      const float m2 = src[D * 64], l2 = src[(D + 1) * 64];
-      const float mm = fmaxf(m, m2);
-      // A wave that saw no key keeps m = -inf, l = 0 and O = 0: its factor is exp2(-inf) = 0; with both at -inf
-      // (no key at all) both factors are 0.
-      const float a1 = mm == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mm);
-      const float a2 = mm == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m2 - mm);
+    for (int blk = blk0; blk < blk1; ++blk) {
+      const uint64_t bits = __builtin_amdgcn_ballot_w64(on != 0);
+      const bool more = blk + 1 < blk1;
+      if (more) {
+        load_block((blk + 1) * kKB);
+        on = load_mask((blk + 1) * kKB);
+      }
+      if (!KMASK || bits != 0ull) {
 #pragma unroll
-      for (int d = 0; d < D; ++d) o[d] = o[d] * a1 + src[d * 64] * a2;
-      l = l * a1 + l2 * a2;
-      m = mm;
+        for (int t = 0; t < 2; ++t) {
+          f32x16_t s;
+          const float* kr = sK + (32 * t + col) * kF32Row;
+#pragma unroll
+          for (int c = 0; c < D / 8; ++c) {
+            const float4 x = *reinterpret_cast<const float4*>(kr + 4 * f32_swz_k(col, 2 * c + hh));
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, qf[4 * c], c == 0 ? f32x16_t{0} : s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, qf[4 * c + 1], s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, qf[4 * c + 2], s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, qf[4 * c + 3], s, 0, 0, 0);
+          }
+          if (bits != ~0ull) {
+            const uint32_t mine = static_cast<uint32_t>(bits >> (32 * t)) >> (4 * hh);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              if (!((mine >> (8 * (i / 4) + i % 4)) & 1u)) s[i] = -INFINITY;
+            }
+          }
+          float mb = s[0];
+#pragma unroll
+          for (int i = 1; i < 16; ++i) mb = fmaxf(mb, s[i]);
+          mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
+          const float mn = fmaxf(m, mb * sl2);
+          if (__builtin_amdgcn_ballot_w64(mn > m) != 0ull) {
+            // alpha is 0 on a query's first attended keys (m = -inf), with O and l still 0.
+            const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+            m = mn;
+            l *= alpha;
+#pragma unroll
+            for (int j = 0; j < kTiles; ++j) {
+#pragma unroll
+              for (int i = 0; i < 16; ++i) o[j][i] *= alpha;
+            }
+          }
+          const float nm = m == -INFINITY ? 0.f : -m;
+          float sum = 0.f;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], sl2, nm));
+            sum += s[i];
+          }
+          l += sum;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int key = 32 * t + 8 * (i / 4) + 4 * hh + i % 4;
+            // f32_swz_v on floats: bit 5 of the row's float index flips with bit 2 of the key, which is hh.
+            const float* vr = sV + key * kF32Row;
+#pragma unroll
+            for (int j = 0; j < kTiles; ++j) {
+              o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[(32 * j + col) ^ (32 * hh)], s[i], o[j], 0, 0, 0);
+            }
+          }
+        }
+      }
+      __syncthreads();
+      if (more) {
+        store_block();
+        __syncthreads();
+      }
     }
-  }
-  if (w == 0 && q_ok) {
-    // No key at all (L = 0, or no attended key): zeros, as the bf16 kernel writes.
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    float* out = p.o + b * p.so_b + h * p.so_h + q * p.so_q;
+    l += __shfl_xor(l, 32, 64);
+
+    if constexpr (SPLIT) {
+      if (blk1 - blk0 < unit_blocks) {
+        float* slot = p.part + (static_cast<int64_t>(2 * team + (blk0 == 0 ? 1 : 0)) * p.q_tiles + qt) *
+                                   split_slot_floats(D);
+        const int ql = w * 32 + col;
 #pragma unroll
-    for (int d = 0; d < D; ++d) out[d] = o[d] * inv;
-  }
+        for (int j = 0; j < kTiles; ++j) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const int d0 = 32 * j + 8 * g + 4 * hh;
+            if (d0 < D) {
+              split_store(slot, d0, ql, o[j][4 * g], o[j][4 * g + 1], o[j][4 * g + 2], o[j][4 * g + 3]);
+            }
+          }
+        }
+        if (hh == 0) {
+          slot[kQTile * D + ql] = l == 0.f ? -INFINITY : m;
+          slot[kQTile * (D + 1) + ql] = l;
+        }
+        continue;
+      }
+    }
+    if (q_ok) {
+      // No key at all (L = 0, or no attended key): zeros, as the bf16 kernel writes.
+      const float inv = l == 0.f ? 0.f : 1.f / l;
+      float* out = p.o + b * p.so_b + h * p.so_h + q * p.so_q;
+#pragma unroll
+      for (int j = 0; j < kTiles; ++j) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int d = 32 * j + 8 * (i / 4) + 4 * hh + i % 4;
+          if (d < D) out[d] = o[j][i] * inv;
+        }
+      }
+    }
+  } while (SPLIT && pos < range_end);
 }
 
-template <int D, bool KMASK>
-static void launch_f32(const XattnF32Params& p, unsigned grid, hipStream_t s, bool vt) {
-  if (vt) {
-    xattn_f32_kernel<D, true, KMASK><<<grid, kF32Threads, 0, s>>>(p);
+template <int D, bool VT, bool KMASK>
+static void launch_f32(const XattnF32Params& p, unsigned grid, hipStream_t s) {
+  if (p.teams) {
+    xattn_f32_kernel<D, VT, KMASK, true><<<static_cast<unsigned>(p.teams) * p.q_tiles, kThreads, 0, s>>>(p);
+    split_join_kernel<float><<<dim3(grid, static_cast<unsigned>(cdiv(D, kJoinDims))), kThreads, 0, s>>>(p);
   } else {
-    xattn_f32_kernel<D, false, KMASK><<<grid, kF32Threads, 0, s>>>(p);
+    xattn_f32_kernel<D, VT, KMASK, false><<<grid, kThreads, 0, s>>>(p);
   }
 }
 
 template <int D>
 static void launch_f32(const XattnF32Params& p, unsigned grid, hipStream_t s, bool vt) {
   if (p.kv_mask) {
-    launch_f32<D, true>(p, grid, s, vt);
+    vt ? launch_f32<D, true, true>(p, grid, s) : launch_f32<D, false, true>(p, grid, s);
   } else {
-    launch_f32<D, false>(p, grid, s, vt);
+    vt ? launch_f32<D, true, false>(p, grid, s) : launch_f32<D, false, false>(p, grid, s);
   }
 }
 
@@ -269,8 +346,8 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
                           int64_t sm_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B, int64_t H,
                           int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q,
                           int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k,
-                          int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* stream,
-                          const char* name) {
+                          int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* workspace,
+                          size_t workspace_bytes, void* stream, const char* name) {
   clear_error();
   SVHIP_REQUIRE(q && k && v && o, "%s: null pointer", name);
   if (kv_mask) {
@@ -302,10 +379,12 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   p.kv_len = kv_len;
   p.cu_seqlens = cu_seqlens;
   p.kv_mask = kv_mask;
+  p.v_scale = nullptr;
   p.sm_b = sm_b;
   p.B = B;
   p.H = H;
   p.Q = Q;
+  p.D = D;
   p.kv_cap = kv_cap;
   p.sq_b = sq_b;
   p.sq_h = sq_h;
@@ -321,9 +400,21 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   p.so_h = so_h;
   p.so_q = so_q;
   p.scale_log2 = scale * kLog2e;
-  p.q_tiles = static_cast<int>(cdiv(Q, 64));
+  p.q_tiles = static_cast<int>(cdiv(Q, kQTile));
   const int64_t grid = static_cast<int64_t>(p.q_tiles) * H * B;
   SVHIP_REQUIRE(grid < (1ll << 31), "%s: grid too large", name);
+  p.part = nullptr;
+  p.teams = 0;
+  if (workspace) {
+    const int teams = split_teams(B, H, Q, kv_cap, kF32Resident);
+    const size_t need = split_workspace_bytes(B, H, Q, D, kv_cap, kF32Resident);
+    if (teams) {
+      SVHIP_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= need,
+                    "%s: workspace too small or unaligned (%zu < %zu bytes)", name, workspace_bytes, need);
+      p.part = static_cast<float*>(workspace);
+      p.teams = teams;
+    }
+  }
   hipStream_t s = as_stream(stream);
   const unsigned g = static_cast<unsigned>(grid);
   switch (D) {
@@ -344,13 +435,31 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   return SVHIP_OK;
 }
 
+extern "C" size_t svhip_xattn_f32_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap) {
+  if (H < 1 || D < 1 || kv_cap < 0) return 0;
+  return split_workspace_bytes(B, H, Q, D, kv_cap, kF32Resident);
+}
+
+extern "C" int svhip_xattn_fwd_f32_ws(const float* q, const float* k, const float* v, float* o, const uint8_t* kv_mask,
+                                      int64_t sm_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B,
+                                      int64_t H, int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h,
+                                      int64_t sq_q, int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b,
+                                      int64_t sv_h, int64_t sv_k, int64_t sv_d, int64_t so_b, int64_t so_h,
+                                      int64_t so_q, float scale, void* workspace, size_t workspace_bytes,
+                                      void* stream) {
+  return xattn_f32_impl(q, k, v, o, kv_mask, sm_b, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b, sk_h,
+                        sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, workspace, workspace_bytes, stream,
+                        "svhip_xattn_fwd_f32_ws");
+}
+
 extern "C" int svhip_xattn_fwd_f32(const float* q, const float* k, const float* v, float* o, const int32_t* kv_len,
                                    const int32_t* cu_seqlens, int64_t B, int64_t H, int64_t Q, int64_t D,
                                    int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q, int64_t sk_b,
                                    int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k, int64_t sv_d,
                                    int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* stream) {
   return xattn_f32_impl(q, k, v, o, nullptr, 0, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b, sk_h,
-                        sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, stream, "svhip_xattn_fwd_f32");
+                        sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0, stream,
+                        "svhip_xattn_fwd_f32");
 }
 
 extern "C" int svhip_xattn_fwd_f32_masked(const float* q, const float* k, const float* v, float* o,
@@ -364,5 +473,6 @@ extern "C" int svhip_xattn_fwd_f32_masked(const float* q, const float* k, const 
   clear_error();
   SVHIP_REQUIRE(kv_mask, "%s: null key mask", name);
   return xattn_f32_impl(q, k, v, o, kv_mask, sm_b, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b,
-                        sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, stream, name);
+                        sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0, stream,
+                        name);
 }

@@ -171,20 +171,17 @@ def _attention_f32(query, key, val, lengths, cu_seqlens, scale, out, key_mask=No
         raise ValueError('head_dim mismatch')
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
     lib = _lib.load()
-    if key_mask is not None:
-        if cu_seqlens is None and key_mask.shape[1] < kcap:
-            raise ValueError(f'key_mask holds {key_mask.shape[1]} keys per window, the cache {kcap}')
-        mask_cap = kcap if cu_seqlens is None else key_mask.shape[1]
-        _lib.check(lib.svhip_xattn_fwd_f32_masked(
-            _lib.ptr(query), _lib.ptr(key), _lib.ptr(val), _lib.ptr(out), _lib.ptr(key_mask.view(torch.uint8)),
-            key_mask.stride(0), _lib.ptr(lengths), _lib.ptr(cu_seqlens), B, H, Q, D, mask_cap,
-            query.stride(0), query.stride(1), query.stride(2), *sk, *sv, out.stride(0), out.stride(1), out.stride(2),
-            scale, _lib.stream_of(query)), 'svhip_xattn_fwd_f32_masked')
-        return out
-    _lib.check(lib.svhip_xattn_fwd_f32(
-        _lib.ptr(query), _lib.ptr(key), _lib.ptr(val), _lib.ptr(out), _lib.ptr(lengths), _lib.ptr(cu_seqlens),
-        B, H, Q, D, kcap, query.stride(0), query.stride(1), query.stride(2), *sk, *sv,
-        out.stride(0), out.stride(1), out.stride(2), scale, _lib.stream_of(query)), 'svhip_xattn_fwd_f32')
+    if key_mask is not None and cu_seqlens is None and key_mask.shape[1] < kcap:
+        raise ValueError(f'key_mask holds {key_mask.shape[1]} keys per window, the cache {kcap}')
+    mask_cap = kcap if key_mask is None or cu_seqlens is None else key_mask.shape[1]
+    nbytes = int(lib.svhip_xattn_f32_workspace_bytes(B, H, Q, D, mask_cap))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device) if nbytes else None
+    mask = None if key_mask is None else key_mask.view(torch.uint8)
+    _lib.check(lib.svhip_xattn_fwd_f32_ws(
+        _lib.ptr(query), _lib.ptr(key), _lib.ptr(val), _lib.ptr(out), _lib.ptr(mask),
+        0 if mask is None else mask.stride(0), _lib.ptr(lengths), _lib.ptr(cu_seqlens), B, H, Q, D, mask_cap,
+        query.stride(0), query.stride(1), query.stride(2), *sk, *sv, out.stride(0), out.stride(1), out.stride(2),
+        scale, _lib.ptr(ws), nbytes, _lib.stream_of(query)), 'svhip_xattn_fwd_f32_ws')
     return out
 
 

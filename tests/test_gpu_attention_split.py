@@ -2,7 +2,7 @@
 
 Window lengths where the split can go wrong: ranges that end on a unit's first and last block, one block past the
 length from which windows are split, empty windows between long ones, a single window cut into many parts, parts that
-a key mask empties. The bars are the unsplit kernels' (bf16 2e-2 and 1e-2 of the largest value: the
+a key mask empties. The bars are the unsplit kernels' (bf16 2e-2 and 1e-2 of the largest value, fp32 2e-5 and 1e-4: the
 parts are kept and joined in fp32, so the split adds no rounding of its own to them)."""
 import math
 
@@ -119,6 +119,25 @@ def test_split_e4m3_against_unsplit(dev):
         torch.cuda.synchronize()
         check(out, one.double().cpu(), 2e-2, 1e-2)
         assert not out[1].any()
+
+
+@pytest.mark.parametrize('lengths', LENGTHS, ids=lambda x: '-'.join(map(str, x)))
+@pytest.mark.parametrize('D', [16, 32, 48, 64])
+def test_split_fp32_windows_match_the_oracle(dev, lengths, D):
+    from streamvoxel_amd.stream.attention import attention
+    B, H, Q, kcap = len(lengths), 2, 130, max(lengths) + 4
+    kcap += -kcap % 4
+    _case(f'split fp32 D={D} lengths={lengths}')
+    q, k, v = qkv(B, H, Q, kcap, D, sum(lengths) + D, torch.float32)
+    ref = A.cross_attention(q, k, v, lengths)
+    lt = torch.tensor(lengths, dtype=torch.int32, device=dev)
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    out = attention(qd, kd, vd, lengths=lt)
+    out_t = attention(qd, kd, vd.transpose(2, 3).contiguous().transpose(2, 3), lengths=lt)
+    out_m = attention(qd, kd, vd, key_mask=torch.arange(kcap, device=dev)[None] < lt[:, None])
+    torch.cuda.synchronize()
+    for x in (out, out_t, out_m):
+        check(x, ref, 2e-5, 1e-4)
 
 
 def test_split_replays_in_a_graph(dev):
