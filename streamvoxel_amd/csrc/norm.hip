@@ -68,6 +68,9 @@ struct NormArgs {
 
 // LPR lanes per row, CH 16-byte chunks per lane (chunk lane + LPR c). RES: a residual branch is added (gated when
 // gate is set). VEC: gate / shift / scale rows take 16-byte loads.
+// A launch is one short chain per row (load, two reductions, store) with four waves a SIMD and nothing behind it, so
+// its loads go out together at the start (AHEAD): branch, gate, shift and scale read after one another, each behind the
+// step before, took 10.2 us for 8 x 1024 rows of 768 with branch, gate and modulation, 9.0 us now (5.6 TB/s). Rows of more than four chunks a lane would not have the registers.
 template <int LPR, int CH, bool RES, bool VEC>
 __global__ __launch_bounds__(kNormThreads) void layer_norm_kernel(NormArgs a) {
   constexpr int kRowsPerBlock = kNormThreads / LPR;
@@ -80,6 +83,22 @@ __global__ __launch_bounds__(kNormThreads) void layer_norm_kernel(NormArgs a) {
   const int64_t b = row / a.N, n = row - b * a.N;
   const uint16_t* xr = a.x + b * a.sxb + n * a.sxn;
   const int chunks = static_cast<int>(a.W / 8);
+  constexpr bool AHEAD = VEC && CH <= 4;
+  [[maybe_unused]] uint4 aw[CH], gw[CH], hw[CH], sw[CH];
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int e = 8 * min(lane + LPR * c, chunks - 1);
+      if constexpr (RES) {
+        aw[c] = *reinterpret_cast<const uint4*>(a.a + b * a.sab + n * a.san + e);
+        if (a.gate) gw[c] = *reinterpret_cast<const uint4*>(a.gate + b * a.s_gate + e);
+      }
+      if (a.scale) {
+        sw[c] = *reinterpret_cast<const uint4*>(a.scale + b * a.s_mod + e);
+        hw[c] = *reinterpret_cast<const uint4*>(a.shift + b * a.s_mod + e);
+      }
+    }
+  }
   float v[CH][8];
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
@@ -97,10 +116,18 @@ __global__ __launch_bounds__(kNormThreads) void layer_norm_kernel(NormArgs a) {
       const int ch = lane + LPR * c;
       if (ch >= chunks) continue;
       float br[8];
-      unpack8(*reinterpret_cast<const uint4*>(ar + 8 * ch), br);
+      if constexpr (AHEAD) {
+        unpack8(aw[c], br);
+      } else {
+        unpack8(*reinterpret_cast<const uint4*>(ar + 8 * ch), br);
+      }
       if (gr) {
         float g[8];
-        load_row8<VEC>(gr + 8 * ch, g);
+        if constexpr (AHEAD) {
+          unpack8(gw[c], g);
+        } else {
+          load_row8<VEC>(gr + 8 * ch, g);
+        }
 #pragma unroll
         for (int j = 0; j < 8; j += 2) {
           br[j] *= g[j];
@@ -156,8 +183,13 @@ __global__ __launch_bounds__(kNormThreads) void layer_norm_kernel(NormArgs a) {
     }
     if (sc) {
       float s8[8], h8[8];
-      load_row8<VEC>(sc + 8 * ch, s8);
-      load_row8<VEC>(sh + 8 * ch, h8);
+      if constexpr (AHEAD) {
+        unpack8(sw[c], s8);
+        unpack8(hw[c], h8);
+      } else {
+        load_row8<VEC>(sc + 8 * ch, s8);
+        load_row8<VEC>(sh + 8 * ch, h8);
+      }
 #pragma unroll
       for (int j = 0; j < 8; j += 2) {
         float o0 = 1.0f + s8[j], o1 = 1.0f + s8[j + 1];
