@@ -311,6 +311,8 @@ int svhip_kv_write(const void* prefix_k, const void* prefix_v, int64_t P, int64_
                    void* cache_v, int64_t scv_h, int64_t scv_k, int64_t scv_d, int64_t kv_cap, int kv_dtype,
                    float* k_scale, float* v_scale, void* workspace, size_t workspace_bytes, void* stream);
 
+/* svhip_kv_write that also sets *length (device) to P + L, the window's entry of kv_len;
+
 /*
  * Self-attention operands of a transformer block from its fused qkv projection: qkv bf16, element (b,n,s,h,d)
  * (s = 0 Q, 1 K, 2 V; the Linear's [3, H, D] row) at b*sx_b + n*sx_n + (s*H + h)*D + d, rows 16-byte aligned.

@@ -67,6 +67,10 @@ SIGNATURES = {
                                       _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_p, _c_i64,
                                       _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_int, _c_p, _c_p, _c_p,
                                       _c_sz, _c_p]),
+    'svhip_kv_write_length': (ctypes.c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_i64,
+                                             _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_p,
+                                             _c_i64, _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_int, _c_p,
+                                             _c_p, _c_p, _c_sz, _c_p, _c_p]),
     'svhip_qkv_rope': (ctypes.c_int, [_c_p, _c_p, _c_p] + [_c_i64] * 8 + [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_i64,
                                                                        _c_i64, _c_i64, _c_p, _c_i64, _c_i64, _c_i64,
                                                                        _c_p]),

@@ -162,6 +162,7 @@ struct KvArgs {
   float* partial;            // [H, tiles, 2] (e4m3)
   int64_t tiles;
   int group;                 // heads of a workgroup (kv_vec_kernel)
+  int32_t* length;           // set to P + L, or null
 };
 
 // K and V pair `pr` of key j of head h (zeros past the window's keys; local K rotated when positions are given).
@@ -225,6 +226,7 @@ __global__ __launch_bounds__(kProducerThreads) void kv_write_kernel(KvArgs a) {
   __shared__ __attribute__((aligned(16))) uint8_t sv[kMaxHeadDim * kTileKeys * (FP8 ? 1 : 2)];
   const int64_t h = blockIdx.y, tile = blockIdx.x;
   const int64_t pairs = a.D / 2;
+  if (a.length && h == 0 && tile == 0 && threadIdx.x == 0) *a.length = static_cast<int32_t>(a.P + a.L);
   float sk = 1.f, svs = 1.f;  // e4m3 scales of K and V
   if constexpr (FP8) {
     float mk = 0.f, mv = 0.f;
@@ -295,9 +297,10 @@ __global__ __launch_bounds__(kProducerThreads) void kv_write_kernel(KvArgs a) {
 // copies when every head forms its own. Workgroup = (64-key tile, kVecHeads heads): the tile's sin / cos (rounded to
 // bf16, packed) go to LDS once, and a thread moves 16-byte chunks of K and V, all of its first batch of loads in
 // flight before the table is formed; V^T goes through LDS and leaves in 16-byte runs of keys. One window of 8 x 48
-// heads, 4096 prefix and 8480 local keys: 19.5 us with the pair kernel above (2.0 TB/s), 14.3 us here (2.7 TB/s).
-constexpr int kVecThreads = 512;
-constexpr int kVecHeads = 4;  // at most (fewer where the tile of V^T would pass 64 KB of LDS)
+// heads, 4096 prefix and 8480 local keys: 19.5 us with the pair kernel above (2.0 TB/s), 14.0 us here (2.8 TB/s; groups
+// of four heads and 512 threads 13.9 us, the length by a launch of its own 2.3 us more).
+constexpr int kVecThreads = 256;
+constexpr int kVecHeads = 2;  // at most (fewer where the tile of V^T would pass 64 KB of LDS)
 constexpr int kVecBatch = 3;  // chunks of K (and of V) a thread has in flight
 
 // 8 fp32 values divided by `scale` and rounded to e4m3 (two dwords).
@@ -332,6 +335,9 @@ __global__ __launch_bounds__(kVecThreads) void kv_vec_kernel(KvArgs a) {
   E* sv = reinterpret_cast<E*>(smem + sizeof(uint32_t) * kTileKeys * pairs);      // [head][d][key]
   const int per_head = kTileKeys * chunks;
   const int total = heads * per_head;
+  if (!STATS && a.length && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    *a.length = static_cast<int32_t>(a.P + a.L);
+  }
 
   uint4 kw[kVecBatch], vw[kVecBatch];
   auto load_batch = [&](int base) __attribute__((always_inline)) {
@@ -665,6 +671,18 @@ extern "C" int svhip_kv_write(const void* prefix_k, const void* prefix_v, int64_
                               int64_t sck_k, void* cache_v, int64_t scv_h, int64_t scv_k, int64_t scv_d,
                               int64_t kv_cap, int kv_dtype, float* k_scale, float* v_scale, void* workspace,
                               size_t workspace_bytes, void* stream) {
+  return svhip_kv_write_length(prefix_k, prefix_v, P, spk_h, spk_l, spv_h, spv_l, local_k, local_v, L, slk_h, slk_l,
+                               slv_h, slv_l, positions, sp_l, freq, H, D, cache_k, sck_h, sck_k, cache_v, scv_h, scv_k,
+                               scv_d, kv_cap, kv_dtype, k_scale, v_scale, workspace, workspace_bytes, nullptr, stream);
+}
+
+extern "C" int svhip_kv_write_length(const void* prefix_k, const void* prefix_v, int64_t P, int64_t spk_h, int64_t spk_l,
+                              int64_t spv_h, int64_t spv_l, const void* local_k, const void* local_v, int64_t L,
+                              int64_t slk_h, int64_t slk_l, int64_t slv_h, int64_t slv_l, const float* positions,
+                              int64_t sp_l, const float* freq, int64_t H, int64_t D, void* cache_k, int64_t sck_h,
+                              int64_t sck_k, void* cache_v, int64_t scv_h, int64_t scv_k, int64_t scv_d,
+                              int64_t kv_cap, int kv_dtype, float* k_scale, float* v_scale, void* workspace,
+                              size_t workspace_bytes, int32_t* length, void* stream) {
   const char* name = "svhip_kv_write";
   clear_error();
   SVHIP_REQUIRE(cache_k && cache_v, "%s: null cache pointer", name);
@@ -701,7 +719,7 @@ extern "C" int svhip_kv_write(const void* prefix_k, const void* prefix_v, int64_
   KvArgs a{static_cast<const uint16_t*>(prefix_k), static_cast<const uint16_t*>(prefix_v), P, spk_h, spk_l, spv_h,
            spv_l, static_cast<const uint16_t*>(local_k), static_cast<const uint16_t*>(local_v), L, slk_h, slk_l,
            slv_h, slv_l, positions, sp_l, freq, H, D, kv_cap, cache_k, sck_h, sck_k, cache_v, scv_h, scv_k, scv_d,
-           k_scale, v_scale, static_cast<float*>(workspace), tiles, 1};
+           k_scale, v_scale, static_cast<float*>(workspace), tiles, 1, length};
   SVHIP_REQUIRE(tiles < 65536 && H < 65536, "%s: grid too large", name);
   const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(H));
   hipStream_t s = as_stream(stream);

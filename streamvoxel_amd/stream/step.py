@@ -96,15 +96,18 @@ class CachedContext:
             ws = self._kv_ws
         ks = self.k_scale[layer][index] if fp8 else None
         vs = self.v_scale[layer][index] if fp8 else None
-        _lib.check(lib.svhip_kv_write(
+        # The window's length goes with the kernel: with the last layer, or when it changes.
+        new_length = layer == self.layers - 1 or self.host_lengths[index] != P + L
+        length = self.lengths[index] if new_length and self.kv_cap else None
+        _lib.check(lib.svhip_kv_write_length(
             _lib.ptr(pk), _lib.ptr(pv), P, pk.stride(0) if P else 0, pk.stride(1) if P else 0,
             pv.stride(0) if P else 0, pv.stride(1) if P else 0, _lib.ptr(key), _lib.ptr(value), L, key.stride(0),
             key.stride(1), value.stride(0), value.stride(1), _lib.ptr(pos), 3, _lib.ptr(freq), H, D, _lib.ptr(kc),
             kc.stride(0), kc.stride(1), _lib.ptr(vc), vc.stride(0), vc.stride(2), vc.stride(1), self.kv_cap, code,
-            _lib.ptr(ks), _lib.ptr(vs), _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream_of(key)),
-            'svhip_kv_write')
-        if layer == self.layers - 1 or self.host_lengths[index] != P + L:
-            self.set_length(index, P + L)
+            _lib.ptr(ks), _lib.ptr(vs), _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.ptr(length),
+            _lib.stream_of(key)), 'svhip_kv_write_length')
+        if new_length:
+            self.host_lengths[index] = P + L
 
     def set_length(self, index, length):
         self.host_lengths[index] = int(length)
