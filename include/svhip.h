@@ -214,11 +214,13 @@ int svhip_xattn_fwd_masked(const void* q, const void* k, const void* v, void* o,
                            int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* stream);
 
 /*
- * svhip_xattn_fwd_masked with the scratch memory of svhip_xattn_fwd_ws (used where kv_len is given). kv_len may come
- * with cu_seqlens here: a window then ends at the smaller of the two lengths.
+ * svhip_xattn_fwd_masked with the scratch memory of svhip_xattn_fwd_ws, used where kv_len and kv_blocks are the results
+ * of svhip_mask_blocks (rows of kv_blocks sb_b apart): blocks without an attended key are then not read either. kv_len
+ * may come with cu_seqlens here: a window then ends at the smaller of the two lengths.
  */
 int svhip_xattn_fwd_masked_ws(const void* q, const void* k, const void* v, void* o, const uint8_t* kv_mask,
-                              int64_t sm_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B, int64_t H,
+                              int64_t sm_b, const int32_t* kv_len, const int32_t* kv_blocks, int64_t sb_b,
+                              const int32_t* cu_seqlens, int64_t B, int64_t H,
                               int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q,
                               int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k,
                               int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* workspace,
@@ -234,6 +236,13 @@ int svhip_xattn_fwd_masked_ws(const void* q, const void* k, const void* v, void*
  */
 int svhip_mask_lengths(const uint8_t* kv_mask, int64_t sm_b, const int32_t* kv_len, int64_t B, int64_t kv_cap,
                        int32_t* out, void* stream);
+
+/*
+ * svhip_mask_lengths (into `lengths`), and for every window the 64-key blocks that hold an attended key: row b of
+ * `blocks` (int32, rows sb_b > ceil(kv_cap / 64) apart, device) gets their count, then their indices in order.
+ */
+int svhip_mask_blocks(const uint8_t* kv_mask, int64_t sm_b, const int32_t* kv_len, int64_t B, int64_t kv_cap,
+                      int32_t* lengths, int32_t* blocks, int64_t sb_b, void* stream);
 
 /*
  * Cross attention in fp32 arithmetic: fp32 q/k/v/o with the layouts and strides of svhip_xattn_fwd (elements, not
@@ -267,11 +276,12 @@ int svhip_xattn_fwd_f32_masked(const float* q, const float* k, const float* v, f
 
 /*
  * The two fp32 forms (kv_mask may be NULL) with scratch memory for the key split, as svhip_xattn_fwd_ws has it: at
- * least svhip_xattn_f32_workspace_bytes bytes, 16-byte aligned. The parts are kept and joined in fp32.
+ * least svhip_xattn_f32_workspace_bytes bytes, 16-byte aligned; with a key mask as svhip_xattn_fwd_masked_ws. The parts are kept and joined in fp32.
  */
 size_t svhip_xattn_f32_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap);
 int svhip_xattn_fwd_f32_ws(const float* q, const float* k, const float* v, float* o, const uint8_t* kv_mask,
-                           int64_t sm_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B, int64_t H,
+                           int64_t sm_b, const int32_t* kv_len, const int32_t* kv_blocks, int64_t sb_b,
+                           const int32_t* cu_seqlens, int64_t B, int64_t H,
                            int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q,
                            int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k,
                            int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* workspace,
@@ -311,7 +321,13 @@ int svhip_kv_write(const void* prefix_k, const void* prefix_v, int64_t P, int64_
                    void* cache_v, int64_t scv_h, int64_t scv_k, int64_t scv_d, int64_t kv_cap, int kv_dtype,
                    float* k_scale, float* v_scale, void* workspace, size_t workspace_bytes, void* stream);
 
-/* svhip_kv_write that also sets *length (device) to P + L, the window's entry of kv_len;
+/* svhip_kv_write that also sets *length (device) to P + L, the window's entry of kv_len; NULL: as svhip_kv_write. */
+int svhip_kv_write_length(const void* prefix_k, const void* prefix_v, int64_t P, int64_t spk_h, int64_t spk_l,
+                   int64_t spv_h, int64_t spv_l, const void* local_k, const void* local_v, int64_t L, int64_t slk_h,
+                   int64_t slk_l, int64_t slv_h, int64_t slv_l, const float* positions, int64_t sp_l,
+                   const float* freq, int64_t H, int64_t D, void* cache_k, int64_t sck_h, int64_t sck_k,
+                   void* cache_v, int64_t scv_h, int64_t scv_k, int64_t scv_d, int64_t kv_cap, int kv_dtype,
+                   float* k_scale, float* v_scale, void* workspace, size_t workspace_bytes, int32_t* length, void* stream);
 
 /*
  * Self-attention operands of a transformer block from its fused qkv projection: qkv bf16, element (b,n,s,h,d)

@@ -1,6 +1,8 @@
 // What the cross-attention kernels share: the tile of a workgroup, the window lengths and the key split.
 //
-// A kernel's parameters P carry B, H, Q, D, q_tiles, the window lengths (kv_len / cu_seqlens / kv_cap, kv_mask), the
+// A kernel's parameters P carry B, H, Q, D, q_tiles, the window lengths (kv_len / cu_seqlens / kv_cap, kv_mask), with a
+// key mask the windows' lists of blocks that hold an attended key (kv_blocks, rows sb_b apart: the count, then the
+// block indices in order, the window's last block the last; the split form with a key mask always has them), the
 // output (o, so_*), v_scale, and for the split form `part` (the slots of the parts, [team][2][query tile] of
 // split_slot_floats(D) floats) and `teams` (teams of q_tiles workgroups in the grid, a multiple of kXcds).
 #pragma once
@@ -60,7 +62,10 @@ template <typename P>
 __device__ __forceinline__ SplitPlan split_plan(const P& p) {
   SplitPlan s;
   const int lane = threadIdx.x & 63;
-  s.blocks = lane < p.B ? (window_length(p, lane) + kKB - 1) / kKB : 0;
+  s.blocks = 0;
+  if (lane < p.B) {
+    s.blocks = p.kv_blocks ? p.kv_blocks[lane * p.sb_b] : (window_length(p, lane) + kKB - 1) / kKB;
+  }
   int incl = s.blocks, longest = s.blocks;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -96,8 +101,18 @@ __device__ __forceinline__ int split_window(const P& p, const SplitPlan& s, int 
 
 // The workspace: the slots of the parts, then for every unit the first and last team that hold a part of it (last <
 // first where one range holds it whole), written by the workgroups that start the units.
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ void split_store(float* slot, int d0, int ql, float a, float b, float c, float d) {
   *reinterpret_cast<float4*>(slot + (static_cast<int64_t>(d0 >> 2) * kQTile + ql) * 4) = make_float4(a, b, c, d);
+}
+
+// Entry i of window b's list of blocks, through the scalar cache: a vector load would have to wait for the staged
+// loads in flight before it.
+template <typename P>
+__device__ __forceinline__ int listed_block(const P& p, int64_t b, int i) {
+  typedef const __attribute__((address_space(4))) int32_t* list_t;
+  return __builtin_amdgcn_readfirstlane(((list_t)(p.kv_blocks + b * p.sb_b + 1))[i]);
 }
 
 __host__ __device__ __forceinline__ int64_t split_slot_floats(int64_t D) { return kQTile * (D + 2); }
@@ -116,12 +131,19 @@ __device__ __forceinline__ int2 split_unit_teams(int team, int first, int unit_b
 
 // Joins the parts of the units that the split kernel cut: O = sum_i w_i O_i, l = sum_i w_i l_i with w_i =
 // exp2(m_i - max m) over the parts in key order, then v_scale O / l in the output's type. Workgroup = (unit, query
-// tile, kJoinDims head_dim elements); a thread holds 4 of them of kJoinItems queries. The parts are read once, from the
-// last-level cache where they were just written, the loads of kJoinAhead parts in flight (one part at a time, with the
-// plan formed here again, the join took 18-23 us of a layer; now 11-14). Windows without keys get their zeros here.
+// tile, kJoinQueries queries, kJoinDims head_dim elements), a thread 4 elements of one query. The parts are read once,
+// from the last-level cache where they were just written: a short chain of loads, so the workgroups are many and a
+// thread has kJoinAhead parts in flight (one window of 12 heads, nine parts a unit: 10.7 us with four queries a thread
+// and three parts in flight, 7.3 us here). Windows without keys get
+// their zeros here.
 constexpr int kJoinDims = 32;
-constexpr int kJoinItems = kQTile * (kJoinDims / 4) / kThreads;
-constexpr int kJoinAhead = 3;
+constexpr int kJoinQueries = kThreads / (kJoinDims / 4);
+constexpr int kJoinAhead = 6;
+
+inline dim3 split_join_grid(unsigned tiles, int64_t D) {
+  return dim3(tiles, static_cast<unsigned>(cdiv(D, kJoinDims)), kQTile / kJoinQueries);
+}
+
 template <typename T, typename P>
 __global__ __launch_bounds__(kThreads) void split_join_kernel(P p) {
   const int u = static_cast<int>(blockIdx.x / p.q_tiles), qt = static_cast<int>(blockIdx.x % p.q_tiles);
@@ -132,67 +154,43 @@ __global__ __launch_bounds__(kThreads) void split_join_kernel(P p) {
   const int t0 = empty ? 0 : teams.x, t1 = empty ? -1 : teams.y;
   if (!empty && t1 < t0) return;  // one range holds the unit: its output is written
   const int64_t slot_floats = split_slot_floats(p.D);
-  const int d0 = static_cast<int>(blockIdx.y) * kJoinDims + 4 * (threadIdx.x % (kJoinDims / 4));
-  if (d0 >= p.D) return;
-  const int ql0 = threadIdx.x / (kJoinDims / 4);
-  constexpr int kStep = kQTile / kJoinItems;  // queries between a thread's items
-  float m[kJoinItems], l[kJoinItems];
-  float4 o[kJoinItems];
-#pragma unroll
-  for (int i = 0; i < kJoinItems; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.f;
-    o[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
+  const int d0 = static_cast<int>(blockIdx.y) * kJoinDims + 4 * static_cast<int>(threadIdx.x % (kJoinDims / 4));
+  const int ql = static_cast<int>(blockIdx.z) * kJoinQueries + static_cast<int>(threadIdx.x / (kJoinDims / 4));
+  const int64_t q = static_cast<int64_t>(qt) * kQTile + ql;
+  if (d0 >= p.D || q >= p.Q) return;
+  float m = -INFINITY, l = 0.f;
+  f32x4_t o = {0.f, 0.f, 0.f, 0.f};
   for (int t = t0; t <= t1; t += kJoinAhead) {
-    float mi[kJoinAhead][kJoinItems], li[kJoinAhead][kJoinItems];
-    float4 oi[kJoinAhead][kJoinItems];
+    float mi[kJoinAhead], li[kJoinAhead];
+    f32x4_t oi[kJoinAhead];
 #pragma unroll
     for (int a = 0; a < kJoinAhead; ++a) {
+      if (t + a > t1) break;  // uniform
       // The first part is the one its team's range ends in (slot 1), the others begin their teams' ranges (slot 0).
-      const int ta = min(t + a, t1);
-      const float* slot = p.part + (static_cast<int64_t>(2 * ta + (ta == t0 ? 1 : 0)) * p.q_tiles + qt) * slot_floats;
-#pragma unroll
-      for (int i = 0; i < kJoinItems; ++i) {
-        const int ql = ql0 + i * kStep;
-        mi[a][i] = slot[kQTile * p.D + ql];
-        li[a][i] = slot[kQTile * (p.D + 1) + ql];
-        oi[a][i] = *reinterpret_cast<const float4*>(slot + (static_cast<int64_t>(d0 >> 2) * kQTile + ql) * 4);
-      }
+      const float* slot =
+          p.part + (static_cast<int64_t>(2 * (t + a) + (t + a == t0 ? 1 : 0)) * p.q_tiles + qt) * slot_floats;
+      mi[a] = slot[kQTile * p.D + ql];
+      li[a] = slot[kQTile * (p.D + 1) + ql];
+      oi[a] = *reinterpret_cast<const f32x4_t*>(slot + (static_cast<int64_t>(d0 >> 2) * kQTile + ql) * 4);
     }
 #pragma unroll
     for (int a = 0; a < kJoinAhead; ++a) {
-#pragma unroll
-      for (int i = 0; i < kJoinItems; ++i) {
-        if (t + a > t1 || li[a][i] == 0.f) continue;
-        const float mn = fmaxf(m[i], mi[a][i]);
-        const float x = __builtin_amdgcn_exp2f(m[i] - mn), y = __builtin_amdgcn_exp2f(mi[a][i] - mn);
-        m[i] = mn;
-        l[i] = l[i] * x + li[a][i] * y;
-        o[i].x = o[i].x * x + oi[a][i].x * y;
-        o[i].y = o[i].y * x + oi[a][i].y * y;
-        o[i].z = o[i].z * x + oi[a][i].z * y;
-        o[i].w = o[i].w * x + oi[a][i].w * y;
-      }
+      if (t + a > t1) break;
+      if (li[a] == 0.f) continue;  // a part without an attended key
+      const float mn = fmaxf(m, mi[a]);
+      const float x = __builtin_amdgcn_exp2f(m - mn), y = __builtin_amdgcn_exp2f(mi[a] - mn);
+      m = mn;
+      l = l * x + li[a] * y;
+      o = o * x + oi[a] * y;
     }
   }
-  T* Op = static_cast<T*>(p.o) + b * p.so_b + h * p.so_h;
-  const float vs = p.v_scale ? p.v_scale[b * p.H + h] : 1.f;
+  T* out = static_cast<T*>(p.o) + b * p.so_b + h * p.so_h + q * p.so_q + d0;
+  const float inv = l == 0.f ? 0.f : (p.v_scale ? p.v_scale[b * p.H + h] : 1.f) / l;
+  if constexpr (sizeof(T) == 4) {
 #pragma unroll
-  for (int i = 0; i < kJoinItems; ++i) {
-    const int64_t q = static_cast<int64_t>(qt) * kQTile + ql0 + i * kStep;
-    if (q >= p.Q) continue;
-    const float inv = l[i] == 0.f ? 0.f : vs / l[i];
-    if constexpr (sizeof(T) == 4) {
-      float* out = Op + q * p.so_q + d0;  // rows of any alignment
-      out[0] = o[i].x * inv;
-      out[1] = o[i].y * inv;
-      out[2] = o[i].z * inv;
-      out[3] = o[i].w * inv;
-    } else {
-      *reinterpret_cast<uint2*>(Op + q * p.so_q + d0) = make_uint2(bf16_pack2(o[i].x * inv, o[i].y * inv),
-                                                                   bf16_pack2(o[i].z * inv, o[i].w * inv));
-    }
+    for (int e = 0; e < 4; ++e) out[e] = o[e] * inv;  // rows of any alignment
+  } else {
+    *reinterpret_cast<uint2*>(out) = make_uint2(bf16_pack2(o[0] * inv, o[1] * inv), bf16_pack2(o[2] * inv, o[3] * inv));
   }
 }
 
@@ -200,10 +198,10 @@ __global__ __launch_bounds__(kThreads) void split_join_kernel(P p) {
 // windows beyond one wave's lanes, no window long enough to be split, or query tiles that fill the rounds of resident
 // workgroups by themselves. There the longest-first order balances uneven windows as well, without the parts' 50 MB
 // (8 windows x 12 heads x 1024 queries, 768 tiles = one full round of 3 per CU: 223-230 us unsplit, 232-240 split; of
-// it the kernel 224-230 against 241 and the join 17). One window of 12 heads (96 tiles) goes from 105 to 53 us, the 512
-// tiles of 8 windows x 8 heads x 48 from 180 to 158.
-// resident: workgroups of the split kernel that a CU holds.
-inline int split_teams(int64_t B, int64_t H, int64_t Q, int64_t kv_cap, int resident) {
+// it the kernel 224-230 against 241 and the join 17). One window of 12 heads (96 tiles) goes from 105 to 48 us, the 512
+// tiles of 8 windows x 8 heads x 48 from 180 to 153.
+// resident: workgroups of the split kernel that a CU holds; turns: ranges per resident team.
+inline int split_teams(int64_t B, int64_t H, int64_t Q, int64_t kv_cap, int resident, int turns = 1) {
   const int64_t q_tiles = cdiv(Q, kQTile);
   const int64_t per_xcd = kCusPerXcd * resident, slots = kXcds * per_xcd;
   if (B < 1 || B > kSplitMaxWindows || q_tiles < 1 || q_tiles > per_xcd / 4) return 0;
@@ -211,11 +209,12 @@ inline int split_teams(int64_t B, int64_t H, int64_t Q, int64_t kv_cap, int resi
   const int64_t tiles = B * H * q_tiles, rounds = cdiv(tiles, slots);
   if (rounds > kSplitMaxRounds || tiles * 100 >= rounds * slots * kSplitFullPercent) return 0;
   if (B * H * cdiv(kv_cap, kKB) >= (1ll << 31)) return 0;
-  return static_cast<int>(kXcds * (per_xcd / q_tiles));
+  return static_cast<int>(kXcds * (per_xcd / q_tiles) * turns);
 }
 
-inline size_t split_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap, int resident) {
-  const int64_t teams = split_teams(B, H, Q, kv_cap, resident);
+inline size_t split_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap, int resident,
+                                    int turns = 1) {
+  const int64_t teams = split_teams(B, H, Q, kv_cap, resident, turns);
   return teams ? static_cast<size_t>(2 * teams * cdiv(Q, kQTile) * split_slot_floats(D)) * sizeof(float) +
                      static_cast<size_t>(B * H) * sizeof(int2)
                : 0;

@@ -75,7 +75,7 @@ static int resident(int64_t D) { return D <= 64 ? 3 : 2; }
 
 static int xattn_impl(const void* q, const void* k, const void* v, void* o, int kv_dtype, const int32_t* kv_len,
                       const int32_t* cu_seqlens, const float* k_scale, const float* v_scale, const uint8_t* kv_mask,
-                      int64_t sm_b, int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b,
+                      int64_t sm_b, const int32_t* kv_blocks, int64_t sb_b, int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b,
                       int64_t sq_h, int64_t sq_q, int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b,
                       int64_t sv_h, int64_t sv_k, int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q,
                       float scale, void* workspace, size_t workspace_bytes, void* stream, const char* name) {
@@ -122,6 +122,8 @@ static int xattn_impl(const void* q, const void* k, const void* v, void* o, int 
   p.v_scale = v_scale;
   p.kv_mask = kv_mask;
   p.sm_b = sm_b;
+  p.kv_blocks = nullptr;
+  p.sb_b = 0;
   p.B = B;
   p.H = H;
   p.Q = Q;
@@ -156,10 +158,10 @@ static int xattn_impl(const void* q, const void* k, const void* v, void* o, int 
              (vt ? !cu_seqlens && sv_d % 8 == 0 && (D * sv_d + kv_cap) * 2 < (1ll << 32)
                  : sv_k % 8 == 0 && (kv_cap * sv_k + D) * 2 < (1ll << 32)));
   // Every form but the e4m3 second product is split, so that all layouts of the same keys are cut alike and give the
-  // same bits; a key mask needs the windows' lengths (svhip_mask_lengths), by which the line of key blocks is cut.
+  // same bits; a key mask needs the windows' lists of attended blocks (svhip_mask_blocks), by which the line is cut.
   p.part = nullptr;
   p.teams = 0;
-  if (workspace && !pv8 && !(kv_mask && !kv_len)) {
+  if (workspace && !pv8 && !(kv_mask && !(kv_len && kv_blocks))) {
     const int teams = split_teams(B, H, Q, kv_cap, resident(D));
     if (teams) {
       SVHIP_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
@@ -168,6 +170,10 @@ static int xattn_impl(const void* q, const void* k, const void* v, void* o, int 
                     svhip_xattn_workspace_bytes(B, H, Q, D, kv_cap));
       p.part = static_cast<float*>(workspace);
       p.teams = teams;
+      if (kv_mask) {
+        p.kv_blocks = kv_blocks;
+        p.sb_b = sb_b;
+      }
     }
   }
   hipStream_t s = as_stream(stream);
@@ -199,6 +205,67 @@ __global__ __launch_bounds__(kThreads) void mask_lengths_kernel(const uint8_t* m
   if (threadIdx.x == 0) out[b] = s_last + 1;
 }
 
+// One workgroup per window: mask_lengths_kernel's result, and the list of the window's 64-key blocks that hold an
+// attended key. A wave looks at one block at a time (a byte a lane, eight blocks' loads in flight), then every thread
+// places one block by the flags before it. Rounds of kListBlocks blocks.
+constexpr int kListThreads = 1024;
+constexpr int kListBlocks = kListThreads;
+__global__ __launch_bounds__(kListThreads) void mask_blocks_kernel(const uint8_t* mask, int64_t sm_b,
+                                                                   const int32_t* kv_len, int64_t kv_cap,
+                                                                   int32_t* lengths, int32_t* blocks, int64_t sb_b) {
+  constexpr int kWaves = kListThreads / 64, kAhead = 8;
+  __shared__ uint8_t s_flag[kListBlocks];
+  __shared__ int s_count[kWaves];
+  __shared__ int s_last;
+  const int64_t b = blockIdx.x;
+  int64_t cap = kv_cap;
+  if (kv_len) cap = min(max(static_cast<int64_t>(kv_len[b]), int64_t{0}), kv_cap);
+  const int n = static_cast<int>(cap), nb = static_cast<int>((cap + kKB - 1) / kKB);
+  const uint8_t* row = mask + b * sm_b;
+  int32_t* list = blocks + b * sb_b;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (threadIdx.x == 0) s_last = -1;
+  int placed = 0, last = -1;
+  for (int base = 0; base < nb; base += kListBlocks) {
+    const int count = min(nb - base, kListBlocks);
+    __syncthreads();  // the flags of the round before have been read
+    for (int k0 = w; k0 < count; k0 += kWaves * kAhead) {
+      uint8_t v[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int64_t j = static_cast<int64_t>(base + k0 + u * kWaves) * kKB + lane;
+        v[u] = row[j < n ? j : n - 1];
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int k = k0 + u * kWaves;
+        if (k >= count) break;
+        const int64_t j = static_cast<int64_t>(base + k) * kKB + lane;
+        const uint64_t bits = __ballot(j < n && v[u] != 0);
+        if (lane == 0) s_flag[k] = bits != 0ull;
+        if (bits != 0ull) last = max(last, (base + k) * kKB + 63 - __clzll(bits));
+      }
+    }
+    __syncthreads();
+    const bool on = static_cast<int>(threadIdx.x) < count && s_flag[threadIdx.x] != 0;
+    const uint64_t flags = __ballot(on);
+    if (lane == 0) s_count[w] = __popcll(flags);
+    __syncthreads();
+    int at = placed + __popcll(flags & ((1ull << lane) - 1ull));
+    for (int i = 0; i < kWaves; ++i) {
+      at += i < w ? s_count[i] : 0;
+      placed += s_count[i];
+    }
+    if (on) list[1 + at] = base + static_cast<int>(threadIdx.x);
+  }
+  if (lane == 0 && last >= 0) atomicMax(&s_last, last);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    lengths[b] = s_last + 1;
+    list[0] = placed;
+  }
+}
+
 }  // namespace svhip
 
 using namespace svhip;
@@ -213,6 +280,21 @@ extern "C" int svhip_mask_lengths(const uint8_t* kv_mask, int64_t sm_b, const in
   if (B == 0) return SVHIP_OK;
   mask_lengths_kernel<<<static_cast<unsigned>(B), kThreads, 0, as_stream(stream)>>>(kv_mask, sm_b, kv_len, kv_cap,
                                                                                       out);
+  SVHIP_LAUNCHED(name);
+  return SVHIP_OK;
+}
+
+extern "C" int svhip_mask_blocks(const uint8_t* kv_mask, int64_t sm_b, const int32_t* kv_len, int64_t B,
+                                 int64_t kv_cap, int32_t* lengths, int32_t* blocks, int64_t sb_b, void* stream) {
+  const char* name = "svhip_mask_blocks";
+  clear_error();
+  SVHIP_REQUIRE(kv_mask && lengths && blocks, "%s: null pointer", name);
+  SVHIP_REQUIRE(B >= 0 && B < (1ll << 31), "%s: bad window count", name);
+  SVHIP_REQUIRE(kv_cap >= 0 && kv_cap < (1ll << 31) - kKB, "%s: kv_cap out of range", name);
+  SVHIP_REQUIRE(B <= 1 || sb_b > cdiv(kv_cap, kKB), "%s: block rows shorter than the windows' lists", name);
+  if (B == 0) return SVHIP_OK;
+  mask_blocks_kernel<<<static_cast<unsigned>(B), kListThreads, 0, as_stream(stream)>>>(kv_mask, sm_b, kv_len, kv_cap,
+                                                                                         lengths, blocks, sb_b);
   SVHIP_LAUNCHED(name);
   return SVHIP_OK;
 }
@@ -249,7 +331,7 @@ extern "C" int svhip_xattn_fwd_ws(const void* q, const void* k, const void* v, v
   const char* name = "svhip_xattn_fwd";
   clear_error();
   SVHIP_REQUIRE(kv_len || cu_seqlens, "%s: need kv_len or cu_seqlens", name);
-  return xattn_impl(q, k, v, o, kv_dtype, kv_len, cu_seqlens, k_scale, v_scale, nullptr, 0, B, H, Q, D, kv_cap, sq_b,
+  return xattn_impl(q, k, v, o, kv_dtype, kv_len, cu_seqlens, k_scale, v_scale, nullptr, 0, nullptr, 0, B, H, Q, D, kv_cap, sq_b,
                     sq_h, sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, workspace,
                     workspace_bytes, stream, name);
 }
@@ -262,13 +344,14 @@ extern "C" int svhip_xattn_fwd_masked(const void* q, const void* k, const void* 
                                       int64_t so_q, float scale, void* stream) {
   clear_error();
   SVHIP_REQUIRE(!(kv_len && cu_seqlens), "svhip_xattn_fwd_masked: kv_len and cu_seqlens are exclusive");
-  return svhip_xattn_fwd_masked_ws(q, k, v, o, kv_mask, sm_b, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q,
+  return svhip_xattn_fwd_masked_ws(q, k, v, o, kv_mask, sm_b, kv_len, nullptr, 0, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q,
                                    sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0,
                                    stream);
 }
 
 extern "C" int svhip_xattn_fwd_masked_ws(const void* q, const void* k, const void* v, void* o, const uint8_t* kv_mask,
-                                      int64_t sm_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B,
+                                      int64_t sm_b, const int32_t* kv_len, const int32_t* kv_blocks, int64_t sb_b,
+                                         const int32_t* cu_seqlens, int64_t B,
                                       int64_t H, int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h,
                                       int64_t sq_q, int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b,
                                       int64_t sv_h, int64_t sv_k, int64_t sv_d, int64_t so_b, int64_t so_h,
@@ -277,7 +360,7 @@ extern "C" int svhip_xattn_fwd_masked_ws(const void* q, const void* k, const voi
   const char* name = "svhip_xattn_fwd_masked";
   clear_error();
   SVHIP_REQUIRE(kv_mask, "%s: null key mask", name);
-  return xattn_impl(q, k, v, o, SVHIP_BF16, kv_len, cu_seqlens, nullptr, nullptr, kv_mask, sm_b, B, H, Q, D, kv_cap,
+  return xattn_impl(q, k, v, o, SVHIP_BF16, kv_len, cu_seqlens, nullptr, nullptr, kv_mask, sm_b, kv_blocks, sb_b, B, H, Q, D, kv_cap,
                     sq_b, sq_h, sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, workspace, workspace_bytes, stream,
                     name);
 }

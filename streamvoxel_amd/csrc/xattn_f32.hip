@@ -35,7 +35,6 @@ constexpr int kF32Row = 64;      // floats of an LDS row (one key)
 constexpr int kF32Resident = 3;  // workgroups per CU (three waves per SIMD)
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 struct XattnF32Params {
   const float* q;
@@ -47,6 +46,8 @@ struct XattnF32Params {
   const uint8_t* kv_mask;  // KMASK: [B, kv_cap] bytes, rows sm_b apart
   const float* v_scale;    // none (the join's output scale)
   int64_t sm_b;
+  const int32_t* kv_blocks;  // SPLIT with KMASK: the windows' attended blocks (key_split.hpp)
+  int64_t sb_b;
   int64_t B, H, Q, D, kv_cap;
   int64_t sq_b, sq_h, sq_q;
   int64_t sk_b, sk_h, sk_k;
@@ -203,19 +204,30 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
         return j < L ? 1 : 0;
       }
     };
+    // First key of block i of the unit (with a key mask the i-th of the window's blocks with an attended key).
+    auto key_of = [&](int i) __attribute__((always_inline)) -> int {
+      if constexpr (SPLIT && KMASK) {
+        return kKB * listed_block(p, b, min(i, unit_blocks - 1));
+      } else {
+        return kKB * i;
+      }
+    };
     int on = 0;
     if (blk0 < blk1) {
-      load_block(blk0 * kKB);
-      on = load_mask(blk0 * kKB);
+      const int kv0 = key_of(blk0);
+      load_block(kv0);
+      on = load_mask(kv0);
       store_block();
     }
+    int kv_next = key_of(blk0 + 1);
     __syncthreads();
     for (int blk = blk0; blk < blk1; ++blk) {
       const uint64_t bits = __builtin_amdgcn_ballot_w64(on != 0);
       const bool more = blk + 1 < blk1;
       if (more) {
-        load_block((blk + 1) * kKB);
-        on = load_mask((blk + 1) * kKB);
+        load_block(kv_next);
+        on = load_mask(kv_next);
+        kv_next = key_of(blk + 2);
       }
       if (!KMASK || bits != 0ull) {
 #pragma unroll
@@ -323,7 +335,7 @@ template <int D, bool VT, bool KMASK>
 static void launch_f32(const XattnF32Params& p, unsigned grid, hipStream_t s) {
   if (p.teams) {
     xattn_f32_kernel<D, VT, KMASK, true><<<static_cast<unsigned>(p.teams) * p.q_tiles, kThreads, 0, s>>>(p);
-    split_join_kernel<float><<<dim3(grid, static_cast<unsigned>(cdiv(D, kJoinDims))), kThreads, 0, s>>>(p);
+    split_join_kernel<float><<<split_join_grid(grid, D), kThreads, 0, s>>>(p);
   } else {
     xattn_f32_kernel<D, VT, KMASK, false><<<grid, kThreads, 0, s>>>(p);
   }
@@ -343,7 +355,7 @@ static void launch_f32(const XattnF32Params& p, unsigned grid, hipStream_t s, bo
 using namespace svhip;
 
 static int xattn_f32_impl(const float* q, const float* k, const float* v, float* o, const uint8_t* kv_mask,
-                          int64_t sm_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B, int64_t H,
+                          int64_t sm_b, const int32_t* kv_blocks, int64_t sb_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B, int64_t H,
                           int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q,
                           int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k,
                           int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* workspace,
@@ -355,7 +367,7 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   } else {
     SVHIP_REQUIRE(kv_len || cu_seqlens, "%s: need kv_len or cu_seqlens", name);
   }
-  SVHIP_REQUIRE(!(kv_len && cu_seqlens), "%s: kv_len and cu_seqlens are exclusive", name);
+  SVHIP_REQUIRE(!(kv_len && cu_seqlens) || kv_blocks, "%s: kv_len and cu_seqlens are exclusive", name);
   SVHIP_REQUIRE(B >= 0 && H >= 1 && Q >= 0, "%s: bad sizes", name);
   SVHIP_REQUIRE(D == 16 || D == 32 || D == 48 || D == 64, "%s: head_dim %lld unsupported (16, 32, 48 or 64)", name,
                 (long long)D);
@@ -381,6 +393,8 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   p.kv_mask = kv_mask;
   p.v_scale = nullptr;
   p.sm_b = sm_b;
+  p.kv_blocks = nullptr;
+  p.sb_b = 0;
   p.B = B;
   p.H = H;
   p.Q = Q;
@@ -405,7 +419,8 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   SVHIP_REQUIRE(grid < (1ll << 31), "%s: grid too large", name);
   p.part = nullptr;
   p.teams = 0;
-  if (workspace) {
+  // A key mask needs the windows' lists of attended blocks (svhip_mask_blocks), by which the line is cut.
+  if (workspace && !(kv_mask && !(kv_len && kv_blocks))) {
     const int teams = split_teams(B, H, Q, kv_cap, kF32Resident);
     const size_t need = split_workspace_bytes(B, H, Q, D, kv_cap, kF32Resident);
     if (teams) {
@@ -413,6 +428,10 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
                     "%s: workspace too small or unaligned (%zu < %zu bytes)", name, workspace_bytes, need);
       p.part = static_cast<float*>(workspace);
       p.teams = teams;
+      if (kv_mask) {
+        p.kv_blocks = kv_blocks;
+        p.sb_b = sb_b;
+      }
     }
   }
   hipStream_t s = as_stream(stream);
@@ -441,14 +460,15 @@ extern "C" size_t svhip_xattn_f32_workspace_bytes(int64_t B, int64_t H, int64_t 
 }
 
 extern "C" int svhip_xattn_fwd_f32_ws(const float* q, const float* k, const float* v, float* o, const uint8_t* kv_mask,
-                                      int64_t sm_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B,
+                                      int64_t sm_b, const int32_t* kv_len, const int32_t* kv_blocks, int64_t sb_b,
+                                      const int32_t* cu_seqlens, int64_t B,
                                       int64_t H, int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h,
                                       int64_t sq_q, int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b,
                                       int64_t sv_h, int64_t sv_k, int64_t sv_d, int64_t so_b, int64_t so_h,
                                       int64_t so_q, float scale, void* workspace, size_t workspace_bytes,
                                       void* stream) {
-  return xattn_f32_impl(q, k, v, o, kv_mask, sm_b, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b, sk_h,
-                        sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, workspace, workspace_bytes, stream,
+  return xattn_f32_impl(q, k, v, o, kv_mask, sm_b, kv_blocks, sb_b, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h,
+                        sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, workspace, workspace_bytes, stream,
                         "svhip_xattn_fwd_f32_ws");
 }
 
@@ -457,7 +477,7 @@ extern "C" int svhip_xattn_fwd_f32(const float* q, const float* k, const float* 
                                    int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q, int64_t sk_b,
                                    int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k, int64_t sv_d,
                                    int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* stream) {
-  return xattn_f32_impl(q, k, v, o, nullptr, 0, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b, sk_h,
+  return xattn_f32_impl(q, k, v, o, nullptr, 0, nullptr, 0, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b, sk_h,
                         sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0, stream,
                         "svhip_xattn_fwd_f32");
 }
@@ -472,7 +492,7 @@ extern "C" int svhip_xattn_fwd_f32_masked(const float* q, const float* k, const 
   const char* name = "svhip_xattn_fwd_f32_masked";
   clear_error();
   SVHIP_REQUIRE(kv_mask, "%s: null key mask", name);
-  return xattn_f32_impl(q, k, v, o, kv_mask, sm_b, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b,
+  return xattn_f32_impl(q, k, v, o, kv_mask, sm_b, nullptr, 0, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b,
                         sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0, stream,
                         name);
 }

@@ -79,7 +79,6 @@ namespace svhip {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
 
@@ -186,6 +185,8 @@ struct XattnParams {
   const float* v_scale;
   const uint8_t* kv_mask;  // optional key mask: key j of window b is attended iff kv_mask[b * sm_b + j] != 0
   int64_t sm_b;
+  const int32_t* kv_blocks;  // key split with a key mask: the windows' attended blocks (key_split.hpp)
+  int64_t sb_b;
   int64_t B, H, Q, D, kv_cap;
   int64_t sq_b, sq_h, sq_q;
   int64_t sk_b, sk_h, sk_k;
@@ -762,7 +763,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     const int bw = split_window(p, plan, pos);
     unit_blocks = __builtin_amdgcn_readlane(plan.blocks, bw);
     const int rel = pos - static_cast<int>(p.H) * __builtin_amdgcn_readlane(plan.before, bw);
-    const int hw = rel / unit_blocks;
+    const int hw = __builtin_amdgcn_readfirstlane(rel / unit_blocks);
     b = bw;
     h = hw;
     blk0 = rel - hw * unit_blocks;
@@ -777,7 +778,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   const int L = [&]() __attribute__((always_inline)) {
     const int n = window_length(p, b);
     if constexpr (!KMASK || SPLIT) {
-      return n;
+      return __builtin_amdgcn_readfirstlane(n);
     } else {
       // With a key mask the window ends at its last attended key: the blocks after it add nothing to O, l or m.
       // One scan of the window's mask row (a wave-uniform result; no attended key gives L = 0 and zeros).
@@ -787,7 +788,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
       const int last = last_attended(p.kv_mask + b * p.sm_b, n);
       if (last >= 0) atomicMax(&s_last, last);
       __syncthreads();
-      return s_last + 1;
+      return __builtin_amdgcn_readfirstlane(s_last) + 1;
     }
   }();
 
@@ -826,8 +827,24 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   // V^T rows allow vector loads when every 8-key run starts aligned (the base, the row stride and the offset).
   const bool vt_vec = VT && ((reinterpret_cast<uintptr_t>(V) & (FP8 ? 7 : 15)) == 0) && (p.sv_d % 8 == 0);
   const int nfull = L / kKB;           // full key blocks
-  const int full_end = SPLIT ? min(blk1, nfull) : nfull;         // end of this part's full blocks
-  const bool tail = SPLIT ? blk1 > nfull : nfull * kKB < L;      // plus one partial block
+  // End of this part's full blocks, and whether the unit's last, partial block follows.
+  const bool partial = nfull * kKB < L;
+  const int full_end = SPLIT ? min(blk1, unit_blocks - (partial ? 1 : 0)) : nfull;
+  const bool tail = SPLIT ? partial && blk1 == unit_blocks : partial;
+  // LIST: block i of the unit is the i-th of the window's blocks with an attended key.
+  constexpr bool LIST = SPLIT && KMASK;
+  auto key_of = [&](int i) __attribute__((always_inline)) -> int {
+    if constexpr (LIST) {
+      return kKB * listed_block(p, b, min(i, unit_blocks - 1));
+    } else {
+      return kKB * i;
+    }
+  };
+  [[maybe_unused]] int kv_cur = 0, kv_next = 0;  // LIST: first keys of the current and the next block
+  if constexpr (LIST) {
+    kv_cur = key_of(blk0);
+    kv_next = key_of(blk0 + 1);
+  }
 
   DirectLanes<DT> dl;
   if constexpr (DIRECT) {
@@ -951,22 +968,21 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   // that key's score however far below 0 it lies.
   [[maybe_unused]] bool placeholder = false;
 
-  // Full block `blk` into (sK, sV): issued now, complete at the next vmem wait (direct) or at `stage_commit`
+  // The full block at key kv0 into (sK, sV): issued now, complete at the next vmem wait (direct) or at `stage_commit`
   // (registers, prefetched into `st`).
   Stage<FP8, VT, DT> st;
-  auto stage_issue = [&](int blk, uint16_t* sK, uint16_t* sV) __attribute__((always_inline)) {
+  auto stage_issue = [&](int kv0, uint16_t* sK, uint16_t* sV) __attribute__((always_inline)) {
     if constexpr (DIRECT) {
-      const int kv0 = blk * kKB;
       stage_direct<DT, STAGING == kDirectFull, VT>(dl, static_cast<uint32_t>(kv0 * p.sk_k * 2),
                                                    static_cast<uint32_t>(kv0 * 2), w, sK, sV);
       if constexpr (VROWS) stage_rows<DT, STAGING == kDirectFull>(dr, static_cast<uint32_t>(kv0 * p.sv_k * 2), w, sV);
     } else {
-      stage_load<FP8, VT, DT, false, ONES, !VD8>(st, p, K, V, L, blk * kKB, dchunks, vt_vec, tid);
+      stage_load<FP8, VT, DT, false, ONES, !VD8>(st, p, K, V, L, kv0, dchunks, vt_vec, tid);
       if constexpr (VD8) {
 #pragma unroll
         for (int t = 0; t < (2 * DT + 3) / 4; ++t) {
           const int j = w + 4 * t;
-          if (j < 2 * DT && dv.ok[t]) direct_v8_load(dv.rsrc, dv.off[t], static_cast<uint32_t>(blk * kKB), sV, j);
+          if (j < 2 * DT && dv.ok[t]) direct_v8_load(dv.rsrc, dv.off[t], static_cast<uint32_t>(kv0), sV, j);
         }
       }
     }
@@ -986,18 +1002,19 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   // blocks are computed in order, so each call takes the byte the previous one fetched (lane l: key kv0 + l) and
   // fetches the next block's: its load completes under the block's compute instead of stalling the next block.
   const uint8_t* mrow = KMASK ? p.kv_mask + b * p.sm_b : nullptr;
-  [[maybe_unused]] int mask_on = 0;
+  // (The byte is kept as loaded, from a clamped index: a test or a branch beside the load would wait for it there.)
+  [[maybe_unused]] int mask_byte = 0, mask_kv0 = 0;
   auto mask_fetch = [&](int kv0) __attribute__((always_inline)) {
     if constexpr (KMASK) {
-      const int j = kv0 + lane;
-      mask_on = (j < L && mrow[j] != 0) ? 1 : 0;
+      mask_kv0 = kv0;
+      mask_byte = mrow[min(kv0 + lane, L - 1)];
     }
   };
-  mask_fetch(blk0 * kKB);
-  auto block_bits = [&](int kv0) __attribute__((always_inline)) -> uint64_t {
+  mask_fetch(key_of(blk0));
+  auto block_bits = [&](int next_kv0) __attribute__((always_inline)) -> uint64_t {
     if constexpr (KMASK) {
-      const uint64_t bits = __builtin_amdgcn_ballot_w64(mask_on != 0);
-      mask_fetch(kv0 + kKB);
+      const uint64_t bits = __builtin_amdgcn_ballot_w64(mask_byte != 0 && mask_kv0 + lane < L);
+      mask_fetch(next_kv0);
       return bits;
     } else {
       return ~0ull;
@@ -1348,9 +1365,16 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   // mask bytes (loaded during the previous block, waited for at its end) then waits for nothing in flight, where
   // after those loads it waited for them all.
   auto full_step = [&](int blk, const uint16_t* Ks, const uint16_t* Vt, uint16_t* nK, uint16_t* nV) __attribute__((always_inline)) {
-    const uint64_t bits = block_bits(blk * kKB);
-    stage_issue(blk + 1, nK, nV);
-    compute(Full{}, Ks, Vt, blk * kKB, bits);
+    const int kv0 = LIST ? kv_cur : blk * kKB, next = LIST ? kv_next : (blk + 1) * kKB;
+    [[maybe_unused]] int after = 0;
+    if constexpr (LIST) after = key_of(blk + 2);
+    const uint64_t bits = block_bits(next);
+    stage_issue(next, nK, nV);
+    compute(Full{}, Ks, Vt, kv0, bits);
+    if constexpr (LIST) {
+      kv_cur = next;
+      kv_next = after;
+    }
     stage_commit(nK, nV);
     wait_vmem();
     __syncthreads();
@@ -1358,7 +1382,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   };
 
   if (full_end > blk0) {
-    stage_issue(blk0, sK0, sV0);
+    stage_issue(key_of(blk0), sK0, sV0);
     stage_commit(sK0, sV0);
   } else {
     stage_tail(sK0, sV0);
@@ -1384,20 +1408,21 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     if (full_end > blk0) {
       // The partial block's loads are in flight during the last full block (the other tiles are free since the
       // last barrier).
-      const uint64_t bits = block_bits(blk * kKB);
+      const int kv0 = LIST ? kv_cur : blk * kKB;
+      const uint64_t bits = block_bits(LIST ? kv_next : kv0 + kKB);
       Stage<FP8, VT, DT> tl;
       if (tail) stage_load<FP8, VT, DT, true, ONES>(tl, p, K, V, L, nfull * kKB, dchunks, vt_vec, tid);
-      compute(Full{}, cK, cV, blk * kKB, bits);
+      compute(Full{}, cK, cV, kv0, bits);
       settle();
       if (tail) {
         stage_store<FP8, VT, DT, ONES, PV8>(tl, nK, nV, dchunks, Dv, tid);
         wait_vmem();
         __syncthreads();
-        compute(Partial{}, nK, nV, nfull * kKB, block_bits(nfull * kKB));
+        compute(Partial{}, nK, nV, nfull * kKB, block_bits(L));
         settle();
       }
     } else {
-      compute(Partial{}, cK, cV, blk0 * kKB, block_bits(blk0 * kKB));
+      compute(Partial{}, cK, cV, nfull * kKB, block_bits(L));
       settle();
     }
   }
@@ -1508,7 +1533,7 @@ void launch_split_impl(const XattnParams& p, unsigned g, hipStream_t s, bool fp8
     vt ? SVHIP_SPLIT(false, true, RS, false) : SVHIP_SPLIT(false, false, RS, false);
   }
 #undef SVHIP_SPLIT
-  split_join_kernel<uint16_t><<<dim3(g, static_cast<unsigned>(cdiv(p.D, kJoinDims))), kThreads, 0, s>>>(p);
+  split_join_kernel<uint16_t><<<split_join_grid(g, p.D), kThreads, 0, s>>>(p);
 }
 
 }  // namespace svhip

@@ -104,11 +104,12 @@ def attention(query, key, val, lengths=None, cu_seqlens=None, scale=None, k_scal
         if cu_seqlens is None and key_mask.shape[1] < kcap:
             raise ValueError(f'key_mask holds {key_mask.shape[1]} keys per window, the cache {kcap}')
         mask_cap = kcap if cu_seqlens is None else key_mask.shape[1]
-        if cu_seqlens is None or nbytes:
-            # The windows' lengths cut at their last attended keys (the same output): the kernel shares the key
-            # blocks out by them, which balances the CUs when the mask, not `lengths`, holds the window lengths.
-            if cu_seqlens is not None:
-                lengths = cu_seqlens[1:] - cu_seqlens[:-1]
+        blocks = None
+        if nbytes:
+            lengths, blocks = _attended_blocks(key_mask, lengths, cu_seqlens, mask_cap)
+        elif cu_seqlens is None:
+            # The windows' lengths cut at their last attended keys (the same output): the kernel ranks the
+            # windows by them, which balances the CUs when the mask, not `lengths`, holds the window lengths.
             cut = torch.empty(B, dtype=torch.int32, device=query.device)
             _lib.check(lib.svhip_mask_lengths(_lib.ptr(key_mask.view(torch.uint8)), key_mask.stride(0),
                                               _lib.ptr(lengths), B, mask_cap, _lib.ptr(cut), _lib.stream_of(query)),
@@ -116,7 +117,8 @@ def attention(query, key, val, lengths=None, cu_seqlens=None, scale=None, k_scal
             lengths = cut
         _lib.check(lib.svhip_xattn_fwd_masked_ws(
             _lib.ptr(query), _lib.ptr(key), _lib.ptr(val), _lib.ptr(out), _lib.ptr(key_mask.view(torch.uint8)),
-            key_mask.stride(0), _lib.ptr(lengths), _lib.ptr(cu_seqlens), B, H, Q, D, mask_cap,
+            key_mask.stride(0), _lib.ptr(lengths), _lib.ptr(blocks), 0 if blocks is None else blocks.stride(0),
+            _lib.ptr(cu_seqlens), B, H, Q, D, mask_cap,
             query.stride(0), query.stride(1), query.stride(2),
             *sk, *sv, out.stride(0), out.stride(1), out.stride(2), scale, _lib.ptr(ws), nbytes,
             _lib.stream_of(query)), 'svhip_xattn_fwd_masked')
@@ -129,6 +131,20 @@ def attention(query, key, val, lengths=None, cu_seqlens=None, scale=None, k_scal
         *sk, *sv, out.stride(0), out.stride(1), out.stride(2), scale, _lib.ptr(ws), nbytes, _lib.stream_of(query)),
         'svhip_xattn_fwd')
     return out
+
+
+def _attended_blocks(key_mask, lengths, cu_seqlens, cap):
+    """(lengths, blocks) of a key mask for the key split: the windows cut at their last attended keys and, in row b of
+    blocks, the count and the indices of the 64-key blocks that hold an attended key (svhip_mask_blocks)."""
+    B = key_mask.shape[0]
+    if cu_seqlens is not None:
+        lengths = cu_seqlens[1:] - cu_seqlens[:-1]
+    cut = torch.empty(B, dtype=torch.int32, device=key_mask.device)
+    blocks = torch.empty(B, 1 + (cap + 63) // 64, dtype=torch.int32, device=key_mask.device)
+    _lib.check(_lib.load().svhip_mask_blocks(_lib.ptr(key_mask.view(torch.uint8)), key_mask.stride(0),
+                                             _lib.ptr(lengths), B, cap, _lib.ptr(cut), _lib.ptr(blocks),
+                                             blocks.stride(0), _lib.stream_of(key_mask)), 'svhip_mask_blocks')
+    return cut, blocks
 
 
 def _attention_f32(query, key, val, lengths, cu_seqlens, scale, out, key_mask=None):
@@ -177,9 +193,13 @@ def _attention_f32(query, key, val, lengths, cu_seqlens, scale, out, key_mask=No
     nbytes = int(lib.svhip_xattn_f32_workspace_bytes(B, H, Q, D, mask_cap))
     ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device) if nbytes else None
     mask = None if key_mask is None else key_mask.view(torch.uint8)
+    blocks = None
+    if mask is not None and nbytes:
+        lengths, blocks = _attended_blocks(key_mask, lengths, cu_seqlens, mask_cap)
     _lib.check(lib.svhip_xattn_fwd_f32_ws(
         _lib.ptr(query), _lib.ptr(key), _lib.ptr(val), _lib.ptr(out), _lib.ptr(mask),
-        0 if mask is None else mask.stride(0), _lib.ptr(lengths), _lib.ptr(cu_seqlens), B, H, Q, D, mask_cap,
+        0 if mask is None else mask.stride(0), _lib.ptr(lengths), _lib.ptr(blocks),
+        0 if blocks is None else blocks.stride(0), _lib.ptr(cu_seqlens), B, H, Q, D, mask_cap,
         query.stride(0), query.stride(1), query.stride(2), *sk, *sv, out.stride(0), out.stride(1), out.stride(2),
         scale, _lib.ptr(ws), nbytes, _lib.stream_of(query)), 'svhip_xattn_fwd_f32_ws')
     return out

@@ -159,3 +159,34 @@ def test_split_replays_in_a_graph(dev):
         want = attention(q, k, v, lengths=lt)
         torch.cuda.synchronize()
         assert torch.equal(out, want), lengths
+
+
+@pytest.mark.parametrize('cap', [1, 63, 64, 65, 1000, 70001])
+def test_mask_blocks_against_torch(dev, cap):
+    """Lengths and lists of attended blocks: capacities around a block and past one round of 1024 blocks, rows of any
+    alignment, windows cut by kv_len, empty ones."""
+    from streamvoxel_amd import _lib
+    g = torch.Generator().manual_seed(cap)
+    B, nb = 5, (cap + 63) // 64
+    mask = torch.rand(B, cap + 3, generator=g) < 0.02
+    mask[1] = True
+    mask[2] = False
+    lens = torch.tensor([cap, cap, cap, cap // 2, 0], dtype=torch.int32)
+    dm = mask.to(dev)
+    lib = _lib.load()
+    for given in (False, True):
+        _case(f'mask blocks cap={cap} lengths={given}')
+        out = torch.full((B,), -7, dtype=torch.int32, device=dev)
+        blocks = torch.full((B, nb + 2), -7, dtype=torch.int32, device=dev)
+        dl = lens.to(dev)
+        _lib.check(lib.svhip_mask_blocks(_lib.ptr(dm.view(torch.uint8)), dm.stride(0), _lib.ptr(dl) if given else None, B,
+                                         cap, _lib.ptr(out), _lib.ptr(blocks), nb + 2, _lib.stream_of(dm)),
+                   'svhip_mask_blocks')
+        torch.cuda.synchronize()
+        for b in range(B):
+            row = mask[b, :int(lens[b]) if given else cap]
+            at = row.nonzero().flatten()
+            want = sorted({int(i) // 64 for i in at})
+            assert int(out[b]) == (int(at[-1]) + 1 if len(at) else 0)
+            assert blocks[b, 0] == len(want) and blocks[b, 1:1 + len(want)].tolist() == want
+            assert (blocks[b, 1 + len(want):] == -7).all()
