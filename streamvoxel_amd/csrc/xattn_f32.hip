@@ -21,18 +21,24 @@
 // The split form (SPLIT) is the bf16 kernel's: see key_split.hpp.
 //
 // One window of 12 x 64 heads, 1024 queries, 9744 keys: 816 us on the VALU (one query a lane, K and V rows broadcast from
-// LDS: 37 TFLOP/s), 283 us here (108 TFLOP/s), 12 us of it the join. The matrix cores are busy 0.70 of the kernel: the
-// three waves of a SIMD do not finish together, and the last one alone does not fill them.
+// LDS: 37 TFLOP/s), 275 us here (112 TFLOP/s), 7 us of it the join. The instruction alone reaches 141 TFLOP/s with two
+// waves a SIMD and dependent accumulators, 147 with three.
 //
 // KMASK: a key mask on top of the window length (the reference's `prefix_valid ++ local_valid`): key j of window b
 // is attended only where kv_mask[b * sm_b + j] != 0. A block that the mask wholly masks is skipped; a query may have
 // seen no attended key yet, its running max then stays -inf and the exponentials are taken against 0.
+#include <type_traits>
+
 #include "key_split.hpp"
 
 namespace svhip {
 
 constexpr int kF32Row = 64;      // floats of an LDS row (one key)
-constexpr int kF32Resident = 3;  // workgroups per CU (three waves per SIMD)
+constexpr int kF32Resident = 2;  // workgroups per CU (two waves per SIMD)
+// Key blocks summed into one accumulator before it is added to the total: shorter chains of fp32 sums (one chain of 29
+// blocks is 8.1e-7 from float64 on the single-column configuration, 5.0e-7 with this; 7.3e-7 on the VALU before).
+constexpr int kF32Fold = 8;
+constexpr float kF32Rise = 16.f;
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
@@ -121,7 +127,7 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
       const int bw = split_window(p, plan, pos);
       unit_blocks = __builtin_amdgcn_readlane(plan.blocks, bw);
       const int rel = pos - static_cast<int>(p.H) * __builtin_amdgcn_readlane(plan.before, bw);
-      const int hw = rel / unit_blocks;
+      const int hw = __builtin_amdgcn_readfirstlane(rel / unit_blocks);
       b = bw;
       h = hw;
       blk0 = rel - hw * unit_blocks;
@@ -150,9 +156,9 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
       qf[4 * s + 2] = x.z;
       qf[4 * s + 3] = x.w;
     }
-    f32x16_t o[kTiles];
+    f32x16_t o[kTiles], total[kTiles];  // O^T of the last blocks, and of those before
 #pragma unroll
-    for (int j = 0; j < kTiles; ++j) o[j] = f32x16_t{0};
+    for (int j = 0; j < kTiles; ++j) o[j] = total[j] = f32x16_t{0};
     float m = -INFINITY, l = 0.f;  // l: the lane's own keys
 
     // Block loads: chunk c = thread + 256 r is key c / kChunks, head_dim 4 (c % kChunks) .. + 3 (of V^T key c % 64,
@@ -207,7 +213,7 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
     // First key of block i of the unit (with a key mask the i-th of the window's blocks with an attended key).
     auto key_of = [&](int i) __attribute__((always_inline)) -> int {
       if constexpr (SPLIT && KMASK) {
-        return kKB * listed_block(p, b, min(i, unit_blocks - 1));
+        return kKB * (p.kv_blocks ? listed_block(p, b, min(i, unit_blocks - 1)) : i);
       } else {
         return kKB * i;
       }
@@ -230,18 +236,45 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
         kv_next = key_of(blk + 2);
       }
       if (!KMASK || bits != 0ull) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        // One weight, formed where it stands in the code: the volatile asm keeps it from sinking to its use.
+        auto weight = [&](float& x, float nm, float& sum) __attribute__((always_inline)) {
+          x = __builtin_amdgcn_exp2f(__builtin_fmaf(x, sl2, nm));
+          sum += x;
+          asm volatile("" : "+v"(x), "+v"(sum));
+        };
+        // S^T of half t (keys 32 t .. 32 t + 31 of the block), the weights of `w` (UNDER) between its products.
+        auto score = [&](int t, auto under, f32x16_t& w) __attribute__((always_inline)) {
+          constexpr bool UNDER = decltype(under)::value;
+          constexpr int kSteps = D / 8, kEach = (16 + kSteps - 1) / kSteps;
+          const float nm = UNDER ? (m == -INFINITY ? 0.f : -m) : 0.f;
           f32x16_t s;
+          float sum = 0.f;
           const float* kr = sK + (32 * t + col) * kF32Row;
+          f32x4_t x = *reinterpret_cast<const f32x4_t*>(kr + 4 * f32_swz_k(col, hh));
 #pragma unroll
-          for (int c = 0; c < D / 8; ++c) {
-            const float4 x = *reinterpret_cast<const float4*>(kr + 4 * f32_swz_k(col, 2 * c + hh));
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, qf[4 * c], c == 0 ? f32x16_t{0} : s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, qf[4 * c + 1], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, qf[4 * c + 2], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, qf[4 * c + 3], s, 0, 0, 0);
+          for (int c = 0; c < kSteps; ++c) {
+            f32x4_t next = x;
+            if (c + 1 < kSteps) next = *reinterpret_cast<const f32x4_t*>(kr + 4 * f32_swz_k(col, 2 * (c + 1) + hh));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              s = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], qf[4 * c + e], c + e == 0 ? f32x16_t{0} : s, 0, 0, 0);
+            }
+            x = next;
+            if constexpr (UNDER) {
+#pragma unroll
+              for (int i = kEach * c; i < kEach * (c + 1) && i < 16; ++i) {
+                float y = w[i];
+                weight(y, nm, sum);
+                w[i] = y;
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
           }
+          if constexpr (UNDER) l += sum;
+          return s;
+        };
+        // The half's largest score, keys not attended put to -inf.
+        auto mask_max = [&](f32x16_t& s, int t) __attribute__((always_inline)) {
           if (bits != ~0ull) {
             const uint32_t mine = static_cast<uint32_t>(bits >> (32 * t)) >> (4 * hh);
 #pragma unroll
@@ -252,36 +285,79 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
           float mb = s[0];
 #pragma unroll
           for (int i = 1; i < 16; ++i) mb = fmaxf(mb, s[i]);
-          mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
-          const float mn = fmaxf(m, mb * sl2);
-          if (__builtin_amdgcn_ballot_w64(mn > m) != 0ull) {
+          return fmaxf(mb, __shfl_xor(mb, 32, 64)) * sl2;
+        };
+        // The running max is raised only where a score passes it by kF32Rise (the weights stay below 2^kF32Rise, which
+        // costs fp32 sums nothing); O, l and the weights `held` already formed come down with it.
+        auto raise = [&](float mb, f32x16_t* held) __attribute__((always_inline)) {
+          if (__builtin_amdgcn_ballot_w64(mb > m + kF32Rise) != 0ull) {
             // alpha is 0 on a query's first attended keys (m = -inf), with O and l still 0.
-            const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+            const float mn = fmaxf(m, mb);
+            const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
             m = mn;
             l *= alpha;
 #pragma unroll
             for (int j = 0; j < kTiles; ++j) {
 #pragma unroll
-              for (int i = 0; i < 16; ++i) o[j][i] *= alpha;
+              for (int i = 0; i < 16; ++i) {
+                o[j][i] *= alpha;
+                total[j][i] *= alpha;
+              }
+            }
+            if (held) {
+#pragma unroll
+              for (int i = 0; i < 16; ++i) (*held)[i] *= alpha;
             }
           }
-          const float nm = m == -INFINITY ? 0.f : -m;
+        };
+        // O^T += V^T . P^T of half t, the weights of `w` (UNDER) between its products.
+        auto pv = [&](const f32x16_t& s, int t, auto under, f32x16_t& w) __attribute__((always_inline)) {
+          constexpr bool UNDER = decltype(under)::value;
+          const float nm = UNDER ? (m == -INFINITY ? 0.f : -m) : 0.f;
           float sum = 0.f;
+          // Entry i is key 32 t + 8 (i / 4) + 4 hh + i % 4; f32_swz_v on floats: bit 5 of the row's float index flips
+          // with bit 2 of the key, which is hh.
+          auto read = [&](int i, int j) __attribute__((always_inline)) {
+            return sV[(32 * t + 8 * (i / 4) + 4 * hh + i % 4) * kF32Row + ((32 * j + col) ^ (32 * hh))];
+          };
+          float x[kTiles], next[kTiles];
+#pragma unroll
+          for (int j = 0; j < kTiles; ++j) x[j] = read(0, j);
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
-            s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], sl2, nm));
-            sum += s[i];
-          }
-          l += sum;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int key = 32 * t + 8 * (i / 4) + 4 * hh + i % 4;
-            // f32_swz_v on floats: bit 5 of the row's float index flips with bit 2 of the key, which is hh.
-            const float* vr = sV + key * kF32Row;
+            for (int j = 0; j < kTiles; ++j) next[j] = i + 1 < 16 ? read(i + 1, j) : 0.f;
 #pragma unroll
             for (int j = 0; j < kTiles; ++j) {
-              o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[(32 * j + col) ^ (32 * hh)], s[i], o[j], 0, 0, 0);
+              o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[j], s[i], o[j], 0, 0, 0);
+              x[j] = next[j];
             }
+            if constexpr (UNDER) {
+              float y = w[i];
+              weight(y, nm, sum);
+              w[i] = y;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if constexpr (UNDER) l += sum;
+        };
+        // Half 0's weights under half 1's score product, half 1's under half 0's second product (a product is 16 passes,
+        // a weight three VALU instructions): a wave left alone on its SIMD still keeps the matrix core busy.
+        f32x16_t none;
+        f32x16_t s0 = score(0, std::false_type{}, none);
+        raise(mask_max(s0, 0), nullptr);
+        f32x16_t s1 = score(1, std::true_type{}, s0);
+        raise(mask_max(s1, 1), &s0);
+        pv(s0, 0, std::true_type{}, s1);
+        pv(s1, 1, std::false_type{}, none);
+      }
+      if ((blk - blk0) % kF32Fold == kF32Fold - 1 || !more) {
+#pragma unroll
+        for (int j = 0; j < kTiles; ++j) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            total[j][i] += o[j][i];
+            o[j][i] = 0.f;
           }
         }
       }
@@ -304,7 +380,7 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
           for (int g = 0; g < 4; ++g) {
             const int d0 = 32 * j + 8 * g + 4 * hh;
             if (d0 < D) {
-              split_store(slot, d0, ql, o[j][4 * g], o[j][4 * g + 1], o[j][4 * g + 2], o[j][4 * g + 3]);
+              split_store(slot, d0, ql, total[j][4 * g], total[j][4 * g + 1], total[j][4 * g + 2], total[j][4 * g + 3]);
             }
           }
         }
@@ -324,7 +400,7 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const int d = 32 * j + 8 * (i / 4) + 4 * hh + i % 4;
-          if (d < D) out[d] = o[j][i] * inv;
+          if (d < D) out[d] = total[j][i] * inv;
         }
       }
     }
@@ -419,8 +495,9 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   SVHIP_REQUIRE(grid < (1ll << 31), "%s: grid too large", name);
   p.part = nullptr;
   p.teams = 0;
-  // A key mask needs the windows' lists of attended blocks (svhip_mask_blocks), by which the line is cut.
-  if (workspace && !(kv_mask && !(kv_len && kv_blocks))) {
+  // Several windows with a key mask need their lists of attended blocks (svhip_mask_blocks), by which the line is cut; a
+  // single one is cut by its capacity.
+  if (workspace && !(kv_mask && B > 1 && !(kv_len && kv_blocks))) {
     const int teams = split_teams(B, H, Q, kv_cap, kF32Resident);
     const size_t need = split_workspace_bytes(B, H, Q, D, kv_cap, kF32Resident);
     if (teams) {
