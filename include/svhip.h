@@ -188,7 +188,8 @@ int svhip_xattn_fwd(const void* q, const void* k, const void* v, void* o, int kv
  * svhip_xattn_fwd with scratch memory, with which the keys of a (window, head) may be split over several workgroups
  * (few windows, or windows of different lengths, otherwise leave part of the chip idle): 16-byte aligned, at least
  * svhip_xattn_workspace_bytes(B, H, Q, D, kv_cap) bytes, its content of no meaning before or after the call. The
- * query returns 0 where these sizes are never split; a NULL workspace never splits. The parts are joined in fp32.
+ * query returns 0 where these sizes are never split; a NULL workspace and an e4m3 cache never split. The parts are
+ * joined in fp32; where a window's keys are cut depends on all windows' lengths, so the last bits of its result do too.
  */
 size_t svhip_xattn_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap);
 int svhip_xattn_fwd_ws(const void* q, const void* k, const void* v, void* o, int kv_dtype, const int32_t* kv_len,

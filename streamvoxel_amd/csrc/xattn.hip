@@ -10,7 +10,7 @@ template <int DT, bool ONES>
 void launch_dt(const XattnParams& p, unsigned g, hipStream_t s, bool fp8, bool pv8, bool vt, bool direct) {
   constexpr int RS = ONES ? kRegister : kRegisterFull;
   if (p.teams) {
-    launch_split<DT, ONES>(p, g, s, fp8, vt, direct);
+    launch_split<DT, ONES>(p, g, s, vt, direct);
     return;
   }
   if (p.kv_mask) {  // bf16 only (checked by the entry point)
@@ -157,11 +157,11 @@ static int xattn_impl(const void* q, const void* k, const void* v, void* o, int 
              (kv_cap * sk_k + D) * 2 < (1ll << 32) &&
              (vt ? !cu_seqlens && sv_d % 8 == 0 && (D * sv_d + kv_cap) * 2 < (1ll << 32)
                  : sv_k % 8 == 0 && (kv_cap * sv_k + D) * 2 < (1ll << 32)));
-  // Every form but the e4m3 second product is split, so that all layouts of the same keys are cut alike and give the
-  // same bits; a key mask needs the windows' lists of attended blocks (svhip_mask_blocks), by which the line is cut.
+  // Every bf16 form is split, so that all layouts of the same keys are cut alike and give the same bits. An e4m3 cache
+  // is not: its windows' bits do not depend on the batch they are attended in, and the cuts of the line do. A key mask needs the windows' lists of attended blocks (svhip_mask_blocks), by which the line is cut.
   p.part = nullptr;
   p.teams = 0;
-  if (workspace && !pv8 && !(kv_mask && !(kv_len && kv_blocks))) {
+  if (workspace && !fp8 && !(kv_mask && !(kv_len && kv_blocks))) {
     const int teams = split_teams(B, H, Q, kv_cap, resident(D));
     if (teams) {
       SVHIP_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&

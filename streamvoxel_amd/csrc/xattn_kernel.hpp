@@ -1507,30 +1507,28 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
 #endif  // __HIP_DEVICE_COMPILE__
 }
 
-// The split form and its join (defined in xattn_split.hip and xattn_split_wide.hip): the instantiations that
-// launch_dt has for the unsplit one.
+// The split form and its join (defined in xattn_split.hip and xattn_split_wide.hip): the bf16 instantiations
+// that launch_dt has for the unsplit one.
 template <int DT, bool ONES>
-void launch_split(const XattnParams& p, unsigned g, hipStream_t s, bool fp8, bool vt, bool direct);
+void launch_split(const XattnParams& p, unsigned g, hipStream_t s, bool vt, bool direct);
 
 template <int DT, bool ONES>
-void launch_split_impl(const XattnParams& p, unsigned g, hipStream_t s, bool fp8, bool vt, bool direct) {
+void launch_split_impl(const XattnParams& p, unsigned g, hipStream_t s, bool vt, bool direct) {
   constexpr int RS = ONES ? kRegister : kRegisterFull;
   constexpr int DS = ONES ? kDirect : kDirectFull;
   const unsigned n = static_cast<unsigned>(p.teams) * p.q_tiles;
-#define SVHIP_SPLIT(FP8, VT, STAGING, KMASK) \
-  xattn_fwd_kernel<FP8, VT, STAGING, DT, ONES, KMASK, false, false, true><<<n, kThreads, 0, s>>>(p)
+#define SVHIP_SPLIT(VT, STAGING, KMASK) \
+  xattn_fwd_kernel<false, VT, STAGING, DT, ONES, KMASK, false, false, true><<<n, kThreads, 0, s>>>(p)
   if (p.kv_mask) {
     if (direct) {
-      vt ? SVHIP_SPLIT(false, true, DS, true) : SVHIP_SPLIT(false, false, DS, true);
+      vt ? SVHIP_SPLIT(true, DS, true) : SVHIP_SPLIT(false, DS, true);
     } else {
-      vt ? SVHIP_SPLIT(false, true, RS, true) : SVHIP_SPLIT(false, false, RS, true);
+      vt ? SVHIP_SPLIT(true, RS, true) : SVHIP_SPLIT(false, RS, true);
     }
-  } else if (fp8) {
-    vt ? SVHIP_SPLIT(true, true, RS, false) : SVHIP_SPLIT(true, false, RS, false);
   } else if (direct) {
-    vt ? SVHIP_SPLIT(false, true, DS, false) : SVHIP_SPLIT(false, false, DS, false);
+    vt ? SVHIP_SPLIT(true, DS, false) : SVHIP_SPLIT(false, DS, false);
   } else {
-    vt ? SVHIP_SPLIT(false, true, RS, false) : SVHIP_SPLIT(false, false, RS, false);
+    vt ? SVHIP_SPLIT(true, RS, false) : SVHIP_SPLIT(false, RS, false);
   }
 #undef SVHIP_SPLIT
   split_join_kernel<uint16_t><<<split_join_grid(g, p.D), kThreads, 0, s>>>(p);

@@ -4,13 +4,13 @@
 namespace svhip {
 
 template <>
-void launch_split<2, true>(const XattnParams& p, unsigned g, hipStream_t s, bool fp8, bool vt, bool direct) {
-  launch_split_impl<2, true>(p, g, s, fp8, vt, direct);
+void launch_split<2, true>(const XattnParams& p, unsigned g, hipStream_t s, bool vt, bool direct) {
+  launch_split_impl<2, true>(p, g, s, vt, direct);
 }
 
 template <>
-void launch_split<2, false>(const XattnParams& p, unsigned g, hipStream_t s, bool fp8, bool vt, bool direct) {
-  launch_split_impl<2, false>(p, g, s, fp8, vt, direct);
+void launch_split<2, false>(const XattnParams& p, unsigned g, hipStream_t s, bool vt, bool direct) {
+  launch_split_impl<2, false>(p, g, s, vt, direct);
 }
 
 }  // namespace svhip

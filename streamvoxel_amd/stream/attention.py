@@ -96,7 +96,7 @@ def attention(query, key, val, lengths=None, cu_seqlens=None, scale=None, k_scal
     lib = _lib.load()
     # Scratch for the parts of a window whose keys several workgroups share (none where these sizes never split).
     width = kcap if key_mask is None or cu_seqlens is None else key_mask.shape[1]
-    nbytes = int(lib.svhip_xattn_workspace_bytes(B, H, Q, D, width))
+    nbytes = 0 if fp8 else int(lib.svhip_xattn_workspace_bytes(B, H, Q, D, width))
     ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device) if nbytes else None
     if key_mask is not None:
         if fp8:

@@ -6,7 +6,7 @@
     python -m streamvoxel_amd.xattn_trace --sequence [--lib path/libsvhip.so]   # 12 layers back to back
 
 Runs one layer of the 8-window step workload (12 x 64 heads, 1024 queries, L_b = 1552 + 1024 k_b keys, bf16 cache,
-V stored transposed) through the instrumented build of `xattn_fwd_kernel` (csrc/xattn.hip, -DSVHIP_XATTN_TRACE) and
+V stored transposed) through the instrumented build of `xattn_fwd_kernel` (csrc/xattn_kernel.hpp, -DSVHIP_XATTN_TRACE) and
 prints a summary of what the waves did:
 
 * per 32-key half, the median time (s_memtime ticks) of its phases: score product (operand reads, four 32x32x16

@@ -1,4 +1,4 @@
-"""The row-major V operand reads of the cross-attention kernel (csrc/xattn.hip, VROWS), on the CPU: V rows stored
+"""The row-major V operand reads of the cross-attention kernel (csrc/xattn_kernel.hpp, VROWS), on the CPU: V rows stored
 as the kernel stores them (K's sub-tile layout, 16-byte chunk c of row r at chunk swzv(r, c) = c ^ 4 ((r / 2) % 2)),
 the per-lane byte offsets of output tile j (`rvt` in the kernel) and two reads a k-step (keys + 0..3, + 4..7), run
 through the lane layout of ds_read_b64_tr_b16 measured on the GPU (within each 16-lane group lane i receives, as
