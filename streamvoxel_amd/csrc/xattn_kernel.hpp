@@ -777,8 +777,10 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   const int64_t off = p.cu_seqlens ? p.cu_seqlens[b] : 0;
   const int L = [&]() __attribute__((always_inline)) {
     const int n = window_length(p, b);
-    if constexpr (!KMASK || SPLIT) {
+    if constexpr (SPLIT) {
       return __builtin_amdgcn_readfirstlane(n);
+    } else if constexpr (!KMASK) {
+      return n;
     } else {
       // With a key mask the window ends at its last attended key: the blocks after it add nothing to O, l or m.
       // One scan of the window's mask row (a wave-uniform result; no attended key gives L = 0 and zeros).
@@ -955,10 +957,14 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   f32x16_t o[DT];  // O^T tiles: d in [32 j, 32 j + 32)
 #pragma unroll
   for (int j = 0; j < DT; ++j) {
-    float zero = 0.f;
-    if constexpr (SPLIT) asm volatile("" : "+v"(zero));  // no register tuple of zeros kept for the next part
+    if constexpr (SPLIT) {
+      float zero = 0.f;
+      asm volatile("" : "+v"(zero));  // no register tuple of zeros kept for the next part
 #pragma unroll
-    for (int i = 0; i < 16; ++i) o[j][i] = zero;
+      for (int i = 0; i < 16; ++i) o[j][i] = zero;
+    } else {
+      o[j] = f32x16_t{0};
+    }
   }
   float m = -INFINITY;          // stored running max (log2 units), shared by O and l
   float l = 0.f;                // MSUM: query c's row sum in lane c (lanes 32-63 hold 0)
