@@ -21,7 +21,7 @@
 // The split form (SPLIT) is the bf16 kernel's: see key_split.hpp.
 //
 // One window of 12 x 64 heads, 1024 queries, 9744 keys: 816 us on the VALU (one query a lane, K and V rows broadcast from
-// LDS: 37 TFLOP/s), 275 us here (112 TFLOP/s), 7 us of it the join. The instruction alone reaches 141 TFLOP/s with two
+// LDS: 37 TFLOP/s), 286 us here (107 TFLOP/s), 7 us of it the join. The instruction alone reaches 141 TFLOP/s with two
 // waves a SIMD and dependent accumulators, 147 with three.
 //
 // KMASK: a key mask on top of the window length (the reference's `prefix_valid ++ local_valid`): key j of window b
@@ -35,10 +35,14 @@ namespace svhip {
 
 constexpr int kF32Row = 64;      // floats of an LDS row (one key)
 constexpr int kF32Resident = 2;  // workgroups per CU (two waves per SIMD)
-// Key blocks summed into one accumulator before it is added to the total: shorter chains of fp32 sums (one chain of 29
-// blocks is 8.1e-7 from float64 on the single-column configuration, 5.0e-7 with this; 7.3e-7 on the VALU before).
-constexpr int kF32Fold = 8;
-constexpr float kF32Rise = 16.f;
+// Key blocks summed into one accumulator before it is added to the total: short chains of fp32 sums, as the two chains
+// of a score are. From float64, 128 / 400 / 2300 / 9000 keys: 2.6 / 3.0 / 4.0 / 7.0e-7 on the VALU before, 2.2 / 2.3 /
+// 2.6 / 2.8e-7 so; with one chain a score and two blocks 3.1 / 3.4 / 3.5 / 3.8e-7 (8 us faster on the single column),
+// with one chain over all blocks of a range 8.1e-7 there.
+constexpr int kF32Fold = 1;
+// Scores may pass the running max by this much (log2 units) before it is raised. Small: the exponent is rounded at its
+// own size, so weights far above 1 would carry 2^-24 times that size.
+constexpr float kF32Rise = 1.f;
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
@@ -236,6 +240,9 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
         kv_next = key_of(blk + 2);
       }
       if (!KMASK || bits != 0ull) {
+        // The running max taken off the scores. Without a key mask -inf stays: a query whose every score is -inf gets
+        // NaN, as a softmax over them does.
+        auto bias = [&]() __attribute__((always_inline)) { return KMASK && m == -INFINITY ? 0.f : -m; };
         // One weight, formed where it stands in the code: the volatile asm keeps it from sinking to its use.
         auto weight = [&](float& x, float nm, float& sum) __attribute__((always_inline)) {
           x = __builtin_amdgcn_exp2f(__builtin_fmaf(x, sl2, nm));
@@ -246,8 +253,8 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
         auto score = [&](int t, auto under, f32x16_t& w) __attribute__((always_inline)) {
           constexpr bool UNDER = decltype(under)::value;
           constexpr int kSteps = D / 8, kEach = (16 + kSteps - 1) / kSteps;
-          const float nm = UNDER ? (m == -INFINITY ? 0.f : -m) : 0.f;
-          f32x16_t s;
+          const float nm = UNDER ? bias() : 0.f;
+          f32x16_t s, odd;  // the even and the odd steps' products: two chains half as long
           float sum = 0.f;
           const float* kr = sK + (32 * t + col) * kF32Row;
           f32x4_t x = *reinterpret_cast<const f32x4_t*>(kr + 4 * f32_swz_k(col, hh));
@@ -257,7 +264,8 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
             if (c + 1 < kSteps) next = *reinterpret_cast<const f32x4_t*>(kr + 4 * f32_swz_k(col, 2 * (c + 1) + hh));
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              s = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], qf[4 * c + e], c + e == 0 ? f32x16_t{0} : s, 0, 0, 0);
+              f32x16_t& acc = e % 2 == 0 ? s : odd;
+              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], qf[4 * c + e], c + e / 2 == 0 ? f32x16_t{0} : acc, 0, 0, 0);
             }
             x = next;
             if constexpr (UNDER) {
@@ -271,6 +279,8 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
             __builtin_amdgcn_sched_barrier(0);
           }
           if constexpr (UNDER) l += sum;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[i] += odd[i];
           return s;
         };
         // The half's largest score, keys not attended put to -inf.
@@ -313,7 +323,7 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
         // O^T += V^T . P^T of half t, the weights of `w` (UNDER) between its products.
         auto pv = [&](const f32x16_t& s, int t, auto under, f32x16_t& w) __attribute__((always_inline)) {
           constexpr bool UNDER = decltype(under)::value;
-          const float nm = UNDER ? (m == -INFINITY ? 0.f : -m) : 0.f;
+          const float nm = UNDER ? bias() : 0.f;
           float sum = 0.f;
           // Entry i is key 32 t + 8 (i / 4) + 4 hh + i % 4; f32_swz_v on floats: bit 5 of the row's float index flips
           // with bit 2 of the key, which is hh.

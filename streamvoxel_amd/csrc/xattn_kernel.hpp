@@ -745,10 +745,13 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   do {
   // SPLIT: the thread index is opaque in every part of the range, or the compiler would form the addresses of the
   // parts' beginning and end once, outside this loop, and hold them in registers through the key blocks (88 spilled).
-  int tid = threadIdx.x;
-  if constexpr (SPLIT) asm volatile("" : "+v"(tid));
-  const int lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // (Elsewhere threadIdx.x itself, whose known range a variable that the lambdas capture does not carry: ten more
+  // instructions a block in the register-staged forms.)
+  [[maybe_unused]] int part_tid = threadIdx.x;
+  if constexpr (SPLIT) asm volatile("" : "+v"(part_tid));
+#define SVHIP_TID (SPLIT ? part_tid : static_cast<int>(threadIdx.x))
+  const int lane = SVHIP_TID & 63;
+  const int w = __builtin_amdgcn_readfirstlane(SVHIP_TID >> 6);
   const int col = lane & 31;  // query column within the wave
   const int hh = lane >> 5;   // lane half
   const int64_t q = static_cast<int64_t>(qt) * kQTile + w * 32 + col;
@@ -769,7 +772,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     blk0 = rel - hw * unit_blocks;
     blk1 = min(unit_blocks, blk0 + (range_end - pos));
     pos += blk1 - blk0;
-    if (blk0 == 0 && qt == 0 && tid == 0) {
+    if (blk0 == 0 && qt == 0 && SVHIP_TID == 0) {
       split_units(p)[b * p.H + h] =
           split_unit_teams(team, pos - blk1, unit_blocks, blk1 == unit_blocks, s_total, s_teams);
     }
@@ -785,7 +788,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
       // With a key mask the window ends at its last attended key: the blocks after it add nothing to O, l or m.
       // One scan of the window's mask row (a wave-uniform result; no attended key gives L = 0 and zeros).
       __shared__ int s_last;
-      if (tid == 0) s_last = -1;
+      if (SVHIP_TID == 0) s_last = -1;
       __syncthreads();
       const int last = last_attended(p.kv_mask + b * p.sm_b, n);
       if (last >= 0) atomicMax(&s_last, last);
@@ -855,7 +858,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     if (STAGING == kDirect && dchunks < 4 * DT) {
       // Chunks past head_dim of the K tiles that the score product reads are never loaded by direct loads; they
       // must hold zeros.
-      for (int i = tid; i < kSubTiles * kKB * 8; i += kThreads) {
+      for (int i = SVHIP_TID; i < kSubTiles * kKB * 8; i += kThreads) {
         const int u = i / (kKB * 8), R = (i >> 3) % kKB, c = i & 7;
         if (8 * u + c >= dchunks) {
           const int e = u * kKTile + R * kRow + swz(R, c) * 8;
@@ -867,7 +870,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     if constexpr (VROWS) {
       // Direct loads never write the chunks of V rows past head_dim: zeros, and with ONES the ones column D.
       if (dchunks < 8 * kSubTiles) {
-        for (int i = tid; i < kSubTiles * kKB * 8; i += kThreads) {
+        for (int i = SVHIP_TID; i < kSubTiles * kKB * 8; i += kThreads) {
           const int u = i / (kKB * 8), R = (i >> 3) % kKB, c = i & 7;
           if (8 * u + c >= dchunks) {
             const int e = u * kKTile + R * kRow + swzv(R, c) * 8;
@@ -877,10 +880,10 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
           }
         }
       }
-    } else if (ONES && tid < 16) {
+    } else if (ONES && SVHIP_TID < 16) {
       // Direct loads never write V^T rows >= D: row D of both buffers holds ones for the whole kernel.
-      const int R = static_cast<int>(p.D), c = tid & 7;
-      uint16_t* buf = tid < 8 ? sV0 : sV1;
+      const int R = static_cast<int>(p.D), c = SVHIP_TID & 7;
+      uint16_t* buf = SVHIP_TID < 8 ? sV0 : sV1;
       *reinterpret_cast<uint4*>(buf + R * kRow + swz(R, c) * 8) = raw_one<false>();
     }
   }
@@ -893,7 +896,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   if constexpr (VD8) {
     dv = direct_v8<DT>(p, reinterpret_cast<const uint8_t*>(V), nfull, w);
     // V^T rows D .. 32 DT - 1 of both tiles, which direct loads never write: zeros (row D ones with ONES).
-    for (int i = tid; i < (32 * DT - Dv) * 4; i += kThreads) {
+    for (int i = SVHIP_TID; i < (32 * DT - Dv) * 4; i += kThreads) {
       const int R = Dv + (i >> 2), c = i & 3;
       const uint32_t x = (ONES && R == Dv) ? 0x38383838u : 0u;  // e4m3 1.0
       *reinterpret_cast<uint4*>(reinterpret_cast<uint8_t*>(sV0) + R * kRow8 + c * 16) = make_uint4(x, x, x, x);
@@ -983,7 +986,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
                                                    static_cast<uint32_t>(kv0 * 2), w, sK, sV);
       if constexpr (VROWS) stage_rows<DT, STAGING == kDirectFull>(dr, static_cast<uint32_t>(kv0 * p.sv_k * 2), w, sV);
     } else {
-      stage_load<FP8, VT, DT, false, ONES, !VD8>(st, p, K, V, L, kv0, dchunks, vt_vec, tid);
+      stage_load<FP8, VT, DT, false, ONES, !VD8>(st, p, K, V, L, kv0, dchunks, vt_vec, SVHIP_TID);
       if constexpr (VD8) {
 #pragma unroll
         for (int t = 0; t < (2 * DT + 3) / 4; ++t) {
@@ -994,13 +997,13 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     }
   };
   auto stage_commit = [&](uint16_t* sK, uint16_t* sV) __attribute__((always_inline)) {
-    if constexpr (!DIRECT) stage_store<FP8, VT, DT, ONES, PV8, !VD8>(st, sK, sV, dchunks, Dv, tid);
+    if constexpr (!DIRECT) stage_store<FP8, VT, DT, ONES, PV8, !VD8>(st, sK, sV, dchunks, Dv, SVHIP_TID);
   };
   // The partial block, synchronously through registers.
   auto stage_tail = [&](uint16_t* sK, uint16_t* sV) __attribute__((always_inline)) {
     Stage<FP8, VT, DT> tmp;
-    stage_load<FP8, VT, DT, true, ONES>(tmp, p, K, V, L, nfull * kKB, dchunks, vt_vec, tid);
-    stage_store<FP8, VT, DT, ONES, PV8>(tmp, sK, sV, dchunks, Dv, tid);
+    stage_load<FP8, VT, DT, true, ONES>(tmp, p, K, V, L, nfull * kKB, dchunks, vt_vec, SVHIP_TID);
+    stage_store<FP8, VT, DT, ONES, PV8>(tmp, sK, sV, dchunks, Dv, SVHIP_TID);
   };
 
 
@@ -1417,11 +1420,11 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
       const int kv0 = LIST ? kv_cur : blk * kKB;
       const uint64_t bits = block_bits(LIST ? kv_next : kv0 + kKB);
       Stage<FP8, VT, DT> tl;
-      if (tail) stage_load<FP8, VT, DT, true, ONES>(tl, p, K, V, L, nfull * kKB, dchunks, vt_vec, tid);
+      if (tail) stage_load<FP8, VT, DT, true, ONES>(tl, p, K, V, L, nfull * kKB, dchunks, vt_vec, SVHIP_TID);
       compute(Full{}, cK, cV, kv0, bits);
       settle();
       if (tail) {
-        stage_store<FP8, VT, DT, ONES, PV8>(tl, nK, nV, dchunks, Dv, tid);
+        stage_store<FP8, VT, DT, ONES, PV8>(tl, nK, nV, dchunks, Dv, SVHIP_TID);
         wait_vmem();
         __syncthreads();
         compute(Partial{}, nK, nV, nfull * kKB, block_bits(L));
@@ -1510,6 +1513,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   }
   if constexpr (SPLIT) __syncthreads();  // the next part stages into the tiles
   } while (SPLIT && pos < range_end);
+#undef SVHIP_TID
 #endif  // __HIP_DEVICE_COMPILE__
 }
 

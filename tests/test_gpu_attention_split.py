@@ -185,3 +185,24 @@ def test_mask_blocks_against_torch(dev, cap):
             assert int(out[b]) == (int(at[-1]) + 1 if len(at) else 0)
             assert blocks[b, 0] == len(want) and blocks[b, 1:1 + len(want)].tolist() == want
             assert (blocks[b, 1 + len(want):] == -7).all()
+
+
+@pytest.mark.parametrize('L', [40, 5000])
+def test_fp32_rows_of_infinite_scores(dev, L):
+    """A query whose every score is -inf, or that meets +inf, gets NaN without a key mask, as torch's softmax gives;
+    the other queries of its tile are untouched (unsplit and split lengths)."""
+    from streamvoxel_amd.stream.attention import attention
+    B, H, Q, D = 1, 2, 70, 64
+    _case(f'fp32 infinite scores L={L}')
+    q, k, v = qkv(B, H, Q, L, D, L, torch.float32)
+    k[..., 0] = k[..., 0].abs() + 0.1
+    clean = q.clone()
+    q[0, 0, 3, 0], q[0, 1, 69, 0] = -math.inf, math.inf
+    lt = torch.tensor([L], dtype=torch.int32, device=dev)
+    out = attention(q.to(dev), k.to(dev), v.to(dev), lengths=lt).cpu()
+    want = attention(clean.to(dev), k.to(dev), v.to(dev), lengths=lt).cpu()
+    bad = torch.zeros(B, H, Q, dtype=torch.bool)
+    bad[0, 0, 3] = bad[0, 1, 69] = True
+    assert out[bad].isnan().all()
+    # An infinite score may raise the running max of the wave it is in, never another query's.
+    assert torch.allclose(out[~bad], want[~bad], rtol=1e-5, atol=1e-6)
