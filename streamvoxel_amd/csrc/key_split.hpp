@@ -49,8 +49,8 @@ __device__ __forceinline__ int window_length(const P& p, int64_t b) {
 // XCD, so its L2 still serves a block to all of them. The grid is what the chip holds at once, so every CU has the
 // same count of key blocks to do. A range that holds a unit whole writes its output; a part of a unit leaves O, its
 // running max and its row sum in fp32, in the team's slot 0 (the range starts inside the unit) or 1 (it only ends
-// inside it), and split_join_kernel joins the parts. Where a unit is cut depends on all windows' lengths, and the last bits
-// of its result with it (one rounding of P against another running max).
+// inside it), and split_join_kernel joins the parts. Where a unit is cut depends on all windows' lengths, and the last
+// bits of its result with it (one rounding of P against another running max).
 // The lengths are on the device, so every workgroup forms the plan for itself: lane b holds window b's block count.
 struct SplitPlan {
   int before, blocks;  // of lane b: blocks of one head in the windows before b, and in b

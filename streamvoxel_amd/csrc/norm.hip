@@ -70,7 +70,8 @@ struct NormArgs {
 // gate is set). VEC: gate / shift / scale rows take 16-byte loads.
 // A launch is one short chain per row (load, two reductions, store) with four waves a SIMD and nothing behind it, so
 // its loads go out together at the start (AHEAD): branch, gate, shift and scale read after one another, each behind the
-// step before, took 10.2 us for 8 x 1024 rows of 768 with branch, gate and modulation, 9.0 us now (5.6 TB/s). Rows of more than four chunks a lane would not have the registers.
+// step before, took 10.2 us for 8 x 1024 rows of 768 with branch, gate and modulation, 9.0 us now (5.6 TB/s). Rows of
+// more than four chunks a lane would not have the registers.
 template <int LPR, int CH, bool RES, bool VEC>
 __global__ __launch_bounds__(kNormThreads) void layer_norm_kernel(NormArgs a) {
   constexpr int kRowsPerBlock = kNormThreads / LPR;

@@ -265,7 +265,8 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               f32x16_t& acc = e % 2 == 0 ? s : odd;
-              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], qf[4 * c + e], c + e / 2 == 0 ? f32x16_t{0} : acc, 0, 0, 0);
+              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], qf[4 * c + e], c + e / 2 == 0 ? f32x16_t{0} : acc, 0, 0,
+                                                         0);
             }
             x = next;
             if constexpr (UNDER) {
@@ -441,7 +442,8 @@ static void launch_f32(const XattnF32Params& p, unsigned grid, hipStream_t s, bo
 using namespace svhip;
 
 static int xattn_f32_impl(const float* q, const float* k, const float* v, float* o, const uint8_t* kv_mask,
-                          int64_t sm_b, const int32_t* kv_blocks, int64_t sb_b, const int32_t* kv_len, const int32_t* cu_seqlens, int64_t B, int64_t H,
+                          int64_t sm_b, const int32_t* kv_blocks, int64_t sb_b, const int32_t* kv_len,
+                          const int32_t* cu_seqlens, int64_t B, int64_t H,
                           int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q,
                           int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k,
                           int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* workspace,
