@@ -131,7 +131,9 @@ __device__ __forceinline__ int2 split_unit_teams(int team, int first, int unit_b
 }
 
 // Joins the parts of the units that the split kernel cut: O = sum_i w_i O_i, l = sum_i w_i l_i with w_i =
-// exp2(m_i - max m) over the parts in key order, then v_scale O / l in the output's type. Workgroup = (unit, query
+// exp2(m_i - max m) over the parts in key order, then v_scale O / l in the output's type. A part's l is 0 without an
+// attended key (only a key mask makes such parts), and also where the query is NaN (the weights' clamp turns NaN to 0):
+// only under a key mask is it taken for nothing, so that a NaN query ends in 0 / 0 as in the unsplit form. Workgroup = (unit, query
 // tile, kJoinQueries queries, kJoinDims head_dim elements), a thread 4 elements of one query. The parts are read once,
 // from the last-level cache where they were just written: a short chain of loads, so the workgroups are many and a
 // thread has kJoinAhead parts in flight (one window of 12 heads, nine parts a unit: 10.7 us with four queries a thread
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(kThreads) void split_join_kernel(P p) {
   const int u = static_cast<int>(blockIdx.x / p.q_tiles), qt = static_cast<int>(blockIdx.x % p.q_tiles);
   const int H = static_cast<int>(p.H);
   const int64_t b = u / H, h = u % H;
-  const bool empty = window_length(p, b) == 0;
+  const bool empty = window_length(p, b) == 0, masked = p.kv_mask != nullptr;
   const int2 teams = split_units(p)[u];  // (left as it was for an empty window)
   const int t0 = empty ? 0 : teams.x, t1 = empty ? -1 : teams.y;
   if (!empty && t1 < t0) return;  // one range holds the unit: its output is written
@@ -177,7 +179,7 @@ __global__ __launch_bounds__(kThreads) void split_join_kernel(P p) {
 #pragma unroll
     for (int a = 0; a < kJoinAhead; ++a) {
       if (t + a > t1) break;
-      if (li[a] == 0.f) continue;  // a part without an attended key
+      if (masked && li[a] == 0.f) continue;  // a part without an attended key
       const float mn = fmaxf(m, mi[a]);
       const float x = __builtin_amdgcn_exp2f(m - mn), y = __builtin_amdgcn_exp2f(mi[a] - mn);
       m = mn;
@@ -186,7 +188,7 @@ __global__ __launch_bounds__(kThreads) void split_join_kernel(P p) {
     }
   }
   T* out = static_cast<T*>(p.o) + b * p.so_b + h * p.so_h + q * p.so_q + d0;
-  const float inv = l == 0.f ? 0.f : (p.v_scale ? p.v_scale[b * p.H + h] : 1.f) / l;
+  const float inv = empty || (masked && l == 0.f) ? 0.f : (p.v_scale ? p.v_scale[b * p.H + h] : 1.f) / l;
   if constexpr (sizeof(T) == 4) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) out[e] = o[e] * inv;  // rows of any alignment

@@ -206,3 +206,33 @@ def test_fp32_rows_of_infinite_scores(dev, L):
     assert out[bad].isnan().all()
     # An infinite score may raise the running max of the wave it is in, never another query's.
     assert torch.allclose(out[~bad], want[~bad], rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize('D', [48, 64, 96])
+@pytest.mark.parametrize('lengths', [[700], [6000], [5000, 40, 4000, 1600]], ids=lambda x: '-'.join(map(str, x)))
+def test_nan_queries_stay_nan(dev, D, lengths):
+    """A NaN query gives NaN rows, whether its window is attended whole or in parts; the queries of other waves (32
+    queries each) keep their bits, the ones of the same wave may see their running max raised (the tile's bars). At
+    head_dim 96 the row sums of queries c and c + 16 of a wave share an operand column, so query 21 is left out."""
+    from streamvoxel_amd.stream.attention import attention
+    B, H, Q, kcap = len(lengths), 2, 200, max(lengths) + 8
+    _case(f'NaN queries D={D} lengths={lengths}')
+    q, k, v = qkv(B, H, Q, kcap, D, D + B, torch.bfloat16)
+    bad = torch.zeros(B, H, Q, dtype=torch.bool)
+    bad[0, 1, 5] = bad[B - 1, 0, 199] = True
+    qn = q.clone()
+    qn[0, 1, 5] = math.nan
+    qn[B - 1, 0, 199, 3] = math.nan
+    lt = torch.tensor(lengths, dtype=torch.int32, device=dev)
+    kd, vd = k.to(dev), v.to(dev)
+    vt = vd.transpose(2, 3).contiguous().transpose(2, 3)
+    same_wave = torch.zeros_like(bad)
+    same_wave[0, 1, :32] = same_wave[B - 1, 0, 192:] = True
+    for val in (vd, vt):
+        want = attention(q.to(dev), kd, val, lengths=lt).cpu()
+        got = attention(qn.to(dev), kd, val, lengths=lt).cpu()
+        assert got[bad].isnan().all()
+        assert torch.equal(got[~same_wave], want[~same_wave])
+        near = same_wave & ~bad
+        near[0, 1, 21] = False
+        assert (got[near].float() - want[near].float()).abs().max() <= 2e-2
