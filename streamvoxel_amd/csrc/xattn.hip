@@ -331,9 +331,10 @@ extern "C" int svhip_xattn_fwd_ws(const void* q, const void* k, const void* v, v
   const char* name = "svhip_xattn_fwd";
   clear_error();
   SVHIP_REQUIRE(kv_len || cu_seqlens, "%s: need kv_len or cu_seqlens", name);
-  return xattn_impl(q, k, v, o, kv_dtype, kv_len, cu_seqlens, k_scale, v_scale, nullptr, 0, nullptr, 0, B, H, Q, D, kv_cap, sq_b,
-                    sq_h, sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, workspace,
-                    workspace_bytes, stream, name);
+  if (cu_seqlens) kv_len = nullptr;  // the packed lengths alone hold
+  return xattn_impl(q, k, v, o, kv_dtype, kv_len, cu_seqlens, k_scale, v_scale, nullptr, 0, nullptr, 0, B, H, Q, D,
+                    kv_cap, sq_b, sq_h, sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale,
+                    workspace, workspace_bytes, stream, name);
 }
 
 extern "C" int svhip_xattn_fwd_masked(const void* q, const void* k, const void* v, void* o, const uint8_t* kv_mask,

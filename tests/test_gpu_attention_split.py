@@ -236,3 +236,36 @@ def test_nan_queries_stay_nan(dev, D, lengths):
         near = same_wave & ~bad
         near[0, 1, 21] = False
         assert (got[near].float() - want[near].float()).abs().max() <= 2e-2
+
+
+@pytest.mark.parametrize('workspace', [False, True])
+def test_packed_lengths_win_over_kv_len(dev, workspace):
+    """svhip_xattn_fwd and _ws given both kv_len and cu_seqlens: the packed lengths hold, kv_len is not read."""
+    from streamvoxel_amd import _lib
+    from streamvoxel_amd.stream.attention import attention
+    lengths, H, Q, D = [2000, 500], 2, 130, 64
+    _case(f'packed with kv_len workspace={workspace}')
+    total = sum(lengths)
+    q, k, v = (x.to(dev) for x in qkv(2, H, Q, total, D, 5, torch.bfloat16))
+    kp, vp = k[0].contiguous(), v[0].contiguous()
+    cu = torch.tensor([0, lengths[0], total], dtype=torch.int32, device=dev)
+    lib = _lib.load()
+    nbytes = int(lib.svhip_xattn_workspace_bytes(2, H, Q, D, total))
+    assert nbytes > 0
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if workspace else None
+    outs = []
+    for kv_len in (None, torch.tensor([100, 7], dtype=torch.int32, device=dev)):
+        out = torch.zeros_like(q)
+        args = [_lib.ptr(q), _lib.ptr(kp), _lib.ptr(vp), _lib.ptr(out), _lib.SVHIP_BF16, _lib.ptr(kv_len), _lib.ptr(cu),
+                None, None, 2, H, Q, D, total, *q.stride()[:3], 0, *kp.stride()[:2], 0, *vp.stride(), *out.stride()[:3],
+                1.0 / math.sqrt(D)]
+        if workspace:
+            rc = lib.svhip_xattn_fwd_ws(*args, _lib.ptr(ws), nbytes, _lib.stream_of(q))
+        else:
+            rc = lib.svhip_xattn_fwd(*args, _lib.stream_of(q))
+        _lib.check(rc, 'svhip_xattn_fwd')
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
+    if workspace:
+        assert torch.equal(outs[0], attention(q, kp, vp, cu_seqlens=cu))
