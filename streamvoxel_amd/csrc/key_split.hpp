@@ -152,7 +152,8 @@ __global__ __launch_bounds__(kThreads) void split_join_kernel(P p) {
   const int u = static_cast<int>(blockIdx.x / p.q_tiles), qt = static_cast<int>(blockIdx.x % p.q_tiles);
   const int H = static_cast<int>(p.H);
   const int64_t b = u / H, h = u % H;
-  const bool empty = window_length(p, b) == 0, masked = p.kv_mask != nullptr;
+  // (The plan's own count: a window without blocks has no part on the line and left no teams.)
+  const bool empty = (p.kv_blocks ? p.kv_blocks[b * p.sb_b] : window_length(p, b)) == 0, masked = p.kv_mask != nullptr;
   const int2 teams = split_units(p)[u];  // (left as it was for an empty window)
   const int t0 = empty ? 0 : teams.x, t1 = empty ? -1 : teams.y;
   if (!empty && t1 < t0) return;  // one range holds the unit: its output is written

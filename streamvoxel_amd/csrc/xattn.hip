@@ -109,6 +109,8 @@ static int xattn_impl(const void* q, const void* k, const void* v, void* o, int 
                       (sv_h * eb) % align == 0 && (sv_b * eb) % align == 0,
                   "%s: V rows must be %d-byte aligned", name, (int)align);
   }
+  SVHIP_REQUIRE(!(kv_mask && kv_len && kv_blocks) || B <= 1 || sb_b > cdiv(kv_cap, kKB),
+                "%s: block rows shorter than the windows' lists", name);
   if (B == 0 || Q == 0) return SVHIP_OK;
   SVHIP_REQUIRE(kv_cap >= 0 && kv_cap < (1ll << 31), "%s: kv_cap out of range", name);
   XattnParams p;

@@ -455,7 +455,9 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   } else {
     SVHIP_REQUIRE(kv_len || cu_seqlens, "%s: need kv_len or cu_seqlens", name);
   }
-  SVHIP_REQUIRE(!(kv_len && cu_seqlens) || kv_blocks, "%s: kv_len and cu_seqlens are exclusive", name);
+  // With lists of attended blocks kv_len may come with cu_seqlens (svhip_mask_blocks gives both).
+  const bool listed = kv_mask && kv_len && kv_blocks;
+  SVHIP_REQUIRE(!(kv_len && cu_seqlens) || listed, "%s: kv_len and cu_seqlens are exclusive", name);
   SVHIP_REQUIRE(B >= 0 && H >= 1 && Q >= 0, "%s: bad sizes", name);
   SVHIP_REQUIRE(D == 16 || D == 32 || D == 48 || D == 64, "%s: head_dim %lld unsupported (16, 32, 48 or 64)", name,
                 (long long)D);
@@ -470,6 +472,7 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   SVHIP_REQUIRE(reinterpret_cast<uintptr_t>(v) % 16 == 0 && (vt ? sv_d : sv_k) % 4 == 0 && sv_h % 4 == 0 &&
                     sv_b % 4 == 0,
                 "%s: V rows must be 16-byte aligned", name);
+  SVHIP_REQUIRE(!listed || B <= 1 || sb_b > cdiv(kv_cap, kKB), "%s: block rows shorter than the windows' lists", name);
   if (B == 0 || Q == 0) return SVHIP_OK;
   XattnF32Params p;
   p.q = q;
@@ -509,7 +512,7 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   p.teams = 0;
   // Several windows with a key mask need their lists of attended blocks (svhip_mask_blocks), by which the line is cut; a
   // single one is cut by its capacity.
-  if (workspace && !(kv_mask && B > 1 && !(kv_len && kv_blocks))) {
+  if (workspace && !(kv_mask && B > 1 && !listed)) {
     const int teams = split_teams(B, H, Q, kv_cap, kF32Resident);
     const size_t need = split_workspace_bytes(B, H, Q, D, kv_cap, kF32Resident);
     if (teams) {
@@ -517,7 +520,7 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
                     "%s: workspace too small or unaligned (%zu < %zu bytes)", name, workspace_bytes, need);
       p.part = static_cast<float*>(workspace);
       p.teams = teams;
-      if (kv_mask) {
+      if (listed) {
         p.kv_blocks = kv_blocks;
         p.sb_b = sb_b;
       }

@@ -58,6 +58,29 @@ def test_workspace_queries_and_argument_errors(lib):
     assert rc == -1
 
 
+def test_masked_attention_checks_the_block_lists_on_the_host(lib):
+    """Rows of kv_blocks that are shorter than a window's list are refused (kv_cap 130: 3 blocks and the count, so rows
+    at least 4 apart), and fp32 takes kv_len with cu_seqlens only beside a mask and its lists. No query (Q = 0), so
+    an accepted call launches nothing."""
+    p = ctypes.c_void_p(4096)                    # aligned, never read
+    strides = [64] * 6 + [64, 64, 64, 1] + [64] * 3     # of q, k, v (rows) and o
+    sizes = [2, 1, 0, 64, 130]
+
+    def bf16(sb, lengths=p, cu=None):
+        return lib.svhip_xattn_fwd_masked_ws(p, p, p, p, p, 130, lengths, p, sb, cu, *sizes, *strides, 0.125, None, 0,
+                                             None)
+
+    def fp32(sb, mask=p, lengths=p, blocks=p, cu=None):
+        return lib.svhip_xattn_fwd_f32_ws(p, p, p, p, mask, 130, lengths, blocks, sb, cu, *sizes, *strides, 0.125, None,
+                                          0, None)
+    for call in (bf16, fp32):
+        assert call(4) == 0 and call(4, cu=p) == 0
+        assert call(3) == -1 and b'lists' in lib.svhip_last_error()
+        assert call(3, lengths=None) == 0        # lists without their lengths are not used
+    assert fp32(4, mask=None, cu=p) == -1 and b'exclusive' in lib.svhip_last_error()
+    assert fp32(4, blocks=None, cu=p) == -1 and b'exclusive' in lib.svhip_last_error()
+
+
 def test_noalloc_select_rejects_on_the_host(lib):
     # 200 windows of 65 536 voxels need about 104 MiB of scratch, more than the library's fixed 48 MiB array
     assert lib.svhip_ease_select_workspace_bytes(200, 256, 16, 16, 4) > (48 << 20)

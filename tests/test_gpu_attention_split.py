@@ -269,3 +269,28 @@ def test_packed_lengths_win_over_kv_len(dev, workspace):
     assert torch.equal(outs[0], outs[1])
     if workspace:
         assert torch.equal(outs[0], attention(q, kp, vp, cu_seqlens=cu))
+
+
+@pytest.mark.parametrize('lengths', [False, True])
+def test_fp32_fully_masked_window_with_a_list(dev, lengths):
+    """One fp32 window without an attended key, its list of blocks given with and without its length: zeros, whatever
+    the scratch holds (zeros where an entry could be taken for a team or a slot, ones elsewhere)."""
+    from streamvoxel_amd import _lib
+    H, Q, D, kcap = 2, 130, 64, 4000
+    _case(f'fp32 empty list lengths={lengths}')
+    q, k, v = (x.to(dev) for x in qkv(1, H, Q, kcap, D, 1, torch.float32))
+    mask = torch.zeros(1, kcap, dtype=torch.uint8, device=dev)
+    cut = torch.zeros(1, dtype=torch.int32, device=dev)
+    blocks = torch.zeros(1, 1 + (kcap + 63) // 64, dtype=torch.int32, device=dev)
+    lib = _lib.load()
+    nbytes = int(lib.svhip_xattn_f32_workspace_bytes(1, H, Q, D, kcap))
+    assert nbytes > 0
+    ws = torch.ones(nbytes // 4, dtype=torch.float32, device=dev)
+    ws[-2 * H:] = 0
+    out = torch.full_like(q, 7.0)
+    _lib.check(lib.svhip_xattn_fwd_f32_ws(
+        _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(mask), kcap, _lib.ptr(cut) if lengths else None,
+        _lib.ptr(blocks), blocks.stride(0), None, 1, H, Q, D, kcap, *q.stride()[:3], *k.stride()[:3], *v.stride(),
+        *out.stride()[:3], 0.125, _lib.ptr(ws), nbytes, _lib.stream_of(q)), 'svhip_xattn_fwd_f32_ws')
+    torch.cuda.synchronize()
+    assert not out.any()
