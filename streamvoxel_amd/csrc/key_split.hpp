@@ -24,6 +24,10 @@ constexpr int kSplitMinBlocks = 24;
 constexpr int kSplitMinRange = 6;
 constexpr int kSplitMaxRounds = 4;
 constexpr int kSplitFullPercent = 85;
+// Running max that a part without the unit's first keys starts from, without a key mask: finite, so that keys whose
+// scores are all -inf weigh nothing until a finite score raises it, as they do further inside a walk (from -inf their
+// weights would be exp2(-inf + inf), NaN). The unit's first keys keep -inf: a query without any finite score is NaN.
+constexpr float kPartMax = -3.0e38f;
 
 // Keys of window b.
 template <typename P>

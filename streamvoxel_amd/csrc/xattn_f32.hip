@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
     f32x16_t o[kTiles], total[kTiles];  // O^T of the last blocks, and of those before
 #pragma unroll
     for (int j = 0; j < kTiles; ++j) o[j] = total[j] = f32x16_t{0};
-    float m = -INFINITY, l = 0.f;  // l: the lane's own keys
+    float m = SPLIT && !KMASK && blk0 > 0 ? kPartMax : -INFINITY, l = 0.f;  // l: the lane's own keys
 
     // Block loads: chunk c = thread + 256 r is key c / kChunks, head_dim 4 (c % kChunks) .. + 3 (of V^T key c % 64,
     // head_dim 4 (c / 64) .. + 3: consecutive lanes read consecutive keys of a row). Every load is issued
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
           }
         }
         if (hh == 0) {
-          slot[kQTile * D + ql] = l == 0.f ? -INFINITY : m;
+          slot[kQTile * D + ql] = KMASK && l == 0.f ? -INFINITY : m;
           slot[kQTile * (D + 1) + ql] = l;
         }
         continue;

@@ -969,7 +969,8 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
       o[j] = f32x16_t{0};
     }
   }
-  float m = -INFINITY;          // stored running max (log2 units), shared by O and l
+  // Stored running max (log2 units), shared by O and l.
+  float m = SPLIT && !KMASK && blk0 > 0 ? kPartMax : -INFINITY;
   float l = 0.f;                // MSUM: query c's row sum in lane c (lanes 32-63 hold 0)
   bool first = true;            // uniform: the window's first half always takes the max
   // KMASK: the lane's query has seen no attended key yet (m is then a placeholder 0, O and l are 0); every half
@@ -1464,8 +1465,8 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   SVHIP_TRACE(trace.end(lane, lsum);)
   if constexpr (SPLIT) {
     if (blk1 - blk0 < unit_blocks) {
-      // A part of the unit: O as it stands, [head_dim / 4][query][4], then m and l, [2][query]; a query that has
-      // seen no attended key (l = 0) carries m = -inf.
+      // A part of the unit: O as it stands, [head_dim / 4][query][4], then m and l, [2][query]; under a key
+      // mask a query that has seen no attended key (l = 0) carries m = -inf.
       float* slot = p.part + (static_cast<int64_t>(2 * team + (blk0 == 0 ? 1 : 0)) * p.q_tiles + qt) *
                                  split_slot_floats(p.D);
       const int ql = w * 32 + col;
@@ -1480,7 +1481,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
         }
       }
       if (hh == 0) {
-        slot[kQTile * p.D + ql] = lsum == 0.f ? -INFINITY : m;
+        slot[kQTile * p.D + ql] = KMASK && lsum == 0.f ? -INFINITY : m;
         slot[kQTile * (p.D + 1) + ql] = lsum;
       }
       __syncthreads();  // the next part stages into the tiles

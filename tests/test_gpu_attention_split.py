@@ -294,3 +294,27 @@ def test_fp32_fully_masked_window_with_a_list(dev, lengths):
         *out.stride()[:3], 0.125, _lib.ptr(ws), nbytes, _lib.stream_of(q)), 'svhip_xattn_fwd_f32_ws')
     torch.cuda.synchronize()
     assert not out.any()
+
+
+@pytest.mark.parametrize('dtype,D', [('bf16', 48), ('bf16', 64), ('bf16', 96), ('bf16', 128), ('fp32', 48), ('fp32', 64)])
+@pytest.mark.parametrize('lengths', [[6000], [6000, 2000, 4096]], ids=lambda x: '-'.join(map(str, x)))
+def test_stretch_of_minus_infinite_scores(dev, dtype, D, lengths):
+    """Queries whose scores are -inf (by overflow of the score product) over most of the window, from its second block
+    to its last but one: those keys weigh nothing, wherever the window is cut, and the rows stay finite."""
+    from streamvoxel_amd.stream.attention import attention
+    dt = torch.bfloat16 if dtype == 'bf16' else torch.float32
+    B, H, Q, kcap = len(lengths), 2, 140, max(lengths)
+    _case(f'-inf stretch {dtype} D={D} lengths={lengths}')
+    q, k, v = qkv(B, H, Q, kcap, D, D, torch.float32)
+    q[..., 0], k[..., 0] = 0.0, 0.0
+    bad = torch.zeros(B, H, Q, dtype=torch.bool)
+    bad[:, :, ::7] = True
+    q[..., 0][bad] = 3e38
+    for b, n in enumerate(lengths):
+        k[b, :, 64:n - 100, 0] = -3e38
+    q, k, v = (x.to(dt) for x in (q, k, v))
+    ref = A.cross_attention(q, k, v, lengths)
+    out = attention(q.to(dev), k.to(dev), v.to(dev), lengths=torch.tensor(lengths, dtype=torch.int32, device=dev))
+    torch.cuda.synchronize()
+    assert bool(out.isfinite().all())
+    check(out, ref, *((2e-2, 1e-2) if dtype == 'bf16' else (2e-5, 1e-4)))
