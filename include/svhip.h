@@ -189,7 +189,8 @@ int svhip_xattn_fwd(const void* q, const void* k, const void* v, void* o, int kv
  * (few windows, or windows of different lengths, otherwise leave part of the chip idle): 16-byte aligned, at least
  * svhip_xattn_workspace_bytes(B, H, Q, D, kv_cap) bytes, its content of no meaning before or after the call. The
  * query returns 0 where these sizes are never split; a NULL workspace and an e4m3 cache never split. The parts are
- * joined in fp32; where a window's keys are cut depends on all windows' lengths, so the last bits of its result do too.
+ * joined in fp32. Where a window's keys are cut depends on its own length and on H and Q alone, with and without scratch
+ * memory: a window gives the same bits alone, in any batch and through either call.
  */
 size_t svhip_xattn_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap);
 int svhip_xattn_fwd_ws(const void* q, const void* k, const void* v, void* o, int kv_dtype, const int32_t* kv_len,
@@ -277,7 +278,8 @@ int svhip_xattn_fwd_f32_masked(const float* q, const float* k, const float* v, f
 
 /*
  * The two fp32 forms (kv_mask may be NULL) with scratch memory for the key split, as svhip_xattn_fwd_ws has it: at
- * least svhip_xattn_f32_workspace_bytes bytes, 16-byte aligned; with a key mask as svhip_xattn_fwd_masked_ws. The parts are kept and joined in fp32.
+ * least svhip_xattn_f32_workspace_bytes bytes, 16-byte aligned; with a key mask as svhip_xattn_fwd_masked_ws. The parts
+ * are kept and joined in fp32.
  */
 size_t svhip_xattn_f32_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap);
 int svhip_xattn_fwd_f32_ws(const float* q, const float* k, const float* v, float* o, const uint8_t* kv_mask,

@@ -72,10 +72,13 @@ void launch(const XattnParams& p, unsigned g, hipStream_t s, bool fp8, bool pv8,
 
 // Workgroups of the split kernels resident on a CU: their registers allow three waves per SIMD up to head_dim 64.
 static int resident(int64_t D) { return D <= 64 ? 3 : 2; }
+// (key_split.hpp)
+constexpr int kTilesPerBlock = 8;
 
 static int xattn_impl(const void* q, const void* k, const void* v, void* o, int kv_dtype, const int32_t* kv_len,
                       const int32_t* cu_seqlens, const float* k_scale, const float* v_scale, const uint8_t* kv_mask,
-                      int64_t sm_b, const int32_t* kv_blocks, int64_t sb_b, int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap, int64_t sq_b,
+                      int64_t sm_b, const int32_t* kv_blocks, int64_t sb_b, int64_t B, int64_t H, int64_t Q,
+                      int64_t D, int64_t kv_cap, int64_t sq_b,
                       int64_t sq_h, int64_t sq_q, int64_t sk_b, int64_t sk_h, int64_t sk_k, int64_t sv_b,
                       int64_t sv_h, int64_t sv_k, int64_t sv_d, int64_t so_b, int64_t so_h, int64_t so_q,
                       float scale, void* workspace, size_t workspace_bytes, void* stream, const char* name) {
@@ -109,8 +112,8 @@ static int xattn_impl(const void* q, const void* k, const void* v, void* o, int 
                       (sv_h * eb) % align == 0 && (sv_b * eb) % align == 0,
                   "%s: V rows must be %d-byte aligned", name, (int)align);
   }
-  SVHIP_REQUIRE(!(kv_mask && kv_len && kv_blocks) || B <= 1 || sb_b > cdiv(kv_cap, kKB),
-                "%s: block rows shorter than the windows' lists", name);
+  const bool listed = kv_mask && kv_len && kv_blocks;
+  SVHIP_REQUIRE(!listed || B <= 1 || sb_b > cdiv(kv_cap, kKB), "%s: block rows shorter than the windows' lists", name);
   if (B == 0 || Q == 0) return SVHIP_OK;
   SVHIP_REQUIRE(kv_cap >= 0 && kv_cap < (1ll << 31), "%s: kv_cap out of range", name);
   XattnParams p;
@@ -159,12 +162,16 @@ static int xattn_impl(const void* q, const void* k, const void* v, void* o, int 
              (kv_cap * sk_k + D) * 2 < (1ll << 32) &&
              (vt ? !cu_seqlens && sv_d % 8 == 0 && (D * sv_d + kv_cap) * 2 < (1ll << 32)
                  : sv_k % 8 == 0 && (kv_cap * sv_k + D) * 2 < (1ll << 32)));
-  // Every bf16 form is split, so that all layouts of the same keys are cut alike and give the same bits. An e4m3 cache
-  // is not: its windows' bits do not depend on the batch they are attended in, and the cuts of the line do. A key mask needs the windows' lists of attended blocks (svhip_mask_blocks), by which the line is cut.
+  // Every bf16 form cuts the same keys into the same pieces, split or not, so that all layouts give the same bits. With
+  // a key mask the split form needs the windows' lists of attended blocks (svhip_mask_blocks). An e4m3 cache's windows
+  // are one piece each.
+  p.lone = lone_teams(Q);
+  p.piece_blocks = kPieceBlocks;
   p.part = nullptr;
   p.teams = 0;
-  if (workspace && !fp8 && !(kv_mask && !(kv_len && kv_blocks))) {
-    const int teams = split_teams(B, H, Q, kv_cap, resident(D));
+  p.resident = 0;
+  if (workspace && !fp8 && (!kv_mask || listed)) {
+    const int teams = split_teams(B, H, Q, kv_cap, resident(D), kPieceBlocks, kTilesPerBlock);
     if (teams) {
       SVHIP_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
                         workspace_bytes >= svhip_xattn_workspace_bytes(B, H, Q, D, kv_cap),
@@ -172,7 +179,8 @@ static int xattn_impl(const void* q, const void* k, const void* v, void* o, int 
                     svhip_xattn_workspace_bytes(B, H, Q, D, kv_cap));
       p.part = static_cast<float*>(workspace);
       p.teams = teams;
-      if (kv_mask) {
+      p.resident = resident_teams(Q, resident(D));
+      if (listed) {
         p.kv_blocks = kv_blocks;
         p.sb_b = sb_b;
       }
@@ -310,7 +318,7 @@ extern "C" int svhip_xattn_trace_set(void* buffer) {
 
 extern "C" size_t svhip_xattn_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap) {
   if (H < 1 || D < 8 || D > kMaxD || kv_cap < 0) return 0;
-  return split_workspace_bytes(B, H, Q, D, kv_cap, resident(D));
+  return split_workspace_bytes(B, H, Q, D, kv_cap, resident(D), kPieceBlocks, kTilesPerBlock);
 }
 
 extern "C" int svhip_xattn_fwd(const void* q, const void* k, const void* v, void* o, int kv_dtype,
@@ -347,8 +355,9 @@ extern "C" int svhip_xattn_fwd_masked(const void* q, const void* k, const void* 
                                       int64_t so_q, float scale, void* stream) {
   clear_error();
   SVHIP_REQUIRE(!(kv_len && cu_seqlens), "svhip_xattn_fwd_masked: kv_len and cu_seqlens are exclusive");
-  return svhip_xattn_fwd_masked_ws(q, k, v, o, kv_mask, sm_b, kv_len, nullptr, 0, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q,
-                                   sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0,
+  return svhip_xattn_fwd_masked_ws(q, k, v, o, kv_mask, sm_b, kv_len, nullptr, 0, cu_seqlens, B, H, Q, D, kv_cap, sq_b,
+                                   sq_h, sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale,
+                                   nullptr, 0,
                                    stream);
 }
 
@@ -363,7 +372,7 @@ extern "C" int svhip_xattn_fwd_masked_ws(const void* q, const void* k, const voi
   const char* name = "svhip_xattn_fwd_masked";
   clear_error();
   SVHIP_REQUIRE(kv_mask, "%s: null key mask", name);
-  return xattn_impl(q, k, v, o, SVHIP_BF16, kv_len, cu_seqlens, nullptr, nullptr, kv_mask, sm_b, kv_blocks, sb_b, B, H, Q, D, kv_cap,
-                    sq_b, sq_h, sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, workspace, workspace_bytes, stream,
-                    name);
+  return xattn_impl(q, k, v, o, SVHIP_BF16, kv_len, cu_seqlens, nullptr, nullptr, kv_mask, sm_b, kv_blocks, sb_b, B, H,
+                    Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale,
+                    workspace, workspace_bytes, stream, name);
 }

@@ -20,9 +20,10 @@
 //                             operand as it stands; A = V[that key][32 j + col] from LDS.
 // The split form (SPLIT) is the bf16 kernel's: see key_split.hpp.
 //
-// One window of 12 x 64 heads, 1024 queries, 9744 keys: 816 us on the VALU (one query a lane, K and V rows broadcast from
-// LDS: 37 TFLOP/s), 286 us here (107 TFLOP/s), 7 us of it the join. The instruction alone reaches 141 TFLOP/s with two
-// waves a SIMD and dependent accumulators, 147 with three.
+// One window of 12 x 64 heads, 1024 queries, 9744 keys: 816 us on the VALU (one query a lane, K and V rows broadcast
+// from LDS: 37 TFLOP/s), 316 us here (97 TFLOP/s), 6 us of it the join (286 us where each workgroup walked an equal
+// share of the blocks, whose cuts moved with the other windows' lengths). The instruction alone reaches 141 TFLOP/s
+// with two waves a SIMD and dependent accumulators, 147 with three.
 //
 // KMASK: a key mask on top of the window length (the reference's `prefix_valid ++ local_valid`): key j of window b
 // is attended only where kv_mask[b * sm_b + j] != 0. A block that the mask wholly masks is skipped; a query may have
@@ -35,6 +36,7 @@ namespace svhip {
 
 constexpr int kF32Row = 64;      // floats of an LDS row (one key)
 constexpr int kF32Resident = 2;  // workgroups per CU (two waves per SIMD)
+constexpr int kF32PieceBlocks = 6;  // least key blocks of a piece
 // Key blocks summed into one accumulator before it is added to the total: short chains of fp32 sums, as the two chains
 // of a score are. From float64, 128 / 400 / 2300 / 9000 keys: 2.6 / 3.0 / 4.0 / 7.0e-7 on the VALU before, 2.2 / 2.3 /
 // 2.6 / 2.8e-7 so; with one chain a score and two blocks 3.1 / 3.4 / 3.5 / 3.8e-7 (8 us faster on the single column),
@@ -65,8 +67,10 @@ struct XattnF32Params {
   int64_t so_b, so_h, so_q;
   float scale_log2;  // softmax scale * log2(e)
   int q_tiles;
-  float* part;
+  int lone, piece_blocks;  // by which windows are cut into pieces (pieces_of)
+  float* part;   // split form: the slots of the parts, the teams in the grid and the teams that the chip holds at once
   int teams;
+  int resident;
 };
 
 // LDS rows are 256 bytes, every bank once. K: 16 rows are read at one 16-byte chunk, so chunk c of row r lies at
@@ -84,30 +88,19 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
   constexpr int kTiles = (D + 31) / 32;               // output tiles of 32 head_dim elements
   static_assert(kKB * kChunks % kThreads == 0, "head_dim a multiple of 16");
   __shared__ __attribute__((aligned(16))) float sK[kKB * kF32Row], sV[kKB * kF32Row];
-  [[maybe_unused]] __shared__ int s_before[SPLIT ? kSplitMaxWindows : 1], s_blocks[SPLIT ? kSplitMaxWindows : 1];
-  [[maybe_unused]] __shared__ int s_total, s_teams;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wg = static_cast<int>(blockIdx.x);
-  int qt, team = 0, pos = 0, range_end = 0;
+  int qt;
+  [[maybe_unused]] int team = 0;
+  [[maybe_unused]] SplitItem item = {};
   int64_t b = 0, h = 0;
   if constexpr (SPLIT) {
     const int seq = wg >> 3;
     qt = seq % p.q_tiles;
     team = (seq / p.q_tiles) * kXcds + (wg & 7);
-    const SplitPlan plan = split_plan(p);
-    if (team >= plan.teams) return;
-    pos = split_cut(p, plan, team);
-    range_end = split_cut(p, plan, team + 1);
-    if (pos >= range_end) return;
-    if (threadIdx.x < kSplitMaxWindows) {
-      s_before[threadIdx.x] = plan.before;
-      s_blocks[threadIdx.x] = plan.blocks;
-    }
-    if (threadIdx.x == 0) {
-      s_total = plan.total;
-      s_teams = plan.teams;
-    }
-    __syncthreads();
+    if (!split_item(p, split_plan(p), team, item)) return;
+    b = item.b;
+    h = item.h;
   } else {
     qt = wg % p.q_tiles;
     const int64_t unit = wg / p.q_tiles;
@@ -116,306 +109,364 @@ __global__ __launch_bounds__(kThreads, kF32Resident) void xattn_f32_kernel(Xattn
   }
   const float sl2 = p.scale_log2;
 
-  do {
-    // SPLIT: the thread index is opaque in every part, so that no part's addresses are kept through the key blocks.
-    int tid = threadIdx.x;
-    if constexpr (SPLIT) asm volatile("" : "+v"(tid));
-    const int lane = tid & 63, col = lane & 31, hh = lane >> 5;
-    const int64_t q = static_cast<int64_t>(qt) * kQTile + w * 32 + col;
-    const bool q_ok = q < p.Q;
-    int blk0 = 0, blk1 = 0, unit_blocks = 0;
-    if constexpr (SPLIT) {
-      SplitPlan plan;
-      plan.before = s_before[lane];
-      plan.blocks = s_blocks[lane];
-      const int bw = split_window(p, plan, pos);
-      unit_blocks = __builtin_amdgcn_readlane(plan.blocks, bw);
-      const int rel = pos - static_cast<int>(p.H) * __builtin_amdgcn_readlane(plan.before, bw);
-      const int hw = __builtin_amdgcn_readfirstlane(rel / unit_blocks);
-      b = bw;
-      h = hw;
-      blk0 = rel - hw * unit_blocks;
-      blk1 = min(unit_blocks, blk0 + (range_end - pos));
-      pos += blk1 - blk0;
-      if (blk0 == 0 && qt == 0 && tid == 0) {
-        split_units(p)[b * p.H + h] =
-            split_unit_teams(team, pos - blk1, unit_blocks, blk1 == unit_blocks, s_total, s_teams);
-      }
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, col = lane & 31, hh = lane >> 5;
+  const int64_t q = static_cast<int64_t>(qt) * kQTile + w * 32 + col;
+  const bool q_ok = q < p.Q;
+  const int L = [&]() __attribute__((always_inline)) {
+    const int n = window_length(p, b);
+    if constexpr (!KMASK || SPLIT) {
+      return n;  // (the split form's lengths are cut at the windows' last attended keys)
+    } else {
+      __shared__ int s_last;
+      if (tid == 0) s_last = -1;
+      __syncthreads();
+      const int last = last_attended(p.kv_mask + b * p.sm_b, n);
+      if (last >= 0) atomicMax(&s_last, last);
+      __syncthreads();
+      return __builtin_amdgcn_readfirstlane(s_last) + 1;
     }
-    const int L = window_length(p, b);
-    if constexpr (!SPLIT) blk1 = unit_blocks = (L + kKB - 1) / kKB;
-    const int64_t off = p.cu_seqlens ? p.cu_seqlens[b] : 0;
-    const uint8_t* mrow = KMASK ? p.kv_mask + b * p.sm_b : nullptr;
-    const float* K = p.k + (p.cu_seqlens ? 0 : b * p.sk_b) + h * p.sk_h + off * p.sk_k;
-    const float* V = p.v + (p.cu_seqlens ? 0 : b * p.sv_b) + h * p.sv_h + off * p.sv_k;
+  }();
+  // The walk: pieces [piece, piece_end) of the unit, blocks [blk0, blk1) (with a list, of its entries).
+  constexpr bool LIST = SPLIT && KMASK;
+  const int unit_blocks = (L + kKB - 1) / kKB;
+  const Pieces pieces = pieces_of(unit_blocks, p.H, p.lone, kF32PieceBlocks);
+  const int piece_end = SPLIT ? item.end : pieces.count;
+  int piece = SPLIT ? item.first : 0;
+  auto next_piece = [&]() __attribute__((always_inline)) -> int {
+    return piece + 1 < piece_end ? piece_start(pieces, piece + 1) : 0x7fffffff;
+  };
+  int bound = next_piece();  // first block of the walk's next piece
+  int blk0 = 0, blk1 = unit_blocks;
+  [[maybe_unused]] int listed = 0;
+  if constexpr (SPLIT) {
+    blk0 = piece_start(pieces, item.first);
+    blk1 = piece_start(pieces, item.end);
+  }
+  if constexpr (LIST) {
+    listed = __builtin_amdgcn_readfirstlane(p.kv_blocks[b * p.sb_b]);
+    blk0 = listed_before(p, b, listed, blk0);
+    blk1 = listed_before(p, b, listed, blk1);
+  }
+  const int64_t off = p.cu_seqlens ? p.cu_seqlens[b] : 0;
+  const uint8_t* mrow = KMASK ? p.kv_mask + b * p.sm_b : nullptr;
+  const float* K = p.k + (p.cu_seqlens ? 0 : b * p.sk_b) + h * p.sk_h + off * p.sk_k;
+  const float* V = p.v + (p.cu_seqlens ? 0 : b * p.sv_b) + h * p.sv_h + off * p.sv_k;
 
-    // Q as B operands: entry 4 s + j is head_dim 8 s + 4 hh + j.
-    float qf[D / 2];
+  // Q as B operands: entry 4 s + j is head_dim 8 s + 4 hh + j.
+  float qf[D / 2];
 #pragma unroll
-    for (int s = 0; s < D / 8; ++s) {
-      float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (q_ok) x = *reinterpret_cast<const float4*>(p.q + b * p.sq_b + h * p.sq_h + q * p.sq_q + 8 * s + 4 * hh);
-      qf[4 * s] = x.x;
-      qf[4 * s + 1] = x.y;
-      qf[4 * s + 2] = x.z;
-      qf[4 * s + 3] = x.w;
-    }
-    f32x16_t o[kTiles], total[kTiles];  // O^T of the last blocks, and of those before
+  for (int s = 0; s < D / 8; ++s) {
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (q_ok) x = *reinterpret_cast<const float4*>(p.q + b * p.sq_b + h * p.sq_h + q * p.sq_q + 8 * s + 4 * hh);
+    qf[4 * s] = x.x;
+    qf[4 * s + 1] = x.y;
+    qf[4 * s + 2] = x.z;
+    qf[4 * s + 3] = x.w;
+  }
+  f32x16_t o[kTiles], total[kTiles];  // O^T of the last blocks, and of those before
 #pragma unroll
-    for (int j = 0; j < kTiles; ++j) o[j] = total[j] = f32x16_t{0};
-    float m = SPLIT && !KMASK && blk0 > 0 ? kPartMax : -INFINITY, l = 0.f;  // l: the lane's own keys
+  for (int j = 0; j < kTiles; ++j) o[j] = total[j] = f32x16_t{0};
+  float m = SPLIT && !KMASK && piece > 0 ? kPieceMax : -INFINITY, l = 0.f;  // l: the lane's own keys
 
-    // Block loads: chunk c = thread + 256 r is key c / kChunks, head_dim 4 (c % kChunks) .. + 3 (of V^T key c % 64,
-    // head_dim 4 (c / 64) .. + 3: consecutive lanes read consecutive keys of a row). Every load is issued
-    // (keys >= L read row L - 1, in bounds); their scores are masked, and V rows past L are zeros so that 0 . V
-    // stays 0.
-    f32x4_t nk[kPer], nv[kPer];
-    auto load_block = [&](int kv0) __attribute__((always_inline)) {
-      // Opaque again: the chunks' addresses are formed per block (hidden behind the products); hoisted, they took 16
-      // registers and were spilled.
-      int tb = tid;
-      asm volatile("" : "+v"(tb));
+  // Block loads: chunk c = thread + 256 r is key c / kChunks, head_dim 4 (c % kChunks) .. + 3 (of V^T key c % 64,
+  // head_dim 4 (c / 64) .. + 3: consecutive lanes read consecutive keys of a row). Every load is issued
+  // (keys >= L read row L - 1, in bounds); their scores are masked, and V rows past L are zeros so that 0 . V
+  // stays 0.
+  f32x4_t nk[kPer], nv[kPer];
+  auto load_block = [&](int kv0) __attribute__((always_inline)) {
+    // Opaque again: the chunks' addresses are formed per block (hidden behind the products); hoisted, they took 16
+    // registers and were spilled.
+    int tb = tid;
+    asm volatile("" : "+v"(tb));
 #pragma unroll
-      for (int r = 0; r < kPer; ++r) {
-        const int c = tb + kThreads * r;
-        const int key = kv0 + c / kChunks, d = 4 * (c % kChunks);
-        const int64_t kc = key < L ? key : L - 1;
-        nk[r] = *reinterpret_cast<const f32x4_t*>(K + kc * p.sk_k + d);
-        if constexpr (VT) {
-          const int kt = kv0 + c % kKB;
-          const float* src = V + 4 * (c / kKB) * p.sv_d + (kt < L ? kt : L - 1);
-          nv[r] = f32x4_t{src[0], src[p.sv_d], src[2 * p.sv_d], src[3 * p.sv_d]};
-          if (kt >= L) nv[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        } else {
-          nv[r] = *reinterpret_cast<const f32x4_t*>(V + kc * p.sv_k + d);
-          if (key >= L) nv[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        }
-      }
-    };
-    auto store_block = [&]() __attribute__((always_inline)) {
-      int tb = tid;
-      asm volatile("" : "+v"(tb));
-#pragma unroll
-      for (int r = 0; r < kPer; ++r) {
-        const int c = tb + kThreads * r;
-        const int key = c / kChunks, dc = c % kChunks;
-        *reinterpret_cast<f32x4_t*>(sK + key * kF32Row + 4 * f32_swz_k(key, dc)) = nk[r];
-        const int vkey = VT ? c % kKB : key, vc = VT ? c / kKB : dc;
-        *reinterpret_cast<f32x4_t*>(sV + vkey * kF32Row + 4 * f32_swz_v(vkey, vc)) = nv[r];
-      }
-    };
-    // Bit i: key kv0 + i is below L and attended (wave-uniform; lane i's byte).
-    auto load_mask = [&](int kv0) __attribute__((always_inline)) -> int {
-      const int j = kv0 + lane;
-      if constexpr (KMASK) {
-        const int jc = j < L ? j : L - 1;
-        return (mrow[jc] != 0 && j < L) ? 1 : 0;
+    for (int r = 0; r < kPer; ++r) {
+      const int c = tb + kThreads * r;
+      const int key = kv0 + c / kChunks, d = 4 * (c % kChunks);
+      const int64_t kc = key < L ? key : L - 1;
+      nk[r] = *reinterpret_cast<const f32x4_t*>(K + kc * p.sk_k + d);
+      if constexpr (VT) {
+        const int kt = kv0 + c % kKB;
+        const float* src = V + 4 * (c / kKB) * p.sv_d + (kt < L ? kt : L - 1);
+        nv[r] = f32x4_t{src[0], src[p.sv_d], src[2 * p.sv_d], src[3 * p.sv_d]};
+        if (kt >= L) nv[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       } else {
-        return j < L ? 1 : 0;
+        nv[r] = *reinterpret_cast<const f32x4_t*>(V + kc * p.sv_k + d);
+        if (key >= L) nv[r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       }
-    };
-    // First key of block i of the unit (with a key mask the i-th of the window's blocks with an attended key).
-    auto key_of = [&](int i) __attribute__((always_inline)) -> int {
-      if constexpr (SPLIT && KMASK) {
-        return kKB * (p.kv_blocks ? listed_block(p, b, min(i, unit_blocks - 1)) : i);
-      } else {
-        return kKB * i;
-      }
-    };
-    int on = 0;
-    if (blk0 < blk1) {
-      const int kv0 = key_of(blk0);
-      load_block(kv0);
-      on = load_mask(kv0);
-      store_block();
     }
-    int kv_next = key_of(blk0 + 1);
-    __syncthreads();
-    for (int blk = blk0; blk < blk1; ++blk) {
-      const uint64_t bits = __builtin_amdgcn_ballot_w64(on != 0);
-      const bool more = blk + 1 < blk1;
-      if (more) {
-        load_block(kv_next);
-        on = load_mask(kv_next);
-        kv_next = key_of(blk + 2);
+  };
+  auto store_block = [&]() __attribute__((always_inline)) {
+    int tb = tid;
+    asm volatile("" : "+v"(tb));
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+      const int c = tb + kThreads * r;
+      const int key = c / kChunks, dc = c % kChunks;
+      *reinterpret_cast<f32x4_t*>(sK + key * kF32Row + 4 * f32_swz_k(key, dc)) = nk[r];
+      const int vkey = VT ? c % kKB : key, vc = VT ? c / kKB : dc;
+      *reinterpret_cast<f32x4_t*>(sV + vkey * kF32Row + 4 * f32_swz_v(vkey, vc)) = nv[r];
+    }
+  };
+  // Bit i: key kv0 + i is below L and attended (wave-uniform; lane i's byte).
+  auto load_mask = [&](int kv0) __attribute__((always_inline)) -> int {
+    const int j = kv0 + lane;
+    if constexpr (KMASK) {
+      const int jc = j < L ? j : L - 1;
+      return (mrow[jc] != 0 && j < L) ? 1 : 0;
+    } else {
+      return j < L ? 1 : 0;
+    }
+  };
+  // First key of block i of the unit (of the list).
+  auto key_of = [&](int i) __attribute__((always_inline)) -> int {
+    if constexpr (LIST) {
+      return kKB * listed_block(p, b, min(i, listed - 1));
+    } else {
+      return kKB * i;
+    }
+  };
+  // The pieces walked before the current one, joined (in LDS, of which two workgroups leave enough: a slot per lane).
+  __shared__ __attribute__((aligned(16))) f32x4_t s_joined[4 * kTiles + 1][kThreads];
+  bool folded = false;
+  // The current piece's sums, joined to the pieces before it: m, l (of both lane halves) and `total` are the walk's.
+  auto join = [&]() __attribute__((always_inline)) {
+    l += __shfl_xor(l, 32, 64);
+    if (!folded) return;
+    const f32x4_t ml = s_joined[4 * kTiles][tid];
+    float x, y, mn = ml[0];
+    join_factors(mn, m, x, y);
+    m = mn;
+    l = join_value(ml[1], l, x, y);
+#pragma unroll
+    for (int j = 0; j < kTiles; ++j) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4_t at = s_joined[4 * j + g][tid];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) total[j][4 * g + e] = join_value(at[e], total[j][4 * g + e], x, y);
       }
-      if (!KMASK || bits != 0ull) {
-        // The running max taken off the scores. Without a key mask -inf stays: a query whose every score is -inf gets
-        // NaN, as a softmax over them does.
-        auto bias = [&]() __attribute__((always_inline)) { return KMASK && m == -INFINITY ? 0.f : -m; };
-        // One weight, formed where it stands in the code: the volatile asm keeps it from sinking to its use.
-        auto weight = [&](float& x, float nm, float& sum) __attribute__((always_inline)) {
-          x = __builtin_amdgcn_exp2f(__builtin_fmaf(x, sl2, nm));
-          sum += x;
-          asm volatile("" : "+v"(x), "+v"(sum));
-        };
-        // S^T of half t (keys 32 t .. 32 t + 31 of the block), the weights of `w` (UNDER) between its products.
-        auto score = [&](int t, auto under, f32x16_t& w) __attribute__((always_inline)) {
-          constexpr bool UNDER = decltype(under)::value;
-          constexpr int kSteps = D / 8, kEach = (16 + kSteps - 1) / kSteps;
-          const float nm = UNDER ? bias() : 0.f;
-          f32x16_t s, odd;  // the even and the odd steps' products: two chains half as long
-          float sum = 0.f;
-          const float* kr = sK + (32 * t + col) * kF32Row;
-          f32x4_t x = *reinterpret_cast<const f32x4_t*>(kr + 4 * f32_swz_k(col, hh));
+    }
+  };
+  // A piece has ended inside the walk: start the one that holds the next block, block `next`.
+  auto fold = [&](int next) __attribute__((always_inline)) {
+    join();
 #pragma unroll
-          for (int c = 0; c < kSteps; ++c) {
-            f32x4_t next = x;
-            if (c + 1 < kSteps) next = *reinterpret_cast<const f32x4_t*>(kr + 4 * f32_swz_k(col, 2 * (c + 1) + hh));
+    for (int j = 0; j < kTiles; ++j) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              f32x16_t& acc = e % 2 == 0 ? s : odd;
-              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], qf[4 * c + e], c + e / 2 == 0 ? f32x16_t{0} : acc, 0, 0,
-                                                         0);
-            }
-            x = next;
-            if constexpr (UNDER) {
+      for (int i = 0; i < 16; i += 4) {
+        s_joined[4 * j + i / 4][tid] = f32x4_t{total[j][i], total[j][i + 1], total[j][i + 2], total[j][i + 3]};
+      }
+      total[j] = f32x16_t{0};
+    }
+    s_joined[4 * kTiles][tid] = f32x4_t{m, l, 0.f, 0.f};
+    m = KMASK ? -INFINITY : kPieceMax;
+    l = 0.f;
+    folded = true;
+    do {
+      ++piece;
+      bound = next_piece();
+    } while (next >= bound);
+  };
+  int on = 0;
+  if (blk0 < blk1) {
+    const int kv0 = key_of(blk0);
+    while (kv0 / kKB >= bound) {  // pieces without a listed block add nothing
+      ++piece;
+      bound = next_piece();
+    }
+    load_block(kv0);
+    on = load_mask(kv0);
+    store_block();
+  }
+  int kv_next = blk0 < blk1 ? key_of(blk0 + 1) : 0;
+  __syncthreads();
+  for (int blk = blk0; blk < blk1; ++blk) {
+    const uint64_t bits = __builtin_amdgcn_ballot_w64(on != 0);
+    const bool more = blk + 1 < blk1;
+    const int next = kv_next / kKB;
+    if (more) {
+      load_block(kv_next);
+      on = load_mask(kv_next);
+      kv_next = key_of(blk + 2);
+    }
+    if (!KMASK || bits != 0ull) {
+      // The running max taken off the scores. Without a key mask -inf stays: a query whose every score is -inf gets
+      // NaN, as a softmax over them does.
+      auto bias = [&]() __attribute__((always_inline)) { return KMASK && m == -INFINITY ? 0.f : -m; };
+      // One weight, formed where it stands in the code: the volatile asm keeps it from sinking to its use.
+      auto weight = [&](float& x, float nm, float& sum) __attribute__((always_inline)) {
+        x = __builtin_amdgcn_exp2f(__builtin_fmaf(x, sl2, nm));
+        sum += x;
+        asm volatile("" : "+v"(x), "+v"(sum));
+      };
+      // S^T of half t (keys 32 t .. 32 t + 31 of the block), the weights of `w` (UNDER) between its products.
+      auto score = [&](int t, auto under, f32x16_t& w) __attribute__((always_inline)) {
+        constexpr bool UNDER = decltype(under)::value;
+        constexpr int kSteps = D / 8, kEach = (16 + kSteps - 1) / kSteps;
+        const float nm = UNDER ? bias() : 0.f;
+        f32x16_t s, odd;  // the even and the odd steps' products: two chains half as long
+        float sum = 0.f;
+        const float* kr = sK + (32 * t + col) * kF32Row;
+        f32x4_t x = *reinterpret_cast<const f32x4_t*>(kr + 4 * f32_swz_k(col, hh));
 #pragma unroll
-              for (int i = kEach * c; i < kEach * (c + 1) && i < 16; ++i) {
-                float y = w[i];
-                weight(y, nm, sum);
-                w[i] = y;
-              }
-            }
-            __builtin_amdgcn_sched_barrier(0);
+        for (int c = 0; c < kSteps; ++c) {
+          f32x4_t next = x;
+          if (c + 1 < kSteps) next = *reinterpret_cast<const f32x4_t*>(kr + 4 * f32_swz_k(col, 2 * (c + 1) + hh));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            f32x16_t& acc = e % 2 == 0 ? s : odd;
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], qf[4 * c + e], c + e / 2 == 0 ? f32x16_t{0} : acc, 0, 0,
+                                                       0);
           }
-          if constexpr (UNDER) l += sum;
+          x = next;
+          if constexpr (UNDER) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) s[i] += odd[i];
-          return s;
-        };
-        // The half's largest score, keys not attended put to -inf.
-        auto mask_max = [&](f32x16_t& s, int t) __attribute__((always_inline)) {
-          if (bits != ~0ull) {
-            const uint32_t mine = static_cast<uint32_t>(bits >> (32 * t)) >> (4 * hh);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              if (!((mine >> (8 * (i / 4) + i % 4)) & 1u)) s[i] = -INFINITY;
-            }
-          }
-          float mb = s[0];
-#pragma unroll
-          for (int i = 1; i < 16; ++i) mb = fmaxf(mb, s[i]);
-          return fmaxf(mb, __shfl_xor(mb, 32, 64)) * sl2;
-        };
-        // The running max is raised only where a score passes it by kF32Rise (the weights stay below 2^kF32Rise, which
-        // costs fp32 sums nothing); O, l and the weights `held` already formed come down with it.
-        auto raise = [&](float mb, f32x16_t* held) __attribute__((always_inline)) {
-          if (__builtin_amdgcn_ballot_w64(mb > m + kF32Rise) != 0ull) {
-            // alpha is 0 on a query's first attended keys (m = -inf), with O and l still 0.
-            const float mn = fmaxf(m, mb);
-            const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
-            m = mn;
-            l *= alpha;
-#pragma unroll
-            for (int j = 0; j < kTiles; ++j) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) {
-                o[j][i] *= alpha;
-                total[j][i] *= alpha;
-              }
-            }
-            if (held) {
-#pragma unroll
-              for (int i = 0; i < 16; ++i) (*held)[i] *= alpha;
-            }
-          }
-        };
-        // O^T += V^T . P^T of half t, the weights of `w` (UNDER) between its products.
-        auto pv = [&](const f32x16_t& s, int t, auto under, f32x16_t& w) __attribute__((always_inline)) {
-          constexpr bool UNDER = decltype(under)::value;
-          const float nm = UNDER ? bias() : 0.f;
-          float sum = 0.f;
-          // Entry i is key 32 t + 8 (i / 4) + 4 hh + i % 4; f32_swz_v on floats: bit 5 of the row's float index flips
-          // with bit 2 of the key, which is hh.
-          auto read = [&](int i, int j) __attribute__((always_inline)) {
-            return sV[(32 * t + 8 * (i / 4) + 4 * hh + i % 4) * kF32Row + ((32 * j + col) ^ (32 * hh))];
-          };
-          float x[kTiles], next[kTiles];
-#pragma unroll
-          for (int j = 0; j < kTiles; ++j) x[j] = read(0, j);
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-#pragma unroll
-            for (int j = 0; j < kTiles; ++j) next[j] = i + 1 < 16 ? read(i + 1, j) : 0.f;
-#pragma unroll
-            for (int j = 0; j < kTiles; ++j) {
-              o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[j], s[i], o[j], 0, 0, 0);
-              x[j] = next[j];
-            }
-            if constexpr (UNDER) {
+            for (int i = kEach * c; i < kEach * (c + 1) && i < 16; ++i) {
               float y = w[i];
               weight(y, nm, sum);
               w[i] = y;
             }
-            __builtin_amdgcn_sched_barrier(0);
           }
-          if constexpr (UNDER) l += sum;
-        };
-        // Half 0's weights under half 1's score product, half 1's under half 0's second product (a product is 16 passes,
-        // a weight three VALU instructions): a wave left alone on its SIMD still keeps the matrix core busy.
-        f32x16_t none;
-        f32x16_t s0 = score(0, std::false_type{}, none);
-        raise(mask_max(s0, 0), nullptr);
-        f32x16_t s1 = score(1, std::true_type{}, s0);
-        raise(mask_max(s1, 1), &s0);
-        pv(s0, 0, std::true_type{}, s1);
-        pv(s1, 1, std::false_type{}, none);
-      }
-      if ((blk - blk0) % kF32Fold == kF32Fold - 1 || !more) {
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (UNDER) l += sum;
 #pragma unroll
-        for (int j = 0; j < kTiles; ++j) {
+        for (int i = 0; i < 16; ++i) s[i] += odd[i];
+        return s;
+      };
+      // The half's largest score, keys not attended put to -inf.
+      auto mask_max = [&](f32x16_t& s, int t) __attribute__((always_inline)) {
+        if (bits != ~0ull) {
+          const uint32_t mine = static_cast<uint32_t>(bits >> (32 * t)) >> (4 * hh);
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
-            total[j][i] += o[j][i];
-            o[j][i] = 0.f;
+            if (!((mine >> (8 * (i / 4) + i % 4)) & 1u)) s[i] = -INFINITY;
           }
         }
-      }
-      __syncthreads();
-      if (more) {
-        store_block();
-        __syncthreads();
-      }
-    }
-    l += __shfl_xor(l, 32, 64);
-
-    if constexpr (SPLIT) {
-      if (blk1 - blk0 < unit_blocks) {
-        float* slot = p.part + (static_cast<int64_t>(2 * team + (blk0 == 0 ? 1 : 0)) * p.q_tiles + qt) *
-                                   split_slot_floats(D);
-        const int ql = w * 32 + col;
+        float mb = s[0];
 #pragma unroll
-        for (int j = 0; j < kTiles; ++j) {
+        for (int i = 1; i < 16; ++i) mb = fmaxf(mb, s[i]);
+        return fmaxf(mb, __shfl_xor(mb, 32, 64)) * sl2;
+      };
+      // The running max is raised only where a score passes it by kF32Rise (the weights stay below 2^kF32Rise, which
+      // costs fp32 sums nothing); O, l and the weights `held` already formed come down with it.
+      auto raise = [&](float mb, f32x16_t* held) __attribute__((always_inline)) {
+        if (__builtin_amdgcn_ballot_w64(mb > m + kF32Rise) != 0ull) {
+          // alpha is 0 on a query's first attended keys (m = -inf), with O and l still 0.
+          const float mn = fmaxf(m, mb);
+          const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+          m = mn;
+          l *= alpha;
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int d0 = 32 * j + 8 * g + 4 * hh;
-            if (d0 < D) {
-              split_store(slot, d0, ql, total[j][4 * g], total[j][4 * g + 1], total[j][4 * g + 2], total[j][4 * g + 3]);
+          for (int j = 0; j < kTiles; ++j) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              o[j][i] *= alpha;
+              total[j][i] *= alpha;
             }
           }
+          if (held) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) (*held)[i] *= alpha;
+          }
         }
-        if (hh == 0) {
-          slot[kQTile * D + ql] = KMASK && l == 0.f ? -INFINITY : m;
-          slot[kQTile * (D + 1) + ql] = l;
+      };
+      // O^T += V^T . P^T of half t, the weights of `w` (UNDER) between its products.
+      auto pv = [&](const f32x16_t& s, int t, auto under, f32x16_t& w) __attribute__((always_inline)) {
+        constexpr bool UNDER = decltype(under)::value;
+        const float nm = UNDER ? bias() : 0.f;
+        float sum = 0.f;
+        // Entry i is key 32 t + 8 (i / 4) + 4 hh + i % 4; f32_swz_v on floats: bit 5 of the row's float index flips
+        // with bit 2 of the key, which is hh.
+        auto read = [&](int i, int j) __attribute__((always_inline)) {
+          return sV[(32 * t + 8 * (i / 4) + 4 * hh + i % 4) * kF32Row + ((32 * j + col) ^ (32 * hh))];
+        };
+        float x[kTiles], next[kTiles];
+#pragma unroll
+        for (int j = 0; j < kTiles; ++j) x[j] = read(0, j);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+#pragma unroll
+          for (int j = 0; j < kTiles; ++j) next[j] = i + 1 < 16 ? read(i + 1, j) : 0.f;
+#pragma unroll
+          for (int j = 0; j < kTiles; ++j) {
+            o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[j], s[i], o[j], 0, 0, 0);
+            x[j] = next[j];
+          }
+          if constexpr (UNDER) {
+            float y = w[i];
+            weight(y, nm, sum);
+            w[i] = y;
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
-        continue;
-      }
+        if constexpr (UNDER) l += sum;
+      };
+      // Half 0's weights under half 1's score product, half 1's under half 0's second product (a product is 16 passes,
+      // a weight three VALU instructions): a wave left alone on its SIMD still keeps the matrix core busy.
+      f32x16_t none;
+      f32x16_t s0 = score(0, std::false_type{}, none);
+      raise(mask_max(s0, 0), nullptr);
+      f32x16_t s1 = score(1, std::true_type{}, s0);
+      raise(mask_max(s1, 1), &s0);
+      pv(s0, 0, std::true_type{}, s1);
+      pv(s1, 1, std::false_type{}, none);
     }
-    if (q_ok) {
-      // No key at all (L = 0, or no attended key): zeros, as the bf16 kernel writes.
-      const float inv = l == 0.f ? 0.f : 1.f / l;
-      float* out = p.o + b * p.so_b + h * p.so_h + q * p.so_q;
+    if ((blk - blk0) % kF32Fold == kF32Fold - 1 || !more || next >= bound) {
 #pragma unroll
       for (int j = 0; j < kTiles; ++j) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int d = 32 * j + 8 * (i / 4) + 4 * hh + i % 4;
-          if (d < D) out[d] = total[j][i] * inv;
+          total[j][i] += o[j][i];
+          o[j][i] = 0.f;
         }
       }
     }
-  } while (SPLIT && pos < range_end);
+    if (more && next >= bound) fold(next);
+    __syncthreads();
+    if (more) {
+      store_block();
+      __syncthreads();
+    }
+  }
+  join();
+
+  if constexpr (SPLIT) {
+    split_publish(p, item, team, qt);
+    if (item.first > 0 || item.end < pieces.count) {
+      float* slot = split_slot(p, team, qt);
+      const int ql = w * 32 + col;
+#pragma unroll
+      for (int j = 0; j < kTiles; ++j) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int d0 = 32 * j + 8 * g + 4 * hh;
+          if (d0 < D) {
+            split_store(slot, d0, ql, total[j][4 * g], total[j][4 * g + 1], total[j][4 * g + 2], total[j][4 * g + 3]);
+          }
+        }
+      }
+      if (hh == 0) {
+        slot[kQTile * D + ql] = m;
+        slot[kQTile * (D + 1) + ql] = l;
+      }
+      return;
+    }
+  }
+  if (q_ok) {
+    // No key at all (L = 0, or no attended key): zeros, as the bf16 kernel writes.
+    const float inv = l == 0.f ? 0.f : 1.f / l;
+    float* out = p.o + b * p.so_b + h * p.so_h + q * p.so_q;
+#pragma unroll
+    for (int j = 0; j < kTiles; ++j) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int d = 32 * j + 8 * (i / 4) + 4 * hh + i % 4;
+        if (d < D) out[d] = total[j][i] * inv;
+      }
+    }
+  }
 }
 
 template <int D, bool VT, bool KMASK>
@@ -508,18 +559,21 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
   p.q_tiles = static_cast<int>(cdiv(Q, kQTile));
   const int64_t grid = static_cast<int64_t>(p.q_tiles) * H * B;
   SVHIP_REQUIRE(grid < (1ll << 31), "%s: grid too large", name);
+  p.lone = lone_teams(Q);
+  p.piece_blocks = kF32PieceBlocks;
   p.part = nullptr;
   p.teams = 0;
-  // Several windows with a key mask need their lists of attended blocks (svhip_mask_blocks), by which the line is cut; a
-  // single one is cut by its capacity.
-  if (workspace && !(kv_mask && B > 1 && !listed)) {
-    const int teams = split_teams(B, H, Q, kv_cap, kF32Resident);
-    const size_t need = split_workspace_bytes(B, H, Q, D, kv_cap, kF32Resident);
+  p.resident = 0;
+  // With a key mask the split form needs the windows' lists of attended blocks (svhip_mask_blocks).
+  if (workspace && (!kv_mask || listed)) {
+    const int teams = split_teams(B, H, Q, kv_cap, kF32Resident, kF32PieceBlocks, 0);
+    const size_t need = split_workspace_bytes(B, H, Q, D, kv_cap, kF32Resident, kF32PieceBlocks, 0);
     if (teams) {
       SVHIP_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= need,
                     "%s: workspace too small or unaligned (%zu < %zu bytes)", name, workspace_bytes, need);
       p.part = static_cast<float*>(workspace);
       p.teams = teams;
+      p.resident = resident_teams(Q, kF32Resident);
       if (listed) {
         p.kv_blocks = kv_blocks;
         p.sb_b = sb_b;
@@ -548,7 +602,7 @@ static int xattn_f32_impl(const float* q, const float* k, const float* v, float*
 
 extern "C" size_t svhip_xattn_f32_workspace_bytes(int64_t B, int64_t H, int64_t Q, int64_t D, int64_t kv_cap) {
   if (H < 1 || D < 1 || kv_cap < 0) return 0;
-  return split_workspace_bytes(B, H, Q, D, kv_cap, kF32Resident);
+  return split_workspace_bytes(B, H, Q, D, kv_cap, kF32Resident, kF32PieceBlocks, 0);
 }
 
 extern "C" int svhip_xattn_fwd_f32_ws(const float* q, const float* k, const float* v, float* o, const uint8_t* kv_mask,
@@ -560,8 +614,8 @@ extern "C" int svhip_xattn_fwd_f32_ws(const float* q, const float* k, const floa
                                       int64_t so_q, float scale, void* workspace, size_t workspace_bytes,
                                       void* stream) {
   return xattn_f32_impl(q, k, v, o, kv_mask, sm_b, kv_blocks, sb_b, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h,
-                        sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, workspace, workspace_bytes, stream,
-                        "svhip_xattn_fwd_f32_ws");
+                        sq_q, sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, workspace,
+                        workspace_bytes, stream, "svhip_xattn_fwd_f32_ws");
 }
 
 extern "C" int svhip_xattn_fwd_f32(const float* q, const float* k, const float* v, float* o, const int32_t* kv_len,
@@ -569,8 +623,8 @@ extern "C" int svhip_xattn_fwd_f32(const float* q, const float* k, const float* 
                                    int64_t kv_cap, int64_t sq_b, int64_t sq_h, int64_t sq_q, int64_t sk_b,
                                    int64_t sk_h, int64_t sk_k, int64_t sv_b, int64_t sv_h, int64_t sv_k, int64_t sv_d,
                                    int64_t so_b, int64_t so_h, int64_t so_q, float scale, void* stream) {
-  return xattn_f32_impl(q, k, v, o, nullptr, 0, nullptr, 0, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b, sk_h,
-                        sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0, stream,
+  return xattn_f32_impl(q, k, v, o, nullptr, 0, nullptr, 0, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q,
+                        sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0, stream,
                         "svhip_xattn_fwd_f32");
 }
 
@@ -584,7 +638,7 @@ extern "C" int svhip_xattn_fwd_f32_masked(const float* q, const float* k, const 
   const char* name = "svhip_xattn_fwd_f32_masked";
   clear_error();
   SVHIP_REQUIRE(kv_mask, "%s: null key mask", name);
-  return xattn_f32_impl(q, k, v, o, kv_mask, sm_b, nullptr, 0, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q, sk_b,
-                        sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0, stream,
+  return xattn_f32_impl(q, k, v, o, kv_mask, sm_b, nullptr, 0, kv_len, cu_seqlens, B, H, Q, D, kv_cap, sq_b, sq_h, sq_q,
+                        sk_b, sk_h, sk_k, sv_b, sv_h, sv_k, sv_d, so_b, so_h, so_q, scale, nullptr, 0, stream,
                         name);
 }

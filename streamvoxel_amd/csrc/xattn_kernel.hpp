@@ -27,7 +27,8 @@
 //   * P is formed against the running max m as it stands. The half's row sum (read back from the matrix cores
 //     before the second product is issued) tells whether m still bounds the half's scores: only a sum above 2^20
 //     (and always the window's first half) makes the wave take the half's max (16 three-input maxes and the
-//     partner's over v_permlane32_swap), raise m, rescale O and l and redo P and its sum shifted by the rise. P may thus reach 2^20, harmless in fp32 sums and bf16 P; O and l always share m, so
+//     partner's over v_permlane32_swap), raise m, rescale O and l and redo P and its sum
+//     shifted by the rise. P may thus reach 2^20, harmless in fp32 sums and bf16 P; O and l always share m, so
 //     O / l does not depend on where m sits.
 //   * With direct staging and head_dim below 32 DT (the shipped 48) V^T row D, a padding row, holds ones: the
 //     second product then accumulates the row sum of the bf16 P in O^T row D, and the VALU drops the adds. The
@@ -86,6 +87,7 @@ constexpr int kSub = 64;      // head_dim elements per K sub-tile row (smaller h
 constexpr int kMaxD = 128;    // widest head (DT = 4)
 constexpr int kRow = 64;      // LDS row stride in bf16 elements (128 bytes, 16-byte chunks XOR-swizzled)
 constexpr int kKTile = kKB * kRow;  // bf16 elements of one K sub-tile
+constexpr int kPieceBlocks = 12;  // least key blocks of a piece
 constexpr float kSumHigh = 1048576.0f;  // 2^20: a half's row sum above it makes the running max be raised
 constexpr float kMaxHigh = 20.0f;       // the same bound on a single score above the running max (log2 units)
 // The bf16 row-sum form issues a half's second product before it reads the half's row sum back: its stored max
@@ -194,8 +196,10 @@ struct XattnParams {
   int64_t so_b, so_h, so_q;
   float scale_log2;  // softmax scale * log2(e), > 0
   int q_tiles;
-  float* part;       // key split: the partial results, [team][2][query tile] slots of split_slot_floats(D)
-  int teams;         // key split: teams of q_tiles workgroups in the grid, a multiple of kXcds
+  int lone, piece_blocks;    // by which windows are cut into pieces (pieces_of)
+  float* part;       // split form: the slots of the parts
+  int teams;         // split form: teams of q_tiles workgroups in the grid, a multiple of kXcds
+  int resident;      // split form: the teams that the chip holds at once
 };
 
 // Physical 16-byte chunk of logical chunk c in LDS row r. The 64 banks span two 128-byte rows and a 16-byte read
@@ -360,10 +364,10 @@ __device__ __forceinline__ typename Raw<FP8>::type raw_select(bool keep, const t
 template <bool FP8, bool VT, int DT, bool TAIL, bool ONES = false, bool VREG = true>
 __device__ __forceinline__ void stage_load(Stage<FP8, VT, DT>& st, const XattnParams& p,
                                            const typename Elem<FP8>::T* K, const typename Elem<FP8>::T* V, int L,
-                                           int kv0, int dchunks, bool vt_vec, int tid) {
+                                           int kv0, int dchunks, bool vt_vec) {
 #pragma unroll
   for (int r = 0; r < Width<DT>::kKPasses; ++r) {
-    const int c = tid + kThreads * (r & 1);  // 0..511
+    const int c = threadIdx.x + kThreads * (r & 1);  // 0..511
     const int key = c >> 3, dc = 8 * (r >> 1) + (c & 7);
     const int kg = kv0 + key;
     if constexpr (TAIL) {
@@ -379,7 +383,7 @@ __device__ __forceinline__ void stage_load(Stage<FP8, VT, DT>& st, const XattnPa
   if constexpr (VT && VREG) {
 #pragma unroll
     for (int r = 0; r < DT; ++r) {
-      const int c = tid + kThreads * r;
+      const int c = threadIdx.x + kThreads * r;
       const int d = c >> 3, kc = c & 7;
       const int kg = kv0 + kc * 8;
       if (!TAIL && vt_vec) {
@@ -401,12 +405,12 @@ __device__ __forceinline__ void stage_load(Stage<FP8, VT, DT>& st, const XattnPa
 // row-major V byte by byte.
 template <bool FP8, bool VT, int DT, bool ONES, bool PV8 = false, bool VREG = true>
 __device__ __forceinline__ void stage_store(const Stage<FP8, VT, DT>& st, uint16_t* sK, uint16_t* sV, int dchunks,
-                                            int D, int tid) {
+                                            int D) {
   static_assert(!PV8 || FP8, "the e4m3 second product takes e4m3 V");
   using R8 = typename Raw<FP8>::type;
 #pragma unroll
   for (int r = 0; r < Width<DT>::kKPasses; ++r) {
-    const int c = tid + kThreads * (r & 1);
+    const int c = threadIdx.x + kThreads * (r & 1);
     const int R = PV8 ? pv8_row(c >> 3) : sigma_row(c >> 3), dc = c & 7;
     const bool ok = 8 * (r >> 1) + dc < dchunks;
     *reinterpret_cast<uint4*>(sK + (r >> 1) * kKTile + R * kRow + swz(R, dc) * 8) =
@@ -435,7 +439,7 @@ __device__ __forceinline__ void stage_store(const Stage<FP8, VT, DT>& st, uint16
   if constexpr (VT && VREG) {
 #pragma unroll
     for (int r = 0; r < DT; ++r) {
-      const int c = tid + kThreads * r;
+      const int c = threadIdx.x + kThreads * r;
       const int d = c >> 3, kc = c & 7;
       const R8 vv = raw_select<FP8>(d < D, st.v[r], (ONES && d == D) ? raw_one<FP8>() : raw_zero<FP8>());
       if constexpr (PV8) {
@@ -451,7 +455,8 @@ __device__ __forceinline__ void stage_store(const Stage<FP8, VT, DT>& st, uint16
 // Direct path (bf16 K and V^T, full blocks): buffer_load_dwordx4 ... lds moves a block straight into LDS without
 // registers. Wave instruction j of a tile fills its rows 8 j .. 8 j + 7 (1024 consecutive bytes, lane l at
 // 16 l): row R = 8 j + l / 8, physical chunk l % 8, so the logical chunk c with swz(R, c) = l % 8. The 8
-// instructions of a tile go to the 4 waves two each. A lane's byte offsets from the (window, head) base depend only on the window, so
+// instructions of a tile go to the 4 waves two each. A lane's byte offsets from the (window, head) base depend only on
+// the window, so
 // they are computed once; a block adds kv0 rows of K / columns of V^T through the scalar offset. The buffer
 // descriptors bound the reads to the window's full blocks (an out-of-range read returns zeros).
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -473,8 +478,9 @@ constexpr int kRsrcFlags = 0x00020000;
 
 template <int DT>
 __device__ __forceinline__ DirectLanes<DT> direct_lanes(const XattnParams& p, const uint16_t* K, const uint16_t* V,
-                                                        int dchunks, int nfull, int w, int lane) {
+                                                        int dchunks, int nfull, int w) {
   DirectLanes<DT> dl;
+  const int lane = threadIdx.x & 63;
   const uint32_t k_bytes = static_cast<uint32_t>(((static_cast<int64_t>(nfull) * kKB - 1) * p.sk_k + p.D) * 2);
   const uint32_t v_bytes = static_cast<uint32_t>(((p.D - 1) * p.sv_d + static_cast<int64_t>(nfull) * kKB) * 2);
   dl.k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(K), 0, k_bytes, kRsrcFlags);
@@ -536,8 +542,9 @@ struct DirectRows {
 
 template <int DT>
 __device__ __forceinline__ DirectRows<DT> direct_rows(const XattnParams& p, const uint16_t* V, int dchunks, int nfull,
-                                                      int w, int lane) {
+                                                      int w) {
   DirectRows<DT> dr;
+  const int lane = threadIdx.x & 63;
   const uint32_t bytes = static_cast<uint32_t>(((static_cast<int64_t>(nfull) * kKB - 1) * p.sv_k + p.D) * 2);
   dr.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(V), 0, bytes, kRsrcFlags);
 #pragma unroll
@@ -602,38 +609,6 @@ __device__ __forceinline__ void direct_v8_load(__amdgpu_buffer_rsrc_t rsrc, uint
 
 __device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// The highest index j < n with row[j] != 0 among the ones this thread reads (thread t of kThreads: 16-byte chunks
-// t, t + kThreads, ... of a 16-byte aligned row, four loads in flight; the rest, or an unaligned row, byte by byte
-// with eight loads in flight), or -1. The caller takes the maximum over the workgroup.
-__device__ __forceinline__ int last_attended(const uint8_t* row, int n) {
-  int last = -1;
-  const int nvec = (reinterpret_cast<uintptr_t>(row) & 15) == 0 ? n / 16 : 0;
-  for (int c0 = threadIdx.x; c0 < nvec; c0 += 4 * kThreads) {
-    uint4 x[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int c = c0 + u * kThreads;
-      x[u] = c < nvec ? reinterpret_cast<const uint4*>(row)[c] : make_uint4(0u, 0u, 0u, 0u);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const uint32_t w[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {  // the highest nonzero byte of word q: byte 4 q + (31 - clz) / 8
-        if (w[q] != 0u) last = max(last, 16 * (c0 + u * kThreads) + 4 * q + ((31 - __clz(w[q])) >> 3));
-      }
-    }
-  }
-  for (int j0 = 16 * nvec + threadIdx.x; j0 < n; j0 += 8 * kThreads) {
-    uint8_t v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = row[min(j0 + u * kThreads, n - 1)];  // no branch around the loads
-#pragma unroll
-    for (int u = 0; u < 8; ++u) last = (v[u] && j0 + u * kThreads < n) ? max(last, j0 + u * kThreads) : last;
-  }
-  return last;
-}
-
 // STAGING: kRegister (registers for every block), kDirect (direct loads for full blocks, any head_dim),
 // kDirectFull (the same at head_dim 32 DT), kRegisterFull (registers at head_dim 32 DT). The last, partial block
 // of a window always goes through registers. At head_dim 32 DT the score product's k-steps are all known at
@@ -648,7 +623,7 @@ enum Staging { kRegister = 0, kDirect = 1, kDirectFull = 2, kRegisterFull = 3 };
 // its scores (the register-staged V^T form masks every block).
 // PV8: e4m3 K/V take the second product on the fp8 matrix cores (see the comment at the top).
 // VD8: with PV8, V^T takes direct loads for full blocks (e4m3 rows of 16-byte aligned runs).
-// SPLIT: the workgroup walks a range of the line of key blocks (see split_plan), one unit's part after the other.
+// SPLIT: the workgroup walks the pieces of a unit that split_item gives it, else all of them (key_split.hpp).
 template <bool FP8, bool VT, int STAGING, int DT, bool ONES, bool KMASK = false, bool PV8 = false, bool VD8 = false,
           bool SPLIT = false>
 __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void xattn_fwd_kernel(XattnParams p) {
@@ -687,28 +662,13 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   const int64_t wg = blockIdx.x;
   int qt;
   int64_t unit = 0;
-  // SPLIT: the rest of the team's range, [pos, range_end) of the line.
-  [[maybe_unused]] int team = 0, pos = 0, range_end = 0;
-  [[maybe_unused]] __shared__ int s_before[SPLIT ? kSplitMaxWindows : 1], s_blocks[SPLIT ? kSplitMaxWindows : 1];
-  [[maybe_unused]] __shared__ int s_total, s_teams;
+  [[maybe_unused]] int team = 0;
+  [[maybe_unused]] SplitItem item = {};
   if constexpr (SPLIT) {
     const int seq = static_cast<int>(wg >> 3);
     qt = seq % p.q_tiles;
     team = (seq / p.q_tiles) * kXcds + static_cast<int>(wg & 7);
-    const SplitPlan plan = split_plan(p);
-    if (team >= plan.teams) return;
-    pos = split_cut(p, plan, team);
-    range_end = split_cut(p, plan, team + 1);
-    if (pos >= range_end) return;
-    if (threadIdx.x < kSplitMaxWindows) {
-      s_before[threadIdx.x] = plan.before;
-      s_blocks[threadIdx.x] = plan.blocks;
-    }
-    if (threadIdx.x == 0) {
-      s_total = plan.total;
-      s_teams = plan.teams;
-    }
-    __syncthreads();
+    if (!split_item(p, split_plan(p), team, item)) return;
   } else if ((p.B * p.H) % 8 == 0) {
     const int64_t seq = wg >> 3;
     qt = static_cast<int>(seq % p.q_tiles);
@@ -724,9 +684,9 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     qt = static_cast<int>(wg % p.q_tiles);
     unit = wg / p.q_tiles;
   }
-  int64_t h = unit % p.H;
+  const int64_t h = SPLIT ? item.h : unit % p.H;
   const int64_t rank = unit / p.H;
-  int64_t b = rank;
+  int64_t b = SPLIT ? item.b : rank;
   if (!SPLIT && p.B > 1 && p.B <= kMaxRankWindows) {
     // The window whose (length desc, index asc) rank is `rank`: every thread ranks its candidate windows.
     for (int64_t c = threadIdx.x; c < p.B; c += kThreads) {
@@ -742,41 +702,12 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     b = s_window;
   }
 
-  do {
-  // SPLIT: the thread index is opaque in every part of the range, or the compiler would form the addresses of the
-  // parts' beginning and end once, outside this loop, and hold them in registers through the key blocks (88 spilled).
-  // (Elsewhere threadIdx.x itself, whose known range a variable that the lambdas capture does not carry: ten more
-  // instructions a block in the register-staged forms.)
-  [[maybe_unused]] int part_tid = threadIdx.x;
-  if constexpr (SPLIT) asm volatile("" : "+v"(part_tid));
-#define SVHIP_TID (SPLIT ? part_tid : static_cast<int>(threadIdx.x))
-  const int lane = SVHIP_TID & 63;
-  const int w = __builtin_amdgcn_readfirstlane(SVHIP_TID >> 6);
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 31;  // query column within the wave
   const int hh = lane >> 5;   // lane half
   const int64_t q = static_cast<int64_t>(qt) * kQTile + w * 32 + col;
   const bool q_ok = q < p.Q;
-  // Key blocks [blk0, blk1) of the unit (b, h): all of them, or the range's part of the unit.
-  int blk0 = 0;
-  [[maybe_unused]] int blk1 = 0, unit_blocks = 0;
-  if constexpr (SPLIT) {
-    SplitPlan plan;
-    plan.before = s_before[lane];
-    plan.blocks = s_blocks[lane];
-    const int bw = split_window(p, plan, pos);
-    unit_blocks = __builtin_amdgcn_readlane(plan.blocks, bw);
-    const int rel = pos - static_cast<int>(p.H) * __builtin_amdgcn_readlane(plan.before, bw);
-    const int hw = __builtin_amdgcn_readfirstlane(rel / unit_blocks);
-    b = bw;
-    h = hw;
-    blk0 = rel - hw * unit_blocks;
-    blk1 = min(unit_blocks, blk0 + (range_end - pos));
-    pos += blk1 - blk0;
-    if (blk0 == 0 && qt == 0 && SVHIP_TID == 0) {
-      split_units(p)[b * p.H + h] =
-          split_unit_teams(team, pos - blk1, unit_blocks, blk1 == unit_blocks, s_total, s_teams);
-    }
-  }
   const int64_t off = p.cu_seqlens ? p.cu_seqlens[b] : 0;
   const int L = [&]() __attribute__((always_inline)) {
     const int n = window_length(p, b);
@@ -788,7 +719,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
       // With a key mask the window ends at its last attended key: the blocks after it add nothing to O, l or m.
       // One scan of the window's mask row (a wave-uniform result; no attended key gives L = 0 and zeros).
       __shared__ int s_last;
-      if (SVHIP_TID == 0) s_last = -1;
+      if (threadIdx.x == 0) s_last = -1;
       __syncthreads();
       const int last = last_attended(p.kv_mask + b * p.sm_b, n);
       if (last >= 0) atomicMax(&s_last, last);
@@ -807,7 +738,8 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   }
   const float sl2 = p.scale_log2 * kscale;   // scores -> log2 units
 
-  if (!SPLIT && L == 0) {  // (a part of the line always holds keys)
+  if (L == 0) {
+    if constexpr (SPLIT) split_publish(p, item, team, qt);
     if (q_ok) {
       for (int d = hh; d < p.D; d += 2) Op[q * p.so_q + d] = 0;
     }
@@ -832,33 +764,59 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   // V^T rows allow vector loads when every 8-key run starts aligned (the base, the row stride and the offset).
   const bool vt_vec = VT && ((reinterpret_cast<uintptr_t>(V) & (FP8 ? 7 : 15)) == 0) && (p.sv_d % 8 == 0);
   const int nfull = L / kKB;           // full key blocks
-  // End of this part's full blocks, and whether the unit's last, partial block follows.
   const bool partial = nfull * kKB < L;
-  const int full_end = SPLIT ? min(blk1, unit_blocks - (partial ? 1 : 0)) : nfull;
-  const bool tail = SPLIT ? partial && blk1 == unit_blocks : partial;
+  // An e4m3 cache's windows are never cut: its kernels walk them as one piece.
+  constexpr bool PIECES = !FP8;
   // LIST: block i of the unit is the i-th of the window's blocks with an attended key.
   constexpr bool LIST = SPLIT && KMASK;
+  [[maybe_unused]] const int unit_blocks = (L + kKB - 1) / kKB;
+  [[maybe_unused]] const Pieces pieces =
+      PIECES ? pieces_of(unit_blocks, p.H, p.lone, kPieceBlocks) : Pieces{unit_blocks, unit_blocks, 1};
+  [[maybe_unused]] const int piece_end = SPLIT ? item.end : pieces.count;  // the walk's pieces end here
+  [[maybe_unused]] int piece = SPLIT ? item.first : 0;               // the current one
+  // First block of the next piece of the walk; none: past every block.
+  [[maybe_unused]] auto next_piece = [&]() __attribute__((always_inline)) -> int {
+    return piece + 1 < piece_end ? piece_start(pieces, piece + 1) : 0x7fffffff;
+  };
+  [[maybe_unused]] int bound = PIECES ? next_piece() : 0;
+  // The walk: blocks [blk0, blk1) (of the list), the last one a partial block where `tail`.
+  int blk0 = 0, blk1 = unit_blocks;
+  [[maybe_unused]] int listed = 0;
+  if constexpr (LIST) {
+    listed = __builtin_amdgcn_readfirstlane(p.kv_blocks[b * p.sb_b]);
+    blk0 = listed_before(p, b, listed, piece_start(pieces, item.first));
+    blk1 = listed_before(p, b, listed, piece_start(pieces, item.end));
+  } else if constexpr (SPLIT) {
+    blk0 = piece_start(pieces, item.first);
+    blk1 = piece_start(pieces, item.end);
+  }
+  const bool tail = partial && (LIST ? blk1 == listed : blk1 == unit_blocks);
+  const int full_end = blk1 - (tail ? 1 : 0);
   auto key_of = [&](int i) __attribute__((always_inline)) -> int {
     if constexpr (LIST) {
-      return kKB * listed_block(p, b, min(i, unit_blocks - 1));
+      return kKB * listed_block(p, b, min(i, listed - 1));
     } else {
       return kKB * i;
     }
   };
   [[maybe_unused]] int kv_cur = 0, kv_next = 0;  // LIST: first keys of the current and the next block
-  if constexpr (LIST) {
+  if (LIST && blk0 < blk1) {
     kv_cur = key_of(blk0);
     kv_next = key_of(blk0 + 1);
+    while (kv_cur / kKB >= bound) {  // pieces without a listed block add nothing
+      ++piece;
+      bound = next_piece();
+    }
   }
 
   DirectLanes<DT> dl;
   if constexpr (DIRECT) {
     dl = direct_lanes<DT>(p, reinterpret_cast<const uint16_t*>(K), reinterpret_cast<const uint16_t*>(V), dchunks, nfull,
-                      w, lane);
+                      w);
     if (STAGING == kDirect && dchunks < 4 * DT) {
       // Chunks past head_dim of the K tiles that the score product reads are never loaded by direct loads; they
       // must hold zeros.
-      for (int i = SVHIP_TID; i < kSubTiles * kKB * 8; i += kThreads) {
+      for (int i = threadIdx.x; i < kSubTiles * kKB * 8; i += kThreads) {
         const int u = i / (kKB * 8), R = (i >> 3) % kKB, c = i & 7;
         if (8 * u + c >= dchunks) {
           const int e = u * kKTile + R * kRow + swz(R, c) * 8;
@@ -870,7 +828,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     if constexpr (VROWS) {
       // Direct loads never write the chunks of V rows past head_dim: zeros, and with ONES the ones column D.
       if (dchunks < 8 * kSubTiles) {
-        for (int i = SVHIP_TID; i < kSubTiles * kKB * 8; i += kThreads) {
+        for (int i = threadIdx.x; i < kSubTiles * kKB * 8; i += kThreads) {
           const int u = i / (kKB * 8), R = (i >> 3) % kKB, c = i & 7;
           if (8 * u + c >= dchunks) {
             const int e = u * kKTile + R * kRow + swzv(R, c) * 8;
@@ -880,23 +838,23 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
           }
         }
       }
-    } else if (ONES && SVHIP_TID < 16) {
+    } else if (ONES && threadIdx.x < 16) {
       // Direct loads never write V^T rows >= D: row D of both buffers holds ones for the whole kernel.
-      const int R = static_cast<int>(p.D), c = SVHIP_TID & 7;
-      uint16_t* buf = SVHIP_TID < 8 ? sV0 : sV1;
+      const int R = static_cast<int>(p.D), c = threadIdx.x & 7;
+      uint16_t* buf = threadIdx.x < 8 ? sV0 : sV1;
       *reinterpret_cast<uint4*>(buf + R * kRow + swz(R, c) * 8) = raw_one<false>();
     }
   }
   [[maybe_unused]] DirectRows<DT> dr;
   if constexpr (DIRECT && VROWS) {
-    dr = direct_rows<DT>(p, reinterpret_cast<const uint16_t*>(V), dchunks, nfull, w, lane);
+    dr = direct_rows<DT>(p, reinterpret_cast<const uint16_t*>(V), dchunks, nfull, w);
   }
 
   [[maybe_unused]] DirectV8<DT> dv;
   if constexpr (VD8) {
     dv = direct_v8<DT>(p, reinterpret_cast<const uint8_t*>(V), nfull, w);
     // V^T rows D .. 32 DT - 1 of both tiles, which direct loads never write: zeros (row D ones with ONES).
-    for (int i = SVHIP_TID; i < (32 * DT - Dv) * 4; i += kThreads) {
+    for (int i = threadIdx.x; i < (32 * DT - Dv) * 4; i += kThreads) {
       const int R = Dv + (i >> 2), c = i & 3;
       const uint32_t x = (ONES && R == Dv) ? 0x38383838u : 0u;  // e4m3 1.0
       *reinterpret_cast<uint4*>(reinterpret_cast<uint8_t*>(sV0) + R * kRow8 + c * 16) = make_uint4(x, x, x, x);
@@ -959,24 +917,98 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   }
   f32x16_t o[DT];  // O^T tiles: d in [32 j, 32 j + 32)
 #pragma unroll
-  for (int j = 0; j < DT; ++j) {
-    if constexpr (SPLIT) {
-      float zero = 0.f;
-      asm volatile("" : "+v"(zero));  // no register tuple of zeros kept for the next part
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[j][i] = zero;
-    } else {
-      o[j] = f32x16_t{0};
-    }
-  }
+  for (int j = 0; j < DT; ++j) o[j] = f32x16_t{0};
   // Stored running max (log2 units), shared by O and l.
-  float m = SPLIT && !KMASK && blk0 > 0 ? kPartMax : -INFINITY;
+  float m = SPLIT && !KMASK && piece > 0 ? kPieceMax : -INFINITY;
   float l = 0.f;                // MSUM: query c's row sum in lane c (lanes 32-63 hold 0)
-  bool first = true;            // uniform: the window's first half always takes the max
+  bool first = true;            // uniform: a piece's first half always takes the max
   // KMASK: the lane's query has seen no attended key yet (m is then a placeholder 0, O and l are 0); every half
   // takes the max while any lane of the wave is in that state, so the first half with an attended key sets m to
   // that key's score however far below 0 it lies.
   [[maybe_unused]] bool placeholder = false;
+
+  // The pieces walked before the current one, joined, 4 DT + 1 quads a lane: the first kJoinLds in LDS (as many as
+  // leave the CU its workgroups), the next in registers (direct forms up to head_dim 96), the rest in scratch memory
+  // behind an opaque address (or the compiler would keep it in registers). 8 windows x 12 heads, 4 to 8 pieces each:
+  // 225 us in one piece, 230 so, 261 with all of it in scratch memory (31 MB, which miss the L2s).
+  constexpr int kQuads = 4 * DT + 1;
+  constexpr int kJoinLds = DT == 2 ? 5 : (DT == 3 && VT ? 5 : 3);
+  constexpr int kJoinReg = DIRECT && DT < 4 ? kQuads - kJoinLds : 0;
+  __shared__ __attribute__((aligned(16))) f32x4_t s_joined[PIECES ? kJoinLds : 1][PIECES ? kThreads : 1];
+  [[maybe_unused]] f32x4_t r_joined[kJoinReg ? kJoinReg : 1];
+  [[maybe_unused]] f32x4_t joined[PIECES ? kQuads - kJoinLds - kJoinReg + 1 : 1];
+  [[maybe_unused]] bool folded = false;  // uniform: the quads hold pieces
+  typedef __attribute__((address_space(5))) f32x4_t* joined_t;
+  [[maybe_unused]] auto joined_at = [&]() __attribute__((always_inline)) {
+    uint32_t at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((joined_t)joined));
+    asm volatile("" : "+v"(at));
+    return (joined_t)(static_cast<uintptr_t>(at));
+  };
+  [[maybe_unused]] auto get_joined = [&](f32x4_t(&at)[kQuads]) __attribute__((always_inline)) {
+    const joined_t from = kQuads > kJoinLds + kJoinReg ? joined_at() : nullptr;
+#pragma unroll
+    for (int i = 0; i < kQuads; ++i) {
+      if (i < kJoinLds) {
+        at[i] = s_joined[i][threadIdx.x];
+      } else if (i < kJoinLds + kJoinReg) {
+        at[i] = r_joined[i - kJoinLds];
+      } else {
+        at[i] = from[i - kJoinLds - kJoinReg];
+      }
+    }
+  };
+  [[maybe_unused]] auto set_joined = [&](const f32x4_t(&at)[kQuads]) __attribute__((always_inline)) {
+    const joined_t to = kQuads > kJoinLds + kJoinReg ? joined_at() : nullptr;
+#pragma unroll
+    for (int i = 0; i < kQuads; ++i) {
+      if (i < kJoinLds) {
+        s_joined[i][threadIdx.x] = at[i];
+      } else if (i < kJoinLds + kJoinReg) {
+        r_joined[i - kJoinLds] = at[i];
+      } else {
+        to[i - kJoinLds - kJoinReg] = at[i];
+      }
+    }
+  };
+  // The current piece joined to the ones before it: m, l and O are the walk's so far.
+  [[maybe_unused]] auto join = [&]() __attribute__((always_inline)) {
+    if (KMASK && placeholder) m = -INFINITY;  // no attended key in the piece
+    if (!folded) return;
+    f32x4_t at[kQuads];
+    get_joined(at);
+    const f32x4_t ml = at[4 * DT];
+    float x, y, mn = ml[0];
+    join_factors(mn, m, x, y);
+    m = mn;
+    l = join_value(ml[1], l, x, y);
+#pragma unroll
+    for (int j = 0; j < DT; ++j) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[j][i] = join_value(at[4 * j + i / 4][i % 4], o[j][i], x, y);
+    }
+  };
+  // A piece has ended inside the walk (the next block is block `next`): start the one that holds the next block.
+  [[maybe_unused]] auto fold = [&](int next) __attribute__((always_inline)) {
+    join();
+    f32x4_t at[kQuads];
+#pragma unroll
+    for (int j = 0; j < DT; ++j) {
+#pragma unroll
+      for (int i = 0; i < 16; i += 4) at[4 * j + i / 4] = f32x4_t{o[j][i], o[j][i + 1], o[j][i + 2], o[j][i + 3]};
+      o[j] = f32x16_t{0};
+    }
+    at[4 * DT] = f32x4_t{m, l, 0.f, 0.f};
+    set_joined(at);
+    m = KMASK ? -INFINITY : kPieceMax;
+    l = 0.f;
+    first = true;
+    placeholder = false;
+    folded = true;
+    do {
+      ++piece;
+      bound = next_piece();
+    } while (LIST && next >= bound);
+  };
 
   // The full block at key kv0 into (sK, sV): issued now, complete at the next vmem wait (direct) or at `stage_commit`
   // (registers, prefetched into `st`).
@@ -987,7 +1019,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
                                                    static_cast<uint32_t>(kv0 * 2), w, sK, sV);
       if constexpr (VROWS) stage_rows<DT, STAGING == kDirectFull>(dr, static_cast<uint32_t>(kv0 * p.sv_k * 2), w, sV);
     } else {
-      stage_load<FP8, VT, DT, false, ONES, !VD8>(st, p, K, V, L, kv0, dchunks, vt_vec, SVHIP_TID);
+      stage_load<FP8, VT, DT, false, ONES, !VD8>(st, p, K, V, L, kv0, dchunks, vt_vec);
       if constexpr (VD8) {
 #pragma unroll
         for (int t = 0; t < (2 * DT + 3) / 4; ++t) {
@@ -998,13 +1030,13 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     }
   };
   auto stage_commit = [&](uint16_t* sK, uint16_t* sV) __attribute__((always_inline)) {
-    if constexpr (!DIRECT) stage_store<FP8, VT, DT, ONES, PV8, !VD8>(st, sK, sV, dchunks, Dv, SVHIP_TID);
+    if constexpr (!DIRECT) stage_store<FP8, VT, DT, ONES, PV8, !VD8>(st, sK, sV, dchunks, Dv);
   };
   // The partial block, synchronously through registers.
   auto stage_tail = [&](uint16_t* sK, uint16_t* sV) __attribute__((always_inline)) {
     Stage<FP8, VT, DT> tmp;
-    stage_load<FP8, VT, DT, true, ONES>(tmp, p, K, V, L, nfull * kKB, dchunks, vt_vec, SVHIP_TID);
-    stage_store<FP8, VT, DT, ONES, PV8>(tmp, sK, sV, dchunks, Dv, SVHIP_TID);
+    stage_load<FP8, VT, DT, true, ONES>(tmp, p, K, V, L, nfull * kKB, dchunks, vt_vec);
+    stage_store<FP8, VT, DT, ONES, PV8>(tmp, sK, sV, dchunks, Dv);
   };
 
 
@@ -1020,7 +1052,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
       mask_byte = mrow[min(kv0 + lane, L - 1)];
     }
   };
-  mask_fetch(key_of(blk0));
+  if (!LIST || blk0 < blk1) mask_fetch(key_of(blk0));
   auto block_bits = [&](int next_kv0) __attribute__((always_inline)) -> uint64_t {
     if constexpr (KMASK) {
       const uint64_t bits = __builtin_amdgcn_ballot_w64(mask_byte != 0 && mask_kv0 + lane < L);
@@ -1374,7 +1406,8 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   // are taken, and the next block's mask bytes fetched, before the next block's loads are issued: the wait for the
   // mask bytes (loaded during the previous block, waited for at its end) then waits for nothing in flight, where
   // after those loads it waited for them all.
-  auto full_step = [&](int blk, const uint16_t* Ks, const uint16_t* Vt, uint16_t* nK, uint16_t* nV) __attribute__((always_inline)) {
+  auto full_step = [&](int blk, const uint16_t* Ks, const uint16_t* Vt, uint16_t* nK, uint16_t* nV)
+      __attribute__((always_inline)) {
     const int kv0 = LIST ? kv_cur : blk * kKB, next = LIST ? kv_next : (blk + 1) * kKB;
     [[maybe_unused]] int after = 0;
     if constexpr (LIST) after = key_of(blk + 2);
@@ -1391,25 +1424,37 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
     SVHIP_TRACE(trace.block_end(blk, lane);)
   };
 
-  if (full_end > blk0) {
-    stage_issue(key_of(blk0), sK0, sV0);
-    stage_commit(sK0, sV0);
-  } else {
-    stage_tail(sK0, sV0);
-  }
-  wait_vmem();
-  __syncthreads();
-  int blk = blk0;
-  for (; blk + 2 < full_end; blk += 2) {
-    full_step(blk, sK0, sV0, sK1, sV1);
-    full_step(blk + 1, sK1, sV1, sK0, sV0);
-  }
-  if (blk + 1 < full_end) {
-    full_step(blk, sK0, sV0, sK1, sV1);
-    ++blk;
-  }
-  // blk is the last full block (or blk0 with no full block); its tiles are the ones of its parity.
-  {
+  // With a list, pieces end between any two blocks of it; else with the second block of a pair (piece_start is even).
+  [[maybe_unused]] auto list_fold = [&]() __attribute__((always_inline)) {
+    if (LIST && kv_cur >= kKB * static_cast<int64_t>(bound)) fold(kv_cur / kKB);
+  };
+  if (!LIST || blk0 < blk1) {
+    if (full_end > blk0) {
+      stage_issue(key_of(blk0), sK0, sV0);
+      stage_commit(sK0, sV0);
+    } else {
+      stage_tail(sK0, sV0);
+    }
+    wait_vmem();
+    __syncthreads();
+    int blk = blk0;
+    for (;;) {
+      const int stop = PIECES && !LIST ? min(bound, full_end - 1) : full_end - 1;
+      for (; blk + 2 <= stop; blk += 2) {
+        full_step(blk, sK0, sV0, sK1, sV1);
+        list_fold();
+        full_step(blk + 1, sK1, sV1, sK0, sV0);
+        list_fold();
+      }
+      if (!PIECES || LIST || bound >= full_end) break;
+      fold(blk);
+    }
+    if (blk + 1 < full_end) {
+      full_step(blk, sK0, sV0, sK1, sV1);
+      list_fold();
+      ++blk;
+    }
+    // blk is the last full block (or blk0 with no full block); its tiles are the ones of its parity.
     const bool odd = (blk - blk0) & 1;
     uint16_t* cK = odd ? sK1 : sK0;
     uint16_t* cV = odd ? sV1 : sV0;
@@ -1421,11 +1466,15 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
       const int kv0 = LIST ? kv_cur : blk * kKB;
       const uint64_t bits = block_bits(LIST ? kv_next : kv0 + kKB);
       Stage<FP8, VT, DT> tl;
-      if (tail) stage_load<FP8, VT, DT, true, ONES>(tl, p, K, V, L, nfull * kKB, dchunks, vt_vec, SVHIP_TID);
+      if (tail) stage_load<FP8, VT, DT, true, ONES>(tl, p, K, V, L, nfull * kKB, dchunks, vt_vec);
       compute(Full{}, cK, cV, kv0, bits);
       settle();
       if (tail) {
-        stage_store<FP8, VT, DT, ONES, PV8>(tl, nK, nV, dchunks, Dv, SVHIP_TID);
+        if constexpr (LIST) {
+          kv_cur = nfull * kKB;
+          list_fold();
+        }
+        stage_store<FP8, VT, DT, ONES, PV8>(tl, nK, nV, dchunks, Dv);
         wait_vmem();
         __syncthreads();
         compute(Partial{}, nK, nV, nfull * kKB, block_bits(L));
@@ -1436,6 +1485,7 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
       settle();
     }
   }
+  if constexpr (PIECES) join();
 
   float lsum = l;
   if constexpr (ONES) {
@@ -1464,11 +1514,10 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
   }
   SVHIP_TRACE(trace.end(lane, lsum);)
   if constexpr (SPLIT) {
-    if (blk1 - blk0 < unit_blocks) {
-      // A part of the unit: O as it stands, [head_dim / 4][query][4], then m and l, [2][query]; under a key
-      // mask a query that has seen no attended key (l = 0) carries m = -inf.
-      float* slot = p.part + (static_cast<int64_t>(2 * team + (blk0 == 0 ? 1 : 0)) * p.q_tiles + qt) *
-                                 split_slot_floats(p.D);
+    split_publish(p, item, team, qt);
+    if (item.first > 0 || item.end < pieces.count) {
+      // Not the whole unit: O as it stands, [head_dim / 4][query][4], then m and l, [2][query].
+      float* slot = split_slot(p, team, qt);
       const int ql = w * 32 + col;
 #pragma unroll
       for (int t = 0; t < DT; ++t) {
@@ -1481,11 +1530,10 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
         }
       }
       if (hh == 0) {
-        slot[kQTile * p.D + ql] = KMASK && lsum == 0.f ? -INFINITY : m;
+        slot[kQTile * p.D + ql] = m;
         slot[kQTile * (p.D + 1) + ql] = lsum;
       }
-      __syncthreads();  // the next part stages into the tiles
-      continue;
+      return;
     }
   }
   // A query with no attended key (only possible with a key mask) has l = 0 and O = 0: it gets zeros.
@@ -1512,9 +1560,6 @@ __global__ __launch_bounds__(kThreads, (DT == 2 && (VT || !PV8)) ? 3 : 2) void x
       }
     }
   }
-  if constexpr (SPLIT) __syncthreads();  // the next part stages into the tiles
-  } while (SPLIT && pos < range_end);
-#undef SVHIP_TID
 #endif  // __HIP_DEVICE_COMPILE__
 }
 

@@ -194,7 +194,7 @@ def _attention_f32(query, key, val, lengths, cu_seqlens, scale, out, key_mask=No
     ws = torch.empty(nbytes, dtype=torch.uint8, device=query.device) if nbytes else None
     mask = None if key_mask is None else key_mask.view(torch.uint8)
     blocks = None
-    if mask is not None and nbytes and B > 1:
+    if mask is not None and nbytes:
         lengths, blocks = _attended_blocks(key_mask, lengths, cu_seqlens, mask_cap)
     _lib.check(lib.svhip_xattn_fwd_f32_ws(
         _lib.ptr(query), _lib.ptr(key), _lib.ptr(val), _lib.ptr(out), _lib.ptr(mask),

@@ -2,6 +2,7 @@
 host-side argument checks reject bad input without touching a GPU."""
 import ctypes
 import os
+import random
 import re
 
 import pytest
@@ -79,6 +80,48 @@ def test_masked_attention_checks_the_block_lists_on_the_host(lib):
         assert call(3, lengths=None) == 0        # lists without their lengths are not used
     assert fp32(4, mask=None, cu=p) == -1 and b'exclusive' in lib.svhip_last_error()
     assert fp32(4, blocks=None, cu=p) == -1 and b'exclusive' in lib.svhip_last_error()
+
+
+def _pieces(blocks, heads, lone, least):
+    """(blocks a piece, pieces) of a window of the cross attention: an equal share of the window alone a piece, even, at
+    least `least` blocks and a sixteenth of the window; a last piece of half of `least` or more by itself."""
+    if blocks < 24:
+        return blocks, 1
+    each = max(-(-blocks * heads // lone), least, -(-blocks // 16))
+    if each >= blocks:
+        return blocks, 1
+    each += each % 2
+    full, rest = divmod(blocks, each)
+    return each, max(1, full + (2 * rest >= least))
+
+
+@pytest.mark.parametrize('fp32', [False, True])
+def test_attention_workspace_holds_every_plan(lib, fp32):
+    """The scratch of the key split has a slot for every part of every plan: a team's slot for each window and head, and
+    one for each piece past the window's share (an equal share of all windows' blocks for each resident team)."""
+    g = random.Random(7)
+    seen = 0
+    for _ in range(4000):
+        windows, heads, queries = g.randint(1, 24), g.randint(1, 16), g.choice([1024, g.randint(1, 3000)])
+        width = g.choice([16, 32, 48, 64]) if fp32 else 8 * g.randint(1, 16)
+        cap = g.randint(24, 300)
+        blocks = [cap] + [g.choice([cap, g.randint(0, cap)]) for _ in range(windows - 1)]
+        query = lib.svhip_xattn_f32_workspace_bytes if fp32 else lib.svhip_xattn_workspace_bytes
+        nbytes = query(windows, heads, queries, width, 64 * cap)
+        if nbytes == 0:
+            continue
+        seen += 1
+        tiles = -(-queries // 128)
+        slots = (nbytes - 16 * windows * heads) // (tiles * 128 * (width + 2) * 4)
+        resident = 8 * (32 * (3 if width <= 64 and not fp32 else 2) // tiles)
+        share = sum(blocks) * heads // resident
+        need = 0
+        for n in blocks:
+            each, count = _pieces(n, heads, max(1, 512 // tiles), 6 if fp32 else 12)
+            lead = count if share >= n else min(count, max(1, share // each))
+            need += heads * (1 + count - lead)
+        assert need <= slots, (windows, heads, queries, width, blocks)
+    assert seen > 500
 
 
 def test_noalloc_select_rejects_on_the_host(lib):

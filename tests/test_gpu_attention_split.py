@@ -116,6 +116,69 @@ def test_e4m3_is_not_split(dev, vt):
         assert torch.equal(one, out[b:b + 1])
 
 
+def check_alone_and_in_batches(dev, q, k, v, lengths, batches):
+    """Every window of `lengths` attended alone and in each of `batches` (lists of window indices): the same bits, as
+    rows of padded K/V and under the key mask of the same lengths."""
+    from streamvoxel_amd.stream.attention import attention
+    lt = torch.tensor(lengths, dtype=torch.int32, device=dev)
+    mask = torch.arange(k.shape[2], device=dev)[None] < lt[:, None]
+    alone = [attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], lengths=lt[b:b + 1]) for b in range(len(lengths))]
+    for at in [[b] for b in range(len(lengths))] + batches:
+        out = attention(q[at], k[at], v[at], lengths=lt[at])
+        out_m = attention(q[at], k[at], v[at], key_mask=mask[at])
+        torch.cuda.synchronize()
+        for i, b in enumerate(at):
+            assert torch.equal(out[i:i + 1], alone[b]), (at, b)
+            assert torch.equal(out_m[i:i + 1], alone[b]), ('mask', at, b)
+
+
+# Lengths short of the first cut, on it, at and past the piece counts that follow, with and without a partial block.
+ALONE = [EDGE - 64, EDGE - 63, EDGE + 130, 0, 30 * 64, 4097, 6400, 63]
+# Batches: some, with repetitions that fill the chip (unsplit) or go past one wave's windows (unsplit).
+BATCHES = [[0, 1], [2, 4, 6], list(range(8)), list(range(8)) * 6, list(range(8)) * 9]
+
+
+@pytest.mark.parametrize('D,H,Q', [(48, 8, 1000), (64, 6, 1024), (96, 4, 700), (128, 2, 130), (64, 1, 20), (48, 2, 3300)])
+@pytest.mark.parametrize('vt', [False, True])
+def test_bf16_windows_alone_and_in_batches(dev, D, H, Q, vt):
+    """Where a window is cut depends on itself alone: the same bits alone, in split batches of several sizes and in
+    batches that are not split, over either V layout (head counts and query tiles for 16, 12, 8 pieces and none)."""
+    _case(f'bf16 alone and in batches D={D} H={H} Q={Q} vt={vt}')
+    q, k, v = (x.to(dev) for x in qkv(8, H, Q, 6400, D, D + H, torch.bfloat16, 2.0))
+    if vt:
+        v = v.transpose(2, 3).contiguous().transpose(2, 3)
+    check_alone_and_in_batches(dev, q, k, v, ALONE, BATCHES[:4] if Q > 2000 else BATCHES)
+
+
+@pytest.mark.parametrize('D,H,Q', [(16, 3, 130), (48, 8, 500), (64, 12, 1024)])
+def test_fp32_windows_alone_and_in_batches(dev, D, H, Q):
+    _case(f'fp32 alone and in batches D={D} H={H} Q={Q}')
+    q, k, v = (x.to(dev) for x in qkv(8, H, Q, 6400, D, D + H, torch.float32, 2.0))
+    check_alone_and_in_batches(dev, q, k, v, ALONE, BATCHES)
+
+
+@pytest.mark.parametrize('dtype', ['bf16', 'fp32'])
+def test_windows_under_masks_with_holes_alone_and_in_batches(dev, dtype):
+    """The same under masks that leave out whole pieces, the window's end and every second block."""
+    from streamvoxel_amd.stream.attention import attention
+    H, Q, D, kcap = 6, 512, 64, 6000
+    _case(f'masks alone and in batches {dtype}')
+    q, k, v = (x.to(dev) for x in qkv(6, H, Q, kcap, D, 7, torch.bfloat16 if dtype == 'bf16' else torch.float32, 2.0))
+    mask = torch.rand(6, kcap, generator=torch.Generator().manual_seed(4)) < 0.5
+    mask[0, 200:4000] = False
+    mask[1] = False
+    mask[2, :5900] = False
+    mask[3, 2500:] = False
+    mask[4] = (torch.arange(kcap) // 64) % 2 == 1
+    mask = mask.to(dev)
+    alone = [attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], key_mask=mask[b:b + 1]) for b in range(6)]
+    for at in ([0, 4], list(range(6)), list(range(6)) * 4, list(range(6)) * 12):
+        out = attention(q[at], k[at], v[at], key_mask=mask[at])
+        torch.cuda.synchronize()
+        for i, b in enumerate(at):
+            assert torch.equal(out[i:i + 1], alone[b]), (at, b)
+
+
 @pytest.mark.parametrize('lengths', LENGTHS, ids=lambda x: '-'.join(map(str, x)))
 @pytest.mark.parametrize('D', [16, 32, 48, 64])
 def test_split_fp32_windows_match_the_oracle(dev, lengths, D):
@@ -131,8 +194,9 @@ def test_split_fp32_windows_match_the_oracle(dev, lengths, D):
     out_t = attention(qd, kd, vd.transpose(2, 3).contiguous().transpose(2, 3), lengths=lt)
     out_m = attention(qd, kd, vd, key_mask=torch.arange(kcap, device=dev)[None] < lt[:, None])
     torch.cuda.synchronize()
-    for x in (out, out_t, out_m):
-        check(x, ref, 2e-5, 1e-4)
+    check(out, ref, 2e-5, 1e-4)
+    # Every layout of the same keys is cut alike and gives the same bits.
+    assert torch.equal(out, out_t) and torch.equal(out, out_m)
 
 
 def test_split_replays_in_a_graph(dev):
