@@ -23,6 +23,7 @@ constexpr int kEmbedThreads = 256;
 constexpr int kEmbedSlices = 8;         // column slices, one per XCD
 constexpr int kEmbedBatch = 8;          // table loads a lane has in flight
 constexpr int kEmbedMaxTokens = 64;     // patch tokens per workgroup
+constexpr int64_t kEmbedGroups = 1 << 20;  // token groups per launch (a launch holds fewer than 2^32 threads)
 constexpr int kEmbedMaxOffsets = 64;    // p^3 up to 4^3
 constexpr int kEmbedMaxWidth = 2048;
 
@@ -36,20 +37,21 @@ struct EmbedArgs {
   int* bad;               // set when a token lies outside [0, cells)
   int slice_chunks;       // 16-byte chunks of a column slice
   int wg_tokens;          // patch tokens of a workgroup: kEmbedThreads / slice_chunks, at most kEmbedMaxTokens
+  uint32_t first_group;   // token group of the launch's first workgroups
 };
 
 // P: the patch edge 4 at compile time (the index arithmetic of the table rows is a third of the work otherwise), or 0.
-template <int P>
+// WIDE: the table holds 2^32 16-byte chunks or more.
+template <int P, bool WIDE>
 __global__ __launch_bounds__(kEmbedThreads) void patch_embed_kernel(EmbedArgs a) {
-  // Table row of every (token, offset); offsets past p^3 are never read.
-  // (in 16-byte units).
+  // First 16-byte chunk (WIDE: the index) of every (token, offset)'s table row; offsets past p^3 are never read.
   __shared__ __attribute__((aligned(16))) uint32_t s_row[kEmbedMaxTokens][kEmbedMaxOffsets + 4];
   __shared__ int64_t s_base[kEmbedMaxTokens];  // element of every token's first voxel
   const int p = P ? P : static_cast<int>(a.p), p3 = p * p * p;
   const uint32_t gx = static_cast<uint32_t>(a.X / p), gzx = static_cast<uint32_t>(a.Z / p) * gx;
   const uint32_t per_window = static_cast<uint32_t>(a.Y / p) * gzx;  // B per_window < 2^31 (checked by the host)
   const int slice = static_cast<int>(blockIdx.x % kEmbedSlices);
-  const uint32_t first = blockIdx.x / kEmbedSlices * a.wg_tokens;  // flat (b, n) of token 0
+  const uint32_t first = (a.first_group + blockIdx.x / kEmbedSlices) * a.wg_tokens;  // flat (b, n) of token 0
   const int chunks = static_cast<int>(a.W / 8);
   const int chunk0 = slice * a.slice_chunks;
   if (chunk0 >= chunks) return;
@@ -70,13 +72,16 @@ __global__ __launch_bounds__(kEmbedThreads) void patch_embed_kernel(EmbedArgs a)
       atomicOr(a.bad, 1);
       cell = 0;
     }
-    s_row[t][o] = (static_cast<uint32_t>(cell) * p3 + o) * row_units;
+    s_row[t][o] = (static_cast<uint32_t>(cell) * p3 + o) * (WIDE ? 1u : row_units);
   }
   __syncthreads();
   const int t = static_cast<int>(threadIdx.x) / a.slice_chunks;
   const int ch = chunk0 + static_cast<int>(threadIdx.x) % a.slice_chunks;
   if (t >= count || ch >= chunks) return;
   const uint4* base = reinterpret_cast<const uint4*>(a.table) + ch;
+  auto chunk = [&](uint32_t row) __attribute__((always_inline)) -> const uint4& {
+    return base[WIDE ? static_cast<int64_t>(row) * row_units : static_cast<int64_t>(row)];
+  };
   float acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = 0.f;
@@ -94,13 +99,13 @@ __global__ __launch_bounds__(kEmbedThreads) void patch_embed_kernel(EmbedArgs a)
     uint4 w[kEmbedBatch];
 #pragma unroll
     for (int u = 0; u < kEmbedBatch; ++u) {
-      w[u] = base[s_row[t][o0 + u]];
+      w[u] = chunk(s_row[t][o0 + u]);
     }
 #pragma unroll
     for (int u = 0; u < kEmbedBatch; ++u) add(w[u]);
   }
   for (; o0 < p3; ++o0) {
-    add(base[s_row[t][o0]]);
+    add(chunk(s_row[t][o0]));
   }
   const uint32_t flat = first + t;
   const uint32_t b = flat / per_window, n = flat - b * per_window;
@@ -135,8 +140,7 @@ extern "C" int svhip_patch_embed(const int64_t* tokens, const void* table, const
                 kEmbedMaxOffsets);
   SVHIP_REQUIRE(W >= 8 && W % 8 == 0 && W <= kEmbedMaxWidth, "%s: width %lld unsupported (a multiple of 8 up to %d)",
                 name, (long long)W, kEmbedMaxWidth);
-  SVHIP_REQUIRE(cells * patch * patch * patch < (1ll << 31) && cells * patch * patch * patch * (W / 8) < (1ll << 32),
-                "%s: table too large", name);
+  SVHIP_REQUIRE(cells * patch * patch * patch < (1ll << 31), "%s: table too large", name);
   SVHIP_REQUIRE(reinterpret_cast<uintptr_t>(table) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
                     so_b % 8 == 0 && so_n % 8 == 0,
                 "%s: table and output rows must start on 16-byte boundaries", name);
@@ -147,13 +151,21 @@ extern "C" int svhip_patch_embed(const int64_t* tokens, const void* table, const
                                                                           : kEmbedMaxTokens;
   EmbedArgs a{tokens, static_cast<const uint16_t*>(table), static_cast<const uint16_t*>(bias),
               static_cast<uint16_t*>(out), B, Y, Z, X, patch, cells, W, st_b, so_b, so_n, bad,
-              static_cast<int>(slice_chunks), static_cast<int>(wg_tokens)};
-  const int64_t grid = cdiv(tokens_total, wg_tokens) * kEmbedSlices;
-  SVHIP_REQUIRE(grid < (1ll << 31) && tokens_total < (1ll << 31), "%s: grid too large", name);
-  if (patch == 4) {
-    patch_embed_kernel<4><<<static_cast<unsigned>(grid), kEmbedThreads, 0, as_stream(stream)>>>(a);
-  } else {
-    patch_embed_kernel<0><<<static_cast<unsigned>(grid), kEmbedThreads, 0, as_stream(stream)>>>(a);
+              static_cast<int>(slice_chunks), static_cast<int>(wg_tokens), 0};
+  SVHIP_REQUIRE(tokens_total < (1ll << 31), "%s: grid too large", name);
+  const bool wide = cells * patch * patch * patch * (W / 8) >= (1ll << 32);
+  const int64_t groups = cdiv(tokens_total, wg_tokens);
+  for (int64_t first = 0; first < groups; first += kEmbedGroups) {
+    a.first_group = static_cast<uint32_t>(first);
+    const int64_t count = groups - first < kEmbedGroups ? groups - first : kEmbedGroups;
+    const unsigned grid = static_cast<unsigned>(count * kEmbedSlices);
+    if (wide) {
+      patch_embed_kernel<0, true><<<grid, kEmbedThreads, 0, as_stream(stream)>>>(a);
+    } else if (patch == 4) {
+      patch_embed_kernel<4, false><<<grid, kEmbedThreads, 0, as_stream(stream)>>>(a);
+    } else {
+      patch_embed_kernel<0, false><<<grid, kEmbedThreads, 0, as_stream(stream)>>>(a);
+    }
   }
   SVHIP_LAUNCHED(name);
   return SVHIP_OK;

@@ -80,6 +80,56 @@ def test_gather_patch_column_slices(dev, W, shape, p):
     assert torch.equal(out, ref)
 
 
+def _embed(tokens, table, bias, out, bad, patch):
+    from streamvoxel_amd import _lib
+    B, Y, Z, X = tokens.shape
+    _lib.check(_lib.load().svhip_patch_embed(
+        _lib.ptr(tokens), _lib.ptr(table), _lib.ptr(bias), _lib.ptr(out), _lib.ptr(bad), B, Y, Z, X, patch,
+        table.shape[0] // patch ** 3, table.shape[1], tokens.stride(0), out.stride(0), out.stride(1),
+        _lib.stream_of(out)), 'svhip_patch_embed')
+
+
+def test_patch_embed_of_many_tokens(dev):
+    """More patch tokens than one launch's groups hold, and than 2^24 workgroups of 64 tokens and a column slice would:
+    voxels as patches of edge 1, every output the table row plus the bias."""
+    _case('patch embed 137 M tokens')
+    B, shape, W, C = 2, (16, 2100, 2040), 8, 7
+    table = torch.randn(C, W, device=dev).to(torch.bfloat16)
+    bias = torch.randn(W, device=dev).to(torch.bfloat16)
+    tokens = torch.randint(0, C, (B, *shape), device=dev)
+    out = torch.zeros(B, tokens[0].numel(), W, dtype=torch.bfloat16, device=dev)
+    bad = torch.zeros(1, dtype=torch.int32, device=dev)
+    assert B * tokens[0].numel() > 1 << 27
+    _embed(tokens, table, bias, out, bad, 1)
+    want = table + bias
+    torch.cuda.synchronize()
+    assert int(bad.item()) == 0
+    got, rows = out.view(-1, W), tokens.view(-1)
+    for i in range(0, len(rows), 1 << 22):                  # (torch's own gather of all of them at once leaves zeros)
+        assert torch.equal(got[i:i + (1 << 22)], want[rows[i:i + (1 << 22)]])
+
+
+def test_patch_embed_from_a_table_past_64_gb(dev):
+    """Rows whose first 16-byte chunk lies at 2^32 and beyond."""
+    if torch.cuda.mem_get_info()[0] < 100 << 30:
+        pytest.skip('needs 100 GiB of free device memory')
+    _case('patch embed 2^32 chunks')
+    W, cells, p = 2048, (1 << 24) + 40, 1
+    table = torch.empty(cells, W, dtype=torch.bfloat16, device=dev)
+    rows = torch.tensor([0, 5, (1 << 24) - 1, 1 << 24, cells - 1], device=dev)
+    table[rows] = torch.randn(len(rows), W, device=dev).to(torch.bfloat16)
+    bias = torch.randn(W, device=dev).to(torch.bfloat16)
+    tokens = rows[torch.arange(2 * 4 * 4 * 4, device=dev) % len(rows)].view(2, 4, 4, 4)
+    out = torch.zeros(2, 64, W, dtype=torch.bfloat16, device=dev)
+    bad = torch.zeros(1, dtype=torch.int32, device=dev)
+    _embed(tokens, table, bias, out, bad, p)
+    want = table[tokens.reshape(2, 64)] + bias
+    torch.cuda.synchronize()
+    assert int(bad.item()) == 0 and torch.equal(out, want)
+    del table
+    torch.cuda.empty_cache()
+
+
 def test_gather_patch_flags_tokens_out_of_range(dev):
     from streamvoxel_amd.stream.forward import GatherPatch
     _case('gather patch out-of-range token')
