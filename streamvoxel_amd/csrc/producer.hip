@@ -484,6 +484,8 @@ __global__ __launch_bounds__(kVecThreads) void kv_vec_kernel(KvArgs a) {
   }
 }
 
+__global__ void no_keys_kernel(int32_t* length) { *length = 0; }
+
 // Self-attention operands from the qkv projection, in one launch of two kinds of workgroup:
 //  * rotation, (window b, kRotTokens-token tile): the tile's sin / cos (rounded to bf16) of every (token, pair) go to LDS
 //    once and serve Q and K of all heads (the phase depends on the token and the pair only); the Q | K part of a
@@ -709,7 +711,13 @@ extern "C" int svhip_kv_write_length(const void* prefix_k, const void* prefix_v,
   SVHIP_REQUIRE(even(cache_k, sck_h, sck_k) && (vt || even(cache_v, scv_h, scv_k)),
                 "%s: cache rows must start on pair boundaries", name);
   const int64_t tiles = cdiv(kv_cap, kTileKeys);
-  if (tiles == 0) return SVHIP_OK;
+  if (tiles == 0) {  // no capacity: no key either
+    if (length) {
+      no_keys_kernel<<<1, 1, 0, as_stream(stream)>>>(length);
+      SVHIP_LAUNCHED(name);
+    }
+    return SVHIP_OK;
+  }
   if (fp8) {
     SVHIP_REQUIRE(k_scale && v_scale, "%s: e4m3 needs k_scale and v_scale outputs", name);
     SVHIP_REQUIRE(workspace && workspace_bytes >= svhip_kv_write_workspace_bytes(H, kv_cap),

@@ -55,8 +55,8 @@ class CachedContext:
         keys [0, P) from `prefix` = (prefix_k, prefix_v) [H, P, D] (already rotated, optional), keys [P, P + L)
         from key, value [H, L, D] (the local projections; K rotated by AxialRoPE at fp32 positions [L, 3] with the
         fp32 `frequencies` buffer when given), zeros after; an e4m3 cache also gets its per-(window, head) scales.
-        Inputs are taken as bf16 (the reference's autocast dtype). The window's length is set on the host when the
-        last layer is written or the length changes."""
+        Inputs are taken as bf16 (the reference's autocast dtype). The kernel also sets the window's length, with
+        the last layer or when the length changes."""
         dev = self.k[layer].device
         rows = lambda t: t.to(device=dev, dtype=torch.bfloat16) if t.stride(-1) == 1 else (
             t.to(device=dev, dtype=torch.bfloat16).contiguous())
@@ -98,7 +98,7 @@ class CachedContext:
         vs = self.v_scale[layer][index] if fp8 else None
         # The window's length goes with the kernel: with the last layer, or when it changes.
         new_length = layer == self.layers - 1 or self.host_lengths[index] != P + L
-        length = self.lengths[index] if new_length and self.kv_cap else None
+        length = self.lengths[index] if new_length else None
         _lib.check(lib.svhip_kv_write_length(
             _lib.ptr(pk), _lib.ptr(pv), P, pk.stride(0) if P else 0, pk.stride(1) if P else 0,
             pv.stride(0) if P else 0, pv.stride(1) if P else 0, _lib.ptr(key), _lib.ptr(value), L, key.stride(0),

@@ -238,3 +238,15 @@ def test_kv_write_16_byte_runs_against_pairs(dev, H, D, Pn, L, kcap, fp8, vt):
         outs.append((ck, cv, ks, vs))
     # V^T's padding past the capacity is left as it was by both.
     assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+def test_kv_write_sets_the_length_without_capacity(dev):
+    """A cache of capacity 0 holds no key: the length is set to 0 all the same."""
+    from streamvoxel_amd import _lib
+    _case('kv_write length without capacity')
+    buf = torch.zeros(64, dtype=torch.bfloat16, device=dev)
+    length = torch.full((1,), 7, dtype=torch.int32, device=dev)
+    _lib.check(_lib.load().svhip_kv_write_length(
+        None, None, 0, 0, 0, 0, 0, None, None, 0, 0, 0, 0, 0, None, 0, None, 2, 8, _lib.ptr(buf), 8, 8, _lib.ptr(buf), 8,
+        8, 1, 0, _lib.SVHIP_BF16, None, None, None, 0, _lib.ptr(length), _lib.stream_of(buf)), 'svhip_kv_write_length')
+    assert int(length.item()) == 0
