@@ -161,7 +161,6 @@ struct KvArgs {
   float *k_scale, *v_scale;  // [H] (e4m3)
   float* partial;            // [H, tiles, 2] (e4m3)
   int64_t tiles;
-  int group;                 // heads of a workgroup (kv_vec_kernel)
   int32_t* length;           // set to P + L, or null
 };
 
@@ -300,8 +299,11 @@ __global__ __launch_bounds__(kProducerThreads) void kv_write_kernel(KvArgs a) {
 // heads, 4096 prefix and 8480 local keys: 19.5 us with the pair kernel above (2.0 TB/s), 14.0 us here (2.8 TB/s; groups
 // of four heads and 512 threads 13.9 us, the length by a launch of its own 2.3 us more).
 constexpr int kVecThreads = 256;
-constexpr int kVecHeads = 2;  // at most (fewer where the tile of V^T would pass 64 KB of LDS)
+constexpr int kVecHeads = 2;
 constexpr int kVecBatch = 3;  // chunks of K (and of V) a thread has in flight
+// The widest head's sin / cos table and bf16 V^T tile, with the scales and maxima, within a launch's 64 KB of LDS.
+static_assert(4 * kTileKeys * kMaxHeadDim / 2 + kVecHeads * 2 * kMaxHeadDim * (kTileKeys + 2) + 16 * kVecHeads <= 65536,
+              "LDS of kv_vec_kernel");
 
 // 8 fp32 values divided by `scale` and rounded to e4m3 (two dwords).
 __device__ __forceinline__ uint2 e4m3_pack8(const float* x, float scale) {
@@ -328,8 +330,8 @@ __global__ __launch_bounds__(kVecThreads) void kv_vec_kernel(KvArgs a) {
   constexpr int kRun = 16 / sizeof(E);                 // keys of a 16-byte run of V^T
   constexpr int kRowV = kTileKeys + 4 / sizeof(E);     // LDS V^T row, padded by one bank
   const int D = static_cast<int>(a.D), chunks = D / 8, pairs = D / 2;
-  const int64_t h0 = static_cast<int64_t>(blockIdx.y) * a.group;
-  const int heads = static_cast<int>(a.H - h0 < a.group ? a.H - h0 : a.group);
+  const int64_t h0 = static_cast<int64_t>(blockIdx.y) * kVecHeads;
+  const int heads = static_cast<int>(a.H - h0 < kVecHeads ? a.H - h0 : kVecHeads);
   const int64_t j0 = static_cast<int64_t>(blockIdx.x) * kTileKeys;
   uint32_t* table = reinterpret_cast<uint32_t*>(smem);                            // [key][pair]
   E* sv = reinterpret_cast<E*>(smem + sizeof(uint32_t) * kTileKeys * pairs);      // [head][d][key]
@@ -487,8 +489,8 @@ __global__ __launch_bounds__(kVecThreads) void kv_vec_kernel(KvArgs a) {
 __global__ void no_keys_kernel(int32_t* length) { *length = 0; }
 
 // Self-attention operands from the qkv projection, in one launch of two kinds of workgroup:
-//  * rotation, (window b, kRotTokens-token tile): the tile's sin / cos (rounded to bf16) of every (token, pair) go to LDS
-//    once and serve Q and K of all heads (the phase depends on the token and the pair only); the Q | K part of a
+//  * rotation, (window b, kRotTokens-token tile): the tile's sin / cos (rounded to bf16) of every (token, pair) go to
+//    LDS once and serve Q and K of all heads (the phase depends on the token and the pair only); the Q | K part of a
 //    token's row (2 H D contiguous elements) is then rotated 16 bytes (4 pairs) per thread, four loads in flight;
 //  * layout, (window b, head h, 64-token tile): V rows [64 tokens, D] in through LDS, V^T rows [D, 64 tokens] out,
 //    16 bytes per store.
@@ -678,8 +680,8 @@ extern "C" int svhip_kv_write(const void* prefix_k, const void* prefix_v, int64_
                                scv_d, kv_cap, kv_dtype, k_scale, v_scale, workspace, workspace_bytes, nullptr, stream);
 }
 
-extern "C" int svhip_kv_write_length(const void* prefix_k, const void* prefix_v, int64_t P, int64_t spk_h, int64_t spk_l,
-                              int64_t spv_h, int64_t spv_l, const void* local_k, const void* local_v, int64_t L,
+extern "C" int svhip_kv_write_length(const void* prefix_k, const void* prefix_v, int64_t P, int64_t spk_h,
+                              int64_t spk_l, int64_t spv_h, int64_t spv_l, const void* local_k, const void* local_v, int64_t L,
                               int64_t slk_h, int64_t slk_l, int64_t slv_h, int64_t slv_l, const float* positions,
                               int64_t sp_l, const float* freq, int64_t H, int64_t D, void* cache_k, int64_t sck_h,
                               int64_t sck_k, void* cache_v, int64_t scv_h, int64_t scv_k, int64_t scv_d,
@@ -727,7 +729,7 @@ extern "C" int svhip_kv_write_length(const void* prefix_k, const void* prefix_v,
   KvArgs a{static_cast<const uint16_t*>(prefix_k), static_cast<const uint16_t*>(prefix_v), P, spk_h, spk_l, spv_h,
            spv_l, static_cast<const uint16_t*>(local_k), static_cast<const uint16_t*>(local_v), L, slk_h, slk_l,
            slv_h, slv_l, positions, sp_l, freq, H, D, kv_cap, cache_k, sck_h, sck_k, cache_v, scv_h, scv_k, scv_d,
-           k_scale, v_scale, static_cast<float*>(workspace), tiles, 1, length};
+           k_scale, v_scale, static_cast<float*>(workspace), tiles, length};
   SVHIP_REQUIRE(tiles < 65536 && H < 65536, "%s: grid too large", name);
   const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(H));
   hipStream_t s = as_stream(stream);
@@ -745,10 +747,8 @@ extern "C" int svhip_kv_write_length(const void* prefix_k, const void* prefix_v,
   if (vec) {
     const size_t table = sizeof(uint32_t) * kTileKeys * (D / 2);
     const size_t head = vt ? (fp8 ? 1 : 2) * D * (kTileKeys + (fp8 ? 4 : 2)) : 0;  // V^T of the tile, one head
-    a.group = kVecHeads;
-    while (table + a.group * head > 65536) a.group /= 2;
-    const size_t lds = table + a.group * head;
-    const dim3 g(static_cast<unsigned>(tiles), static_cast<unsigned>(cdiv(H, a.group)));
+    const size_t lds = table + kVecHeads * head;
+    const dim3 g(static_cast<unsigned>(tiles), static_cast<unsigned>(cdiv(H, kVecHeads)));
     if (fp8) {
       kv_vec_kernel<true, false, true><<<g, kVecThreads, table, s>>>(a);
       if (vt) {

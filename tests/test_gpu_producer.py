@@ -201,8 +201,8 @@ def test_kv_write_row_major_v_and_e4m3_codes(dev):
 @pytest.mark.parametrize('vt', [False, True])
 def test_kv_write_16_byte_runs_against_pairs(dev, H, D, Pn, L, kcap, fp8, vt):
     """Rows of 16-byte runs take the vector kernels, local keys moved by two elements the pair kernels: the same
-    codes, scales and zero tail from both (head counts that leave a group part full, the widths where a group holds
-    fewer heads, tiles that mix prefix, local and empty keys, capacities that end inside a run)."""
+    codes, scales and zero tail from both (head counts that leave a workgroup's group of heads part full, the widest
+    head, tiles that mix prefix, local and empty keys, capacities that end inside a run)."""
     from streamvoxel_amd import _lib
     _case(f'kv_write runs H={H} D={D} P={Pn} L={L} kcap={kcap} fp8={fp8} vt={vt}')
     g = torch.Generator().manual_seed(H * D + L)
