@@ -330,7 +330,8 @@ int svhip_kv_write_length(const void* prefix_k, const void* prefix_v, int64_t P,
                    int64_t slk_l, int64_t slv_h, int64_t slv_l, const float* positions, int64_t sp_l,
                    const float* freq, int64_t H, int64_t D, void* cache_k, int64_t sck_h, int64_t sck_k,
                    void* cache_v, int64_t scv_h, int64_t scv_k, int64_t scv_d, int64_t kv_cap, int kv_dtype,
-                   float* k_scale, float* v_scale, void* workspace, size_t workspace_bytes, int32_t* length, void* stream);
+                   float* k_scale, float* v_scale, void* workspace, size_t workspace_bytes, int32_t* length,
+                   void* stream);
 
 /*
  * Self-attention operands of a transformer block from its fused qkv projection: qkv bf16, element (b,n,s,h,d)

@@ -681,9 +681,9 @@ extern "C" int svhip_kv_write(const void* prefix_k, const void* prefix_v, int64_
 }
 
 extern "C" int svhip_kv_write_length(const void* prefix_k, const void* prefix_v, int64_t P, int64_t spk_h,
-                              int64_t spk_l, int64_t spv_h, int64_t spv_l, const void* local_k, const void* local_v, int64_t L,
-                              int64_t slk_h, int64_t slk_l, int64_t slv_h, int64_t slv_l, const float* positions,
-                              int64_t sp_l, const float* freq, int64_t H, int64_t D, void* cache_k, int64_t sck_h,
+                              int64_t spk_l, int64_t spv_h, int64_t spv_l, const void* local_k, const void* local_v,
+                              int64_t L, int64_t slk_h, int64_t slk_l, int64_t slv_h, int64_t slv_l,
+                              const float* positions, int64_t sp_l, const float* freq, int64_t H, int64_t D, void* cache_k, int64_t sck_h,
                               int64_t sck_k, void* cache_v, int64_t scv_h, int64_t scv_k, int64_t scv_d,
                               int64_t kv_cap, int kv_dtype, float* k_scale, float* v_scale, void* workspace,
                               size_t workspace_bytes, int32_t* length, void* stream) {

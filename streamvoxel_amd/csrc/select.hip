@@ -345,8 +345,9 @@ __global__ __launch_bounds__(kWG) void apportion_kernel(const int64_t* __restric
 // The same for one window of at most kGroupBlocks blocks, by a workgroup of 256 threads: every thread holds the keys of
 // blocks t, t + 256, ... in registers; an MSB-first 8-bit radix select finds the threshold, one LDS histogram a digit,
 // and ends as soon as the threshold's bin is taken whole (mostly after three or four of the eight digits). A serial
-// chain of loads, digits and barriers that runs beside the entropy pass; by one wave with the keys in LDS it took longer
-// than the entropy pass beside it (one window of 256 fp32 classes as planes: 28.8 us for the launch, 23.4 us now).
+// chain of loads, digits and barriers that runs beside the entropy pass; by one wave with the keys in LDS it took
+// longer than the entropy pass beside it (one window of 256 fp32 classes as planes: 28.8 us for the launch, 23.4 us
+// now).
 constexpr int kGroupBlocks = 1024;
 constexpr int kGroupThreads = 256;
 
@@ -418,12 +419,15 @@ __device__ void apportion_group(const ApportionArgs& a, int64_t b, ApportionShar
       __syncthreads();
 #pragma unroll
       for (int u = 0; u < kPer; ++u) {
-        if (tid + kGroupThreads * u < nb && (key[u] & mask) == prefix) atomicAdd(&sh.hist[(key[u] >> shift) & 0xff], 1u);
+        if (tid + kGroupThreads * u < nb && (key[u] & mask) == prefix) {
+          atomicAdd(&sh.hist[(key[u] >> shift) & 0xff], 1u);
+        }
       }
       __syncthreads();
       // Every wave scans the bins for itself (four a lane): the bin that holds the take-th key.
       const uint4 h4 = *reinterpret_cast<const uint4*>(&sh.hist[4 * lane]);
-      const int hs[4] = {static_cast<int>(h4.x), static_cast<int>(h4.y), static_cast<int>(h4.z), static_cast<int>(h4.w)};
+      const int hs[4] = {static_cast<int>(h4.x), static_cast<int>(h4.y), static_cast<int>(h4.z),
+                         static_cast<int>(h4.w)};
       const int mine = hs[0] + hs[1] + hs[2] + hs[3];
       int incl = mine;
 #pragma unroll

@@ -36,7 +36,9 @@ namespace svhip {
 
 constexpr int kF32Row = 64;      // floats of an LDS row (one key)
 constexpr int kF32Resident = 2;  // workgroups per CU (two waves per SIMD)
-constexpr int kF32PieceBlocks = 6;  // least key blocks of a piece
+// Least key blocks of a piece (key_split.hpp); a block takes six times the bf16 kernel's. One window of 8 x 48 heads
+// and 29 blocks at 6 / 12: 63 / 90 us; 2 windows of 8 x 64 and 33 blocks at 12 / 16: 115 / 156.
+constexpr int kF32PieceBlocks = 6;
 // Key blocks summed into one accumulator before it is added to the total: short chains of fp32 sums, as the two chains
 // of a score are. From float64, 128 / 400 / 2300 / 9000 keys: 2.6 / 3.0 / 4.0 / 7.0e-7 on the VALU before, 2.2 / 2.3 /
 // 2.6 / 2.8e-7 so; with one chain a score and two blocks 3.1 / 3.4 / 3.5 / 3.8e-7 (8 us faster on the single column),
