@@ -41,6 +41,7 @@ def attention(query, key, val, lengths=None, cu_seqlens=None, scale=None, k_scal
     `out` (optional) [B,H,Q,D] bf16 with head_dim contiguous, e.g. a [B,Q,H,D] buffer's transpose(1, 2) view.
     fp32 query, key and val (head_dim 16, 32, 48 or 64, rows 16-byte aligned) take fp32 arithmetic throughout and
     return fp32 (`svhip_xattn_fwd_f32`, or `svhip_xattn_fwd_f32_masked` with a key mask: the reference's fp32 SDPA).
+    A window's result has the same bits whichever other windows share the call.
     Returns out."""
     _lib.require_gpu(query, key, val, lengths, cu_seqlens, k_scale, v_scale, out)
     if query.dtype == torch.float32:
